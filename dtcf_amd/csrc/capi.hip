@@ -246,6 +246,20 @@ int dtcf_view_create(int64_t rows, int64_t cols, const int64_t *rofs, const int6
     bool rowpairs = beven && ceven && (rows % 2 == 0) && (rpb % 2 == 0);
     for (int64_t r = 0; rowpairs && r + 1 < rows; r += 2)
         rowpairs = (rofs[r + 1] == rofs[r] + 1) && (rofs[r] % 2 == 0);
+    // The same without the alignment (the last column [row] of an odd count
+    // has no partner), and the direction with more unit steps.
+    bool coladj = (cols % 2 == 0) && (cpb % 2 == 0), rowadj = (rows % 2 == 0) && (rpb % 2 == 0);
+    int64_t cunit = 0, runit = 0;
+    for (int64_t c = 0; c + 1 < cols; c++) {
+        const bool one = cofs[c + 1] == cofs[c] + 1;
+        cunit += one;
+        if (c % 2 == 0) coladj = coladj && one;
+    }
+    for (int64_t r = 0; r + 1 < rows; r++) {
+        const bool one = rofs[r + 1] == rofs[r] + 1;
+        runit += one;
+        if (r % 2 == 0) rowadj = rowadj && one;
+    }
 
     dtcf_view_s *v = new dtcf_view_s();
     v->rows = rows;
@@ -257,6 +271,9 @@ int dtcf_view_create(int64_t rows, int64_t cols, const int64_t *rofs, const int6
     v->span = span;
     v->colpairs = colpairs;
     v->rowpairs = rowpairs;
+    v->coladj = coladj;
+    v->rowadj = rowadj;
+    v->rowwise = (double)runit * cols > (double)cunit * rows;
     v->rowrun16 = !blk;
     for (int64_t r = 0; v->rowrun16 && r < rows; r++) v->rowrun16 = rofs[r] == rofs[r & ~15ll] + (r & 15);
     hipError_t e = hipMalloc(&v->rofs, rows * sizeof(int64_t));
@@ -312,6 +329,8 @@ int dtcf_view_sub(dtcf_view p, int64_t r0, int64_t rows, int64_t c0, int64_t col
     }
     v->colpairs = p->colpairs && c0 % 2 == 0 && cols % 2 == 0;
     v->rowpairs = p->rowpairs && r0 % 2 == 0 && rows % 2 == 0;
+    v->coladj = p->coladj && c0 % 2 == 0 && cols % 2 == 0;
+    v->rowadj = p->rowadj && r0 % 2 == 0 && rows % 2 == 0;
     v->rowrun16 = p->rowrun16 && r0 % 16 == 0;
     *out = v;
     return DTCF_OK;
@@ -329,6 +348,21 @@ static void fill_op(OpArgs &o, const dtcf_view_s *v)
     o.div_rpb = FastDiv((uint32_t)v->rpb);
     o.div_cpb = FastDiv((uint32_t)v->cpb);
     o.ncb = v->ncb;
+}
+
+// How the GEMM loads a view operand: aligned pairs along k, along the rows;
+// else adjacent pairs at any alignment; else single elements, paired along
+// the direction whose neighbours are in memory (so a wave's loads stay in
+// few lines).
+static int operand_mode(const dtcf_view_s *v, const double *X, OpArgs &o)
+{
+    const bool al = (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+    const bool rows = (v->colpairs || v->rowpairs) ? !v->colpairs
+                      : (v->coladj || v->rowadj)   ? !v->coladj
+                                                   : v->rowwise;
+    o.vec2 = al && (v->colpairs || v->rowpairs) && !v->blk;
+    o.adj = rows ? v->rowadj : v->coladj;
+    return rows ? kVMN : kVK;
 }
 
 static int gemm_view_impl(int64_t m, int64_t n, int64_t k, double alpha, const double *A,
@@ -384,16 +418,8 @@ static int gemm_view_impl(int64_t m, int64_t n, int64_t k, double alpha, const d
     g.C = C;
     fill_op(g.a, av);
     fill_op(g.b, bv);
-    const bool aal = (reinterpret_cast<uintptr_t>(A) & 15) == 0;
-    const bool bal = (reinterpret_cast<uintptr_t>(B) & 15) == 0;
-    // Prefer k-contiguous loads; fall back to row-contiguous; otherwise
-    // element loads through the k-mode path.
-    if (av->colpairs) { g.amode = kVK; g.a.vec2 = aal; }
-    else if (av->rowpairs) { g.amode = kVMN; g.a.vec2 = aal; }
-    else { g.amode = kVK; g.a.vec2 = 0; }
-    if (bv->colpairs) { g.bmode = kVK; g.b.vec2 = bal; }
-    else if (bv->rowpairs) { g.bmode = kVMN; g.b.vec2 = bal; }
-    else { g.bmode = kVK; g.b.vec2 = 0; }
+    g.amode = operand_mode(av, A, g.a);
+    g.bmode = operand_mode(bv, B, g.b);
     if (cv) {
         fill_op(g.c, cv);
         // column pairs of C adjacent and 16-byte aligned (the thin kernel's

@@ -43,7 +43,8 @@ struct OpArgs {
     FastDiv div_rpb, div_cpb;
     int64_t ncb;
     int32_t vec2;  // 1: (r,c),(r,c+1) [k-mode] or (r,c),(r+1,c) [mn-mode] are adjacent
-                   //    and 16-byte aligned wherever both are in range
+                   //    and 16-byte aligned wherever both are in range (c or r even)
+    int32_t adj;   // views: 1: they are adjacent, at any alignment
 };
 
 struct GemmArgs {
@@ -55,6 +56,7 @@ struct GemmArgs {
     OpArgs a, b, c;
     int32_t amode, bmode, cview;
     uint32_t tiles_m, tiles_n;
+    int64_t nfast;  // K steps loaded without bounds checks (gemm_tile.hpp)
     // Tail split: workgroups [0, t_full) own whole tiles; the remaining
     // tiles t_full.. are split over K into `sk` slices of `kchunk` K steps
     // each, written to `ws` and summed in slice order by a second kernel.
@@ -85,7 +87,7 @@ struct GemmGroupProb {
     int32_t vec2a, vec2b;
     uint32_t tiles_m, tiles_n, wg0;
     uint32_t t_whole, tail0;
-    int64_t kchunk;
+    int64_t kchunk, nfast;
 };
 struct GemmGroupArgs {
     double alpha;
@@ -95,6 +97,20 @@ struct GemmGroupArgs {
     double *ws;             // tail slices, [tail tile][slice][BM][BN]
     GemmGroupProb p[kGroupMax];
 };
+
+// One instantiation per C tile (gemm_tile_*.hip).
+int gemm_tile_128x128(const GemmArgs &g, hipStream_t s);
+int gemm_tile_192x96(const GemmArgs &g, hipStream_t s);
+int gemm_tile_96x192(const GemmArgs &g, hipStream_t s);
+int gemm_tile_64x64(const GemmArgs &g, hipStream_t s);
+int gemm_tile_192x64(const GemmArgs &g, hipStream_t s);
+int gemm_tile_64x192(const GemmArgs &g, hipStream_t s);
+int gemm_group_tile_128x128(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s);
+int gemm_group_tile_192x96(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s);
+int gemm_group_tile_96x192(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s);
+int gemm_group_tile_64x64(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s);
+// Which tiles a launch cuts over K (gemm_f64.hip).
+void gemm_tail_split(uint32_t T, uint32_t slots, int64_t nk, uint32_t &nsplit, uint32_t &sk);
 
 int gemm_f64_group_launch(const GemmGroupArgs &ga, int cfg, int amode, int bmode, hipStream_t s);
 

@@ -1,0 +1,703 @@
+// The FP64 MFMA tile kernels (v_mfma_f64_16x16x4_f64) and their launch, as
+// templates over the C tile; gemm_tile_*.hip instantiate one tile each.
+//
+// Tiling: a 256-thread workgroup (4 wave64) owns a BM x BN block of C; the
+// waves form a (BM/WM) x (BN/WN) grid and each wave owns WM x WN as
+// (WM/16) x (WN/16) MFMA 16x16 accumulators (4 doubles per lane each).  K is
+// walked in steps of BK = 16 through two LDS stages, one barrier per step,
+// the next step loading while this one runs its MFMAs.
+//
+// LDS layout: 16 rows x 16 k of an operand are two fragments h = 0, 1 of 1
+// KiB, 16 bytes per lane l.
+//   k pairs (KC: kDK, kVK):   lane l holds row l % 16, k = 8h + 2 (l / 16) + {0, 1}
+//   row pairs (kDMN, kVMN):   lane l holds rows 2 (l % 8) + {0, 1} of
+//                             k = 8h + 2 ((l / 8) % 4) + l / 32
+// The MFMA k-slice (h, t), t = 0, 1, takes k = 8h + 2 fk + t from its four
+// lane groups fk = l / 16 in both layouts, so operands of either kind
+// combine and the sum over k runs in one order.  A k-pair fragment is read
+// with one 16-byte read per lane for both slices, a row-pair one with an
+// 8-byte read per slice; every read of a wave is one contiguous span (no
+// bank conflicts).
+//
+// Two ways to fill a stage:
+//   direct (both operands' pairs adjacent and 16-byte aligned, no block
+//   table): global_load_lds, 16 bytes per lane, lane l's pair straight to
+//   byte 16 l of its fragment.  No staging registers and no LDS stores, and
+//   the loop body is 64 MFMAs, 16 fragment reads and 8 loads (the register-
+//   staged form took 242-256 VGPRs at 128 x 128 and spilled up to 38 for view
+//   operands; this one takes 220-240 without spills).  Bound by the FP64
+//   MFMA rate: 8192^3 dense 63.7 -> 69.9 TF/s (A m x k, B n x k), 66.4 ->
+//   70.3 (B k x n), 2048^3 56.8 -> 61.6; the 9216^3 ring step through its
+//   views 65.9 -> 67.3 TF/s.
+//   staged (anything else): pairs loaded to registers -- one 16-byte load
+//   at 8-byte alignment where the pair is adjacent (every dense operand,
+//   whatever its pitch), two 8-byte loads where it is not -- and stored to
+//   the other stage after the step's MFMAs are issued.
+//   1331 x 1177 x 905, odd pitches: 160 -> 69 us (it ran element loads with
+//   bounds checks in every step).
+// Only a K step that is not whole (K % 16), or the last one when a row pair
+// may reach past the operand's last row, is loaded element by element with
+// bounds checks (nfast).  Rows past the operand's last (an edge tile) load
+// the last row or row pair again: in range, and never stored.
+#pragma once
+#include <algorithm>
+#include <mutex>
+
+#include "common.hpp"
+#include "gemm_f64.hpp"
+
+namespace dtcf {
+namespace {
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // 16-byte load at 8-byte alignment
+
+constexpr int BK = 16;
+constexpr int NT = 256;
+constexpr int KH = BK / 8;  // fragments per 16 rows and K step
+
+template <int MODE>
+struct ModeT {
+    static constexpr bool KC = (MODE == kDK || MODE == kVK);
+    static constexpr bool VIEW = (MODE == kVK || MODE == kVMN);
+};
+
+// Element offset of (r, c) in an operand.
+template <int MODE>
+__device__ inline int64_t op_addr(const OpArgs &o, int64_t r, int64_t c)
+{
+    if constexpr (MODE == kDK) return r * o.ld + c;
+    else if constexpr (MODE == kDMN) return c * o.ld + r;
+    else {
+        int64_t a = o.rofs[r] + o.cofs[c];
+        if (o.blk) {
+            const uint32_t rb = o.div_rpb.div((uint32_t)r);
+            const uint32_t cb = o.div_cpb.div((uint32_t)c);
+            a += o.blk[(int64_t)rb * o.ncb + cb];
+        }
+        return a;
+    }
+}
+
+// One wave's share of one operand's stage: P of the ROWS/16 * KH fragments,
+// f = wave * P + i: 16-row group f / KH, half f % KH.
+template <int ROWS, int MODE, bool DIRECT>
+struct Loader {
+    typedef ModeT<MODE> M;
+    static constexpr int P = ROWS / 16 * KH / 4;
+    static_assert(ROWS % 32 == 0, "whole fragments per wave");
+    const double *p0[P];  // row part of the pair (its first row)
+    const double *p1[(!DIRECT && !M::KC) ? P : 1];  // second row of a non-adjacent row pair
+    int64_t c0[M::VIEW ? P : 1];                    // column offsets of the next step to load
+    int64_t c1[(M::VIEW && !DIRECT && M::KC) ? P : 1];
+    d2 reg[DIRECT ? 1 : P];
+
+    __device__ static inline int frag_row(int f, int l) { return 16 * (f / KH) + (M::KC ? (l & 15) : 2 * (l & 7)); }
+    __device__ static inline int frag_k(int f, int l)
+    {
+        return 8 * (f % KH) + (M::KC ? 2 * (l >> 4) : 2 * ((l >> 3) & 3) + (l >> 5));
+    }
+
+    __device__ inline void init(const OpArgs &o, const double *base, int64_t row0, int64_t rows, int w, int l)
+    {
+        // whole pairs: rows past the end repeat the last row or row pair (an
+        // odd last row is its own pair; nfast keeps its partner in range)
+        const int64_t last = M::KC ? rows - 1 : (rows - 1) & ~int64_t(1);
+#pragma unroll
+        for (int i = 0; i < P; i++) {
+            const int f = w * P + i;
+            const int64_t r = min(row0 + frag_row(f, l), last);
+            if constexpr (MODE == kDK) p0[i] = base + r * o.ld + frag_k(f, l);
+            else if constexpr (MODE == kDMN) p0[i] = base + frag_k(f, l) * o.ld + r;
+            else {
+                p0[i] = base + o.rofs[r];
+                if constexpr (!DIRECT && !M::KC) p1[i] = base + o.rofs[min(r + 1, rows - 1)];
+            }
+        }
+    }
+    // Column offsets of K step kt (views): fetched a step before their data,
+    // so no data load waits on a table load.
+    __device__ inline void fetch(const OpArgs &o, int64_t kt, int w, int l)
+    {
+        if constexpr (M::VIEW) {
+#pragma unroll
+            for (int i = 0; i < P; i++) {
+                const int64_t c = kt * BK + frag_k(w * P + i, l);
+                c0[i] = o.cofs[c];
+                if constexpr (!DIRECT && M::KC) c1[i] = o.cofs[c + 1];
+            }
+        }
+    }
+    __device__ inline const double *at(const OpArgs &o, int i, int64_t kt) const
+    {
+        if constexpr (MODE == kDK) return p0[i] + kt * BK;
+        else if constexpr (MODE == kDMN) return p0[i] + kt * BK * o.ld;
+        else return p0[i] + c0[i];
+    }
+    // Loads K step kt (kt < nfast) of this wave's fragments: into the stage
+    // (direct) or into registers.
+    __device__ inline void load(const OpArgs &o, d2 *stage, int64_t kt, int w)
+    {
+        if constexpr (DIRECT) {
+#pragma unroll
+            for (int i = 0; i < P; i++)
+                __builtin_amdgcn_global_load_lds(
+                    (const void *)at(o, i, kt),
+                    (__attribute__((address_space(3))) void *)(stage + (w * P + i) * 64), 16, 0, 0);
+        } else if (!M::VIEW || o.adj) {  // uniform
+#pragma unroll
+            for (int i = 0; i < P; i++) reg[i] = *reinterpret_cast<const d2u *>(at(o, i, kt));
+        } else if constexpr (M::VIEW) {
+#pragma unroll
+            for (int i = 0; i < P; i++) {
+                reg[i].x = p0[i][c0[i]];
+                if constexpr (M::KC) reg[i].y = p0[i][c1[i]];
+                else reg[i].y = p1[i][c0[i]];
+            }
+        }
+    }
+    __device__ inline void store(d2 *stage, int w, int l) const
+    {
+#pragma unroll
+        for (int i = 0; i < (DIRECT ? 0 : P); i++) stage[(w * P + i) * 64 + l] = reg[i];
+    }
+    // Loads and stores one K step element by element, zeros outside.
+    __device__ inline void load_checked(const OpArgs &o, const double *base, d2 *stage, int64_t row0,
+                                        int64_t rows, int64_t K, int64_t kt, int w, int l) const
+    {
+#pragma unroll
+        for (int i = 0; i < P; i++) {
+            const int f = w * P + i;
+            const int64_t r = row0 + frag_row(f, l), c = kt * BK + frag_k(f, l);
+            const int64_t r1 = M::KC ? r : r + 1, cc1 = M::KC ? c + 1 : c;
+            d2 v = {0.0, 0.0};
+            if (r < rows && c < K) v.x = base[op_addr<MODE>(o, r, c)];
+            if (r1 < rows && cc1 < K) v.y = base[op_addr<MODE>(o, r1, cc1)];
+            stage[f * 64 + l] = v;
+        }
+    }
+};
+
+// Logical tile q -> (tm, tn) through a grouped (8 tile rows) swizzle.
+__device__ inline void tile_coords(uint32_t q, uint32_t tiles_m, uint32_t tiles_n, uint32_t &tm,
+                                   uint32_t &tn)
+{
+    const uint32_t GROUP = 8;
+    const uint32_t width = GROUP * tiles_n;
+    const uint32_t gid = q / width;
+    const uint32_t first = gid * GROUP;
+    const uint32_t gsz = min(tiles_m - first, GROUP);
+    tm = first + (q % width) % gsz;
+    tn = (q % width) / gsz;
+}
+
+// One workgroup's share of a GEMM: logical tile q over K steps [kt0, kt1);
+// a split slice (split) writes raw partial sums to workspace slot sidx.
+template <int BM, int BN, int WM, int WN, int AMODE, int BMODE, bool DIRECT>
+__device__ __forceinline__ void gemm_tile(const GemmArgs &g, uint32_t q, int64_t kt0, int64_t kt1,
+                                          bool split, uint32_t sidx)
+{
+    static_assert((BM / WM) * (BN / WN) == 4, "four waves per workgroup");
+    constexpr int FM = WM / 16, FN = WN / 16;
+    constexpr int FA = BM / 16 * KH, FB = BN / 16 * KH;  // fragments per stage
+    constexpr bool AKC = ModeT<AMODE>::KC, BKC = ModeT<BMODE>::KC;
+    extern __shared__ d2 smem[];  // two stages of (FA + FB) x 64
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / (BN / WN), wn = wave % (BN / WN);
+
+    uint32_t tm, tn;
+    tile_coords(q, g.tiles_m, g.tiles_n, tm, tn);
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+
+    Loader<BM, AMODE, DIRECT> la;
+    Loader<BN, BMODE, DIRECT> lb;
+    d4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) acc[i][j] = (d4){0.0, 0.0, 0.0, 0.0};
+
+    // K steps [0, n) of this share; the first nf are loaded unchecked.
+    const int n = (int)(kt1 - kt0), nf = (int)min(max(g.nfast - kt0, int64_t(0)), kt1 - kt0);
+    auto stage = [&](int s) __attribute__((always_inline)) { return smem + (s & 1) * (FA + FB) * 64; };
+    auto begin = [&](int s) __attribute__((always_inline)) {
+        la.load(g.a, stage(s), kt0 + s, wave);
+        lb.load(g.b, stage(s) + FA * 64, kt0 + s, wave);
+        if (s + 1 < nf) {
+            la.fetch(g.a, kt0 + s + 1, wave, lane);
+            lb.fetch(g.b, kt0 + s + 1, wave, lane);
+        }
+    };
+    auto finish = [&](int s) __attribute__((always_inline)) {
+        la.store(stage(s), wave, lane);
+        lb.store(stage(s) + FA * 64, wave, lane);
+    };
+    auto checked = [&](int s) __attribute__((always_inline)) {
+        la.load_checked(g.a, g.A, stage(s), m0, g.m, g.k, kt0 + s, wave, lane);
+        lb.load_checked(g.b, g.B, stage(s) + FA * 64, n0, g.n, g.k, kt0 + s, wave, lane);
+    };
+    // The direct loads are counted by vmcnt and the compiler does not tie
+    // them to the LDS reads: every wave waits for its own, then the barrier
+    // makes everyone's visible.  The clobber keeps LDS accesses on their side;
+    // the scheduling barrier keeps the step's MFMAs above the wait (the
+    // compiler otherwise sinks them below it, and a step then starts by
+    // waiting for the loads it just issued: 25.4 instead of 23.6 ms for the
+    // ring step).
+    auto sync = []() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(7 << 4);  // vmcnt 0, lgkmcnt 0
+        asm volatile("s_barrier" ::: "memory");
+    };
+    // The second half's fragments are read after the first MFMAs of the
+    // first half are issued, and complete under the rest of them.
+    auto compute = [&](int s, bool store_next) __attribute__((always_inline)) {
+        const d2 *a_s = stage(s), *b_s = a_s + FA * 64;
+        d2 af[KH][FM], bf[KH][FN];
+        auto frags = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                const d2 *f = b_s + ((wn * FN + j) * KH + h) * 64;
+                const double *e = reinterpret_cast<const double *>(f);
+                if constexpr (BKC) bf[h][j] = f[lane];
+                else bf[h][j] = (d2){e[lane], e[64 + lane]};
+            }
+#pragma unroll
+            for (int i = 0; i < FM; i++) {
+                const d2 *f = a_s + ((wm * FM + i) * KH + h) * 64;
+                const double *e = reinterpret_cast<const double *>(f);
+                if constexpr (AKC) af[h][i] = f[lane];
+                else af[h][i] = (d2){e[lane], e[64 + lane]};
+            }
+        };
+        auto row = [&](int h, int t, int i) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[h][i][t], bf[h][j][t], acc[i][j], 0, 0, 0);
+        };
+        // The wave starting a K step takes issue priority for its first half,
+        // so the two workgroups sharing a CU drift apart and one's loads and
+        // barrier overlap the other's MFMAs.
+        __builtin_amdgcn_s_setprio(1);
+        frags(0);
+        __builtin_amdgcn_sched_barrier(0);
+        row(0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        frags(1);
+#pragma unroll
+        for (int x = 1; x < 2 * FM; x++) row(0, x / FM, x % FM);
+        __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+        for (int x = 0; x < 2 * FM; x++) row(1, x / FM, x % FM);
+        // The other stage was last read before the previous barrier: the
+        // staged form stores the next step after the last MFMAs are issued.
+        if (!DIRECT && store_next) finish(s + 1);
+    };
+
+    if (nf > 0) {
+        la.init(g.a, g.A, m0, g.m, wave, lane);
+        lb.init(g.b, g.B, n0, g.n, wave, lane);
+        la.fetch(g.a, kt0, wave, lane);
+        lb.fetch(g.b, kt0, wave, lane);
+        begin(0);
+        finish(0);
+    } else if (n > 0) {
+        checked(0);
+    }
+    sync();
+    int s = 0;
+    for (; s + 1 < nf; s++) {
+        begin(s + 1);
+        compute(s, true);
+        sync();
+    }
+    // the last unchecked step and the checked one, out of the loop's code
+    for (; s < n; s++) {
+        if (s + 1 < n) checked(s + 1);
+        compute(s, false);
+        sync();
+    }
+
+    const int fr = lane & 15, fq = lane >> 4;
+    if (split) {
+        // K slice of a remainder tile: raw partial sums to the workspace,
+        // laid out [slice index][BM][BN]; the reduce kernel adds them to C.
+        double *w = g.ws + (int64_t)sidx * BM * BN;
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    w[(wm * WM + i * 16 + fq + 4 * r) * BN + wn * WN + j * 16 + fr] = acc[i][j][r];
+        return;
+    }
+
+    // Epilogue: C += alpha * acc  (beta = 1, as every reference call site),
+    // or C = alpha * acc when the caller asked for an overwrite.  Sixteen
+    // rows at a time: their addresses, then the old values in one batch of
+    // loads, then the stores (a load per store would wait for each in turn).
+    const double alpha = g.alpha;
+    int64_t co[FN];
+#pragma unroll
+    for (int j = 0; j < FN; j++) {
+        const int64_t col = min(n0 + wn * WN + j * 16 + fr, g.n - 1);
+        co[j] = g.cview ? g.c.cofs[col] : col;
+    }
+#pragma unroll
+    for (int i = 0; i < FM; i++) {
+        int64_t ad[4][FN];
+        double old[4][FN];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int64_t row = min(m0 + wm * WM + i * 16 + fq + 4 * r, g.m - 1);
+            const int64_t ro = g.cview ? g.c.rofs[row] : row * g.c.ld;
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                ad[r][j] = ro + co[j];
+                if (g.cview && g.c.blk) {
+                    const int64_t col = min(n0 + wn * WN + j * 16 + fr, g.n - 1);
+                    ad[r][j] += g.c.blk[(int64_t)g.c.div_rpb.div((uint32_t)row) * g.c.ncb +
+                                        g.c.div_cpb.div((uint32_t)col)];
+                }
+            }
+        }
+        if (!g.overwrite) {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int j = 0; j < FN; j++) old[r][j] = g.C[ad[r][j]];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            if (m0 + wm * WM + i * 16 + fq + 4 * r >= g.m) continue;
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                if (n0 + wn * WN + j * 16 + fr >= g.n) continue;
+                const double v = alpha * acc[i][j][r];
+                g.C[ad[r][j]] = g.overwrite ? v : old[r][j] + v;
+            }
+        }
+    }
+}
+
+// K steps that need no bounds checks (gemm_tile): whole ones, less the last
+// when a row pair of a dense row-contiguous operand with an odd row count
+// reads one element past the operand's last k row.
+inline int64_t fast_steps(int64_t k, bool odd_pairs, bool table)
+{
+    if (table) return 0;
+    return (odd_pairs && k % BK == 0) ? k / BK - 1 : k / BK;
+}
+
+template <int BM, int BN>
+struct Occ {
+    // Two workgroups per CU (their LDS stages take 64-74 KiB each at the
+    // large tiles).
+    static constexpr int v = 2;
+};
+
+template <int BM, int BN, int WM, int WN, int AMODE, int BMODE, bool DIRECT>
+__global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_kernel(GemmArgs g)
+{
+    // Workgroups below t_full own whole tiles; their ids are first remapped
+    // so consecutive tiles land on one XCD (its own L2).  Workgroups above
+    // own one K slice of a remainder tile.
+    const uint32_t bid = blockIdx.x;
+    const int64_t nk_all = (g.k + BK - 1) / BK;
+    uint32_t q, sidx = 0;
+    int64_t kt0 = 0, kt1 = nk_all;
+    bool split = false;
+    if (bid < g.t_full) {
+        q = bid;
+        if ((g.t_full & 7u) == 0) q = (bid & 7u) * (g.t_full >> 3) + (bid >> 3);
+    } else {
+        split = true;
+        sidx = bid - g.t_full;
+        q = g.t_full + sidx / g.sk;
+        kt0 = (int64_t)(sidx % g.sk) * g.kchunk;
+        kt1 = min(nk_all, kt0 + g.kchunk);
+    }
+    gemm_tile<BM, BN, WM, WN, AMODE, BMODE, DIRECT>(g, q, kt0, kt1, split, sidx);
+}
+
+// Problem owning tail tile ti (tail tiles are numbered problem by problem).
+__device__ inline int tail_problem(const GemmGroupArgs &ga, uint32_t ti)
+{
+    int p = 0;
+    for (int i = 0; i < ga.np; i++) {
+        const GemmGroupProb &P = ga.p[i];
+        if (ti >= P.tail0 && ti < P.tail0 + (P.tiles_m * P.tiles_n - P.t_whole)) p = i;
+    }
+    return p;
+}
+
+// Several independent dense GEMMs C_p (+)= alpha A_p B_p^T in one launch.
+// Problem p's whole tiles own workgroups [wg0_p, wg0_p + t_whole_p rounded
+// up to 8); wg0_p is a multiple of 8, so a workgroup's XCD is its local id
+// mod 8 and each problem gets the same XCD-contiguous tile order as a lone
+// launch.  (Cutting the list of all whole tiles into eight runs of equal
+// work, one per XCD, was measured slower: 8 x 2048^3 55.0 against 56.6
+// TF/s, 2 x 4096 x 4096 x 2048 59.0 against 63.7.)  Workgroups past a
+// problem's last whole tile exit at once.  The workgroups after wg_whole
+// each own one K slice of a tail tile.
+template <int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
+__global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_group_kernel(GemmGroupArgs ga)
+{
+    const uint32_t bid = blockIdx.x;
+    int p = 0;
+    uint32_t q, sidx = 0;
+    bool split = false;
+    if (bid < ga.wg_whole) {
+        for (int i = 1; i < ga.np; i++)
+            if (bid >= ga.p[i].wg0) p = i;
+        const GemmGroupProb &P = ga.p[p];
+        const uint32_t T = P.t_whole, T8 = (T + 7u) & ~7u;
+        const uint32_t local = bid - P.wg0;
+        q = (local & 7u) * (T8 >> 3) + (local >> 3);
+        if (q >= T) return;  // whole workgroup: no barrier has been reached
+    } else {
+        split = true;
+        sidx = bid - ga.wg_whole;
+        const uint32_t ti = sidx / ga.sk;
+        p = tail_problem(ga, ti);
+        q = ga.p[p].t_whole + (ti - ga.p[p].tail0);
+    }
+    const GemmGroupProb &P = ga.p[p];
+    const int64_t nk = (P.k + BK - 1) / BK;
+    int64_t kt0 = 0, kt1 = nk;
+    if (split) {
+        kt0 = min(nk, (int64_t)(sidx % ga.sk) * P.kchunk);
+        kt1 = min(nk, kt0 + P.kchunk);
+    }
+    GemmArgs g{};
+    g.m = P.m;
+    g.n = P.n;
+    g.k = P.k;
+    g.nfast = P.nfast;
+    g.alpha = ga.alpha;
+    g.A = P.A;
+    g.B = P.B;
+    g.C = P.C;
+    g.a.ld = P.lda;
+    g.b.ld = P.ldb;
+    g.c.ld = P.ldc;
+    g.tiles_m = P.tiles_m;
+    g.tiles_n = P.tiles_n;
+    g.overwrite = ga.overwrite;
+    g.ws = ga.ws;
+    gemm_tile<BM, BN, WM, WN, AM, BMD, DIRECT>(g, q, kt0, kt1, split, sidx);
+}
+
+// Sums the K slices of each tail tile of a group in slice order and adds
+// alpha * sum to (or, overwriting, stores it in) the problem's C.
+template <int BM, int BN>
+__global__ __launch_bounds__(256) void group_split_reduce_kernel(GemmGroupArgs ga)
+{
+    const uint32_t ti = blockIdx.y;
+    const GemmGroupProb &P = ga.p[tail_problem(ga, ti)];
+    uint32_t tm, tn;
+    tile_coords(P.t_whole + (ti - P.tail0), P.tiles_m, P.tiles_n, tm, tn);
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < BM * BN; e += gridDim.x * 256) {
+        const int64_t row = (int64_t)tm * BM + e / BN, col = (int64_t)tn * BN + e % BN;
+        if (row >= P.m || col >= P.n) continue;
+        const double sum = sum_in_order(ga.ws + (int64_t)ti * ga.sk * BM * BN + e, ga.sk, BM * BN);
+        const int64_t addr = row * P.ldc + col;
+        if (ga.overwrite) P.C[addr] = ga.alpha * sum;
+        else P.C[addr] += ga.alpha * sum;
+    }
+}
+
+// Sums the K slices of each remainder tile in slice order and adds
+// alpha * sum to C (deterministic: the order does not depend on timing).
+template <int BM, int BN>
+__global__ __launch_bounds__(256) void split_reduce_kernel(GemmArgs g)
+{
+    const uint32_t t = blockIdx.y;  // remainder tile
+    uint32_t tm, tn;
+    tile_coords(g.t_full + t, g.tiles_m, g.tiles_n, tm, tn);
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < BM * BN; e += gridDim.x * 256) {
+        const int64_t row = (int64_t)tm * BM + e / BN, col = (int64_t)tn * BN + e % BN;
+        if (row >= g.m || col >= g.n) continue;
+        const double sum = sum_in_order(g.ws + (int64_t)t * g.sk * BM * BN + e, g.sk, BM * BN);
+        const int64_t addr = g.cview ? op_addr<kVK>(g.c, row, col) : row * g.c.ld + col;
+        if (g.overwrite) g.C[addr] = g.alpha * sum;
+        else g.C[addr] += g.alpha * sum;
+    }
+}
+
+// Large dynamic LDS needs the attribute once per kernel.
+template <typename K>
+int allow_lds(K kern, size_t lds, std::once_flag &once, hipError_t &err)
+{
+    if (lds > 65536)
+        std::call_once(once, [&] {
+            err = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        });
+    DTCF_HIP(err);
+    return DTCF_OK;
+}
+
+template <int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
+int launch_one(GemmArgs g, hipStream_t s)
+{
+    auto kern = gemm_f64_kernel<BM, BN, WM, WN, AM, BMD, DIRECT>;
+    constexpr size_t lds = (size_t)2 * (BM + BN) * BK * sizeof(double);
+    static std::once_flag once;
+    static hipError_t attr_err = hipSuccess;
+    int st = allow_lds(kern, lds, once, attr_err);
+    if (st != DTCF_OK) return st;
+    // Tail split: when the last wave of whole tiles would leave most slots
+    // idle, its tiles are cut into K slices that fill one wave instead.
+    int cus = 0;
+    st = gemm_device_cus(&cus);
+    if (st != DTCF_OK) return st;
+    const uint32_t T = g.tiles_m * g.tiles_n;
+    const uint32_t slots = (uint32_t)cus * (uint32_t)Occ<BM, BN>::v;
+    const int64_t nk = (g.k + BK - 1) / BK;
+    g.t_full = T;
+    g.sk = 1;
+    g.kchunk = nk;
+    uint32_t nsplit = 0, sk = 0;
+    gemm_tail_split(T, slots, nk, nsplit, sk);
+    if (sk >= 2) {
+        const int64_t kchunk = (nk + sk - 1) / sk;
+        sk = (uint32_t)((nk + kchunk - 1) / kchunk);
+        double *ws = nullptr;
+        st = gemm_workspace(s, (size_t)nsplit * sk * BM * BN * sizeof(double), &ws);
+        if (st != DTCF_OK) return st;
+        g.ws = ws;
+        g.t_full = T - nsplit;
+        g.sk = sk;
+        g.kchunk = kchunk;
+    }
+    const unsigned grid = g.t_full + (T - g.t_full) * g.sk;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds, s, g);
+    DTCF_HIP(hipGetLastError());
+    if (g.t_full < T) {
+        hipLaunchKernelGGL((split_reduce_kernel<BM, BN>), dim3((BM * BN + 255) / 256, T - g.t_full),
+                           dim3(256), 0, s, g);
+        DTCF_HIP(hipGetLastError());
+    }
+    return DTCF_OK;
+}
+
+template <int BM, int BN, int WM, int WN, bool DIRECT>
+int launch_modes(const GemmArgs &g, hipStream_t s)
+{
+    const int am = g.amode, bm = g.bmode;
+    if (am == kDK && bm == kDK) return launch_one<BM, BN, WM, WN, kDK, kDK, DIRECT>(g, s);
+    if (am == kDK && bm == kDMN) return launch_one<BM, BN, WM, WN, kDK, kDMN, DIRECT>(g, s);
+    if (am == kDMN && bm == kDK) return launch_one<BM, BN, WM, WN, kDMN, kDK, DIRECT>(g, s);
+    if (am == kDMN && bm == kDMN) return launch_one<BM, BN, WM, WN, kDMN, kDMN, DIRECT>(g, s);
+    if (am == kVK && bm == kVK) return launch_one<BM, BN, WM, WN, kVK, kVK, DIRECT>(g, s);
+    if (am == kVK && bm == kVMN) return launch_one<BM, BN, WM, WN, kVK, kVMN, DIRECT>(g, s);
+    if (am == kVMN && bm == kVK) return launch_one<BM, BN, WM, WN, kVMN, kVK, DIRECT>(g, s);
+    if (am == kVMN && bm == kVMN) return launch_one<BM, BN, WM, WN, kVMN, kVMN, DIRECT>(g, s);
+    set_error("gemm: unsupported operand mode combination");
+    return DTCF_ERR_INVALID;
+}
+
+template <int BM, int BN, int WM, int WN>
+int launch_tile(GemmArgs g, hipStream_t s)
+{
+    g.tiles_m = (uint32_t)((g.m + BM - 1) / BM);
+    g.tiles_n = (uint32_t)((g.n + BN - 1) / BN);
+    g.nfast = fast_steps(g.k, (g.amode == kDMN && g.m % 2) || (g.bmode == kDMN && g.n % 2),
+                         (g.amode >= kVK && g.a.blk) || (g.bmode >= kVK && g.b.blk));
+    // direct loads need every pair adjacent and 16-byte aligned
+    if (g.a.vec2 && g.b.vec2) return launch_modes<BM, BN, WM, WN, true>(g, s);
+    return launch_modes<BM, BN, WM, WN, false>(g, s);
+}
+
+template <int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
+int launch_group(GemmGroupArgs ga, hipStream_t s)
+{
+    auto kern = gemm_f64_group_kernel<BM, BN, WM, WN, AM, BMD, DIRECT>;
+    constexpr size_t lds = (size_t)2 * (BM + BN) * BK * sizeof(double);
+    static std::once_flag once;
+    static hipError_t attr_err = hipSuccess;
+    int st = allow_lds(kern, lds, once, attr_err);
+    if (st != DTCF_OK) return st;
+    uint64_t total = 0;
+    int64_t nk_min = INT64_MAX;
+    for (int i = 0; i < ga.np; i++) {
+        GemmGroupProb &P = ga.p[i];
+        P.tiles_m = (uint32_t)((P.m + BM - 1) / BM);
+        P.tiles_n = (uint32_t)((P.n + BN - 1) / BN);
+        P.nfast = fast_steps(P.k, (AM == kDMN && P.m % 2) || (BMD == kDMN && P.n % 2), false);
+        total += (uint64_t)P.tiles_m * P.tiles_n;
+        nk_min = std::min<int64_t>(nk_min, (P.k + BK - 1) / BK);
+    }
+    DTCF_REQUIRE(total + 8 * kGroupMax < (1ull << 31), "gemm group: too many tiles");
+    if (total == 0) return DTCF_OK;
+    // Tail split over the whole group: the last tiles (of the last
+    // problems, the shortest in K) are cut into K slices as a single GEMM's
+    // would be, with the shortest K of the group bounding the slice count.
+    int cus = 0;
+    st = gemm_device_cus(&cus);
+    if (st != DTCF_OK) return st;
+    uint32_t nsplit = 0, sk = 0;
+    gemm_tail_split((uint32_t)total, (uint32_t)cus * (uint32_t)Occ<BM, BN>::v, nk_min, nsplit, sk);
+    if (sk < 2) nsplit = 0;
+    ga.sk = sk < 2 ? 1 : sk;
+    ga.ws = nullptr;
+    if (nsplit) {
+        st = gemm_workspace(s, (size_t)nsplit * sk * BM * BN * sizeof(double), &ga.ws);
+        if (st != DTCF_OK) return st;
+    }
+    uint32_t left = nsplit;
+    for (int i = ga.np - 1; i >= 0; i--) {
+        GemmGroupProb &P = ga.p[i];
+        const uint32_t T = P.tiles_m * P.tiles_n, take = std::min(left, T);
+        P.t_whole = T - take;
+        left -= take;
+        const int64_t nk = (P.k + BK - 1) / BK;
+        P.kchunk = (nk + ga.sk - 1) / ga.sk;
+    }
+    uint64_t wg = 0;
+    uint32_t tail = 0;
+    for (int i = 0; i < ga.np; i++) {
+        GemmGroupProb &P = ga.p[i];
+        P.wg0 = (uint32_t)wg;
+        wg += ((uint64_t)P.t_whole + 7) & ~7ull;
+        P.tail0 = tail;
+        tail += P.tiles_m * P.tiles_n - P.t_whole;
+    }
+    ga.wg_whole = (uint32_t)wg;
+    const uint64_t grid = (uint64_t)ga.wg_whole + (uint64_t)nsplit * ga.sk;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NT), lds, s, ga);
+    DTCF_HIP(hipGetLastError());
+    if (nsplit) {
+        hipLaunchKernelGGL((group_split_reduce_kernel<BM, BN>), dim3((BM * BN + 255) / 256, nsplit),
+                           dim3(256), 0, s, ga);
+        DTCF_HIP(hipGetLastError());
+    }
+    return DTCF_OK;
+}
+
+template <int BM, int BN, int WM, int WN, bool DIRECT>
+int launch_group_modes(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s)
+{
+    if (amode == kDK && bmode == kDK) return launch_group<BM, BN, WM, WN, kDK, kDK, DIRECT>(ga, s);
+    if (amode == kDK && bmode == kDMN) return launch_group<BM, BN, WM, WN, kDK, kDMN, DIRECT>(ga, s);
+    if (amode == kDMN && bmode == kDK) return launch_group<BM, BN, WM, WN, kDMN, kDK, DIRECT>(ga, s);
+    if (amode == kDMN && bmode == kDMN) return launch_group<BM, BN, WM, WN, kDMN, kDMN, DIRECT>(ga, s);
+    set_error("gemm group: unsupported operand layout");
+    return DTCF_ERR_INVALID;
+}
+
+template <int BM, int BN, int WM, int WN>
+int launch_group_tile(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s)
+{
+    bool direct = true;
+    for (int i = 0; i < ga.np; i++) direct = direct && ga.p[i].vec2a && ga.p[i].vec2b;
+    if (direct) return launch_group_modes<BM, BN, WM, WN, true>(ga, amode, bmode, s);
+    return launch_group_modes<BM, BN, WM, WN, false>(ga, amode, bmode, s);
+}
+
+}  // namespace
+}  // namespace dtcf

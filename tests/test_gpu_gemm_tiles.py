@@ -1,0 +1,96 @@
+"""FP64 GEMM tiles at the sizes where their loads change form: whole and
+partial K steps of 16, odd extents and pitches, buffers off 16-byte
+alignment, and views whose pairs are adjacent, adjacent off alignment, or
+not adjacent.  Against torch's float64 product; every C element sums K
+products of N(0, 1) numbers, so the bound is 1e-12 of the largest result,
+as in test_gpu_core."""
+import numpy as np
+import pytest
+import torch
+
+from dtcf_amd import ops
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-12
+
+
+def _rand(n, seed, dev):
+    g = torch.Generator(device="cpu")
+    g.manual_seed(seed)
+    return torch.randn(n, dtype=torch.float64, generator=g).to(dev)
+
+
+def _close(got, ref, what):
+    err = ((got - ref).abs().max() / ref.abs().max().clamp_min(1e-300)).item()
+    assert err <= TOL, (what, err)
+
+
+@pytest.fixture
+def cfg_reset():
+    yield
+    ops.set_gemm_config(-1)
+
+
+SIZES = ((1, 1, 1), (1, 3, 17), (2, 64, 15), (63, 65, 16), (64, 64, 31), (65, 63, 32), (127, 129, 33),
+         (129, 255, 48), (131, 97, 113), (257, 191, 160))
+
+
+@pytest.mark.parametrize("cfg", [-1, 0, 1, 2, 3, 4, 5])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_dense_odd_sizes_and_pitches(dev, cfg_reset, cfg, ta, tb):
+    ops.set_gemm_config(cfg)
+    for m, n, k in SIZES:
+        for pad, off in ((0, 0), (1, 0), (2, 1), (3, 0)):
+            ra, ca = (k, m) if ta else (m, k)
+            rb, cb = (n, k) if tb else (k, n)
+            lda, ldb, ldc = ca + pad, cb + pad, n + pad
+            # buffers end with the operand's last element: no slack behind it
+            A = _rand(off + (ra - 1) * lda + ca, 1, dev)
+            B = _rand(off + (rb - 1) * ldb + cb, 2, dev)
+            C = _rand((m - 1) * ldc + n, 3, dev)
+            a = torch.as_strided(A, (ra, ca), (lda, 1), off)
+            b = torch.as_strided(B, (rb, cb), (ldb, 1), off)
+            ref = C.clone()
+            torch.as_strided(ref, (m, n), (ldc, 1)).add_(
+                0.5 * ((a.t() if ta else a).contiguous() @ (b.t() if tb else b).contiguous()))
+            print("dense", cfg, ta, tb, m, n, k, pad, off, flush=True)
+            ops.gemm(ta, tb, m, n, k, 0.5, A[off:], lda, B[off:], ldb, C, ldc)
+            _close(C, ref, (m, n, k, pad, off))
+
+
+def _offsets(rows, cols, kind, rng):
+    """rows x cols offset tables over a dense array: the columns (k...) or the
+    rows (r...) contiguous, in runs of an odd length, or off alignment."""
+    if kind == "k":
+        return np.arange(rows) * (cols + cols % 2), np.arange(cols)
+    if kind == "k odd":  # pairs adjacent, rows at odd offsets
+        return np.arange(rows) * (cols | 1), np.arange(cols)
+    if kind == "k runs":  # runs of 7 columns
+        return np.arange(rows) * 7, (np.arange(cols) // 7) * (7 * rows) + np.arange(cols) % 7
+    if kind == "r":
+        return np.arange(rows), np.arange(cols) * (rows + rows % 2)
+    if kind == "r odd":
+        return np.arange(rows), np.arange(cols) * (rows | 1)
+    if kind == "r runs":
+        return (np.arange(rows) // 5) * (5 * cols) + np.arange(rows) % 5, np.arange(cols) * 5
+    return rng.permutation(rows) * cols, rng.permutation(cols)  # neither
+
+
+@pytest.mark.parametrize("cfg", [-1, 0, 3, 4])
+@pytest.mark.parametrize("ka", ["k", "k odd", "k runs", "r", "r odd", "r runs", "none"])
+@pytest.mark.parametrize("kb", ["k", "k odd", "r odd", "r runs", "none"])
+def test_views_off_alignment(dev, cfg_reset, cfg, ka, kb):
+    ops.set_gemm_config(cfg)
+    rng = np.random.default_rng(5)
+    for m, n, k in ((66, 70, 34), (65, 129, 47), (140, 67, 16), (3, 5, 9)):
+        ra, ca = _offsets(m, k, ka, rng)
+        rb, cb = _offsets(n, k, kb, rng)
+        A, B = _rand(int(ra.max() + ca.max()) + 1, 4, dev), _rand(int(rb.max() + cb.max()) + 1, 5, dev)
+        C = _rand(m * n, 6, dev)
+        ia = torch.from_numpy(ra[:, None] + ca[None, :]).to(dev)
+        ib = torch.from_numpy(rb[:, None] + cb[None, :]).to(dev)
+        ref = C + (A[ia] @ B[ib].t().contiguous()).reshape(-1)
+        cv = ops.View(m, n, np.arange(m) * n, np.arange(n)) if m % 2 else None
+        print("view", cfg, ka, kb, m, n, k, flush=True)
+        ops.gemm_view(m, n, k, 1.0, A, ops.View(m, k, ra, ca), B, ops.View(n, k, rb, cb), C, cv, ldc=n)
+        _close(C, ref, (ka, kb, m, n, k))

@@ -27,25 +27,12 @@ static std::atomic<int> g_cfg{-1};
 
 int ccsd_scratch_setup(int dev);  // ccsd.hip
 
-// Tile-shape choice when no explicit configuration is set.  The table is
-// filled by the autotuner (dtcf_amd/autotune.py) from measurements on the
-// device; the defaults keep 128x128 everywhere except small grids, where a
-// smaller tile gives more workgroups, and thin results (64 or 96 wide), whose
-// tile matches their width.
+// Tile-shape choice when no explicit configuration is set.  (192 x 96 and 96
+// x 192 were never the fastest and are used only when forced.)
 int pick_config(int64_t m, int64_t n, int64_t k)
 {
     const int forced = g_cfg.load();
     if (forced >= 0) return forced;
-    // Measured on gfx950 (view operands, every configuration forced in turn):
-    // with K <= 1024 the 64 x 64 tile wins or ties at every shape (9216 x
-    // 9216 x 192: 42.6 against 30.8 TF/s; 36864 x 2304 x 768: 54.4 / 54.0):
-    // a short K loop leaves the tile prologue and epilogue a large share,
-    // and two workgroups per CU overlap them.  Longer K takes 128 x 128
-    // unless its padding costs more than 12% over 64 x 64's (m = 192: 256
-    // padded rows; 1000 x 1000 x 100000: 63.6 against 50.7 TF/s, with the
-    // few tiles split over K).  192 x 96 and 96 x 192 were never the
-    // fastest (9216^3: 42.8 / 47.1 against 67.0 TF/s) and are used only
-    // when forced.
     // Thin results (one side at most 48) with short K stream their long
     // operand past the thin one held in LDS (thin_f64_launch): 4.2 against
     // 3.2 TB/s at 7077888 x 48 x 192, even at 442368 rows, slower than 64 x
@@ -58,9 +45,31 @@ int pick_config(int64_t m, int64_t n, int64_t k)
         const int64_t w = std::max(m, n);
         if ((w + 191) / 192 * 192 <= 1.12 * ((w + 63) / 64 * 64)) return m >= n ? kCfg192x64 : kCfg64x192;
     }
+    // Measured on gfx950 with every configuration forced in turn.  K <= 1024:
+    // 64 x 64 wins or ties (9216 x 9216 x 192: 660 against 704 us, 9900 x 990
+    // x 100: 62 / 90; 36864 x 2304 x 768: 2095 / 2108): the epilogue is a large
+    // share, and four workgroups per CU overlap it.
     if (k <= 1024) return kCfg64x64;
+    // One side at most 128: the long operand is read once per 64 (128)
+    // columns, so 128 x 128 unless its padding costs more than 12% over 64 x
+    // 64's (10000 x 100 x 10000: 424 against 471 us).
     auto padded = [&](int64_t t) { return (double)((m + t - 1) / t * t) * (double)((n + t - 1) / t * t); };
-    return padded(128) <= 1.12 * padded(64) ? kCfg128x128 : kCfg64x64;
+    if (std::min(m, n) <= 128) return padded(128) <= 1.12 * padded(64) ? kCfg128x128 : kCfg64x64;
+    // Otherwise the shorter predicted time (gemm_split_plan): 128 x 128 runs 70
+    // TF/s on a large product, 64 x 64 62 to 64, but a quarter of the tile
+    // fills the last round and the edges better (2048^3: 286 / 265 us, 2400^3:
+    // 475 / 447, 700 x 700 x 5000: 117 / 95; 4096^3: 2008 / 2052, 9216^3: 22.7
+    // / 24.5 ms).
+    int cus = 0;
+    if (gemm_device_cus(&cus) != DTCF_OK) cus = 256;
+    auto predicted = [&](int cfg) {
+        const TileRate t = tile_rate(cfg);
+        const int64_t tm = (m + t.bm - 1) / t.bm, tn = (n + t.bn - 1) / t.bn;
+        if ((double)tm * tn >= 2147483648.0) return 1e300;
+        return gemm_split_plan((uint32_t)(tm * tn), (k + 15) / 16, tm * t.bm + tn * t.bn, cus, t).us;
+    };
+    // (within 2%, 128 x 128: it draws less on the L2s)
+    return predicted(kCfg64x64) < 0.98 * predicted(kCfg128x128) ? kCfg64x64 : kCfg128x128;
 }
 
 }  // namespace dtcf

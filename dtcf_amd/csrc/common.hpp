@@ -8,20 +8,18 @@
 
 namespace dtcf {
 
-// Sum of w[0], w[stride], ..., w[(n - 1) * stride] added in that order (the
-// K slices of a split product), with the loads issued eight at a time.
-__device__ inline double sum_in_order(const double *w, uint32_t n, int64_t stride)
+// sum + w[0] + w[stride] + ... + w[(n - 1) * stride], added in that order
+// (the K slices of a split product), with the loads issued eight at a time:
+// past the end they repeat the last one, so a short list costs one wait too.
+__device__ inline double sum_in_order(const double *w, uint32_t n, int64_t stride, double sum = 0.0)
 {
-    double sum = 0.0;
-    uint32_t i = 0;
-    for (; i + 8 <= n; i += 8) {
+    for (uint32_t i = 0; i < n; i += 8) {
         double v[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = w[(int64_t)(i + u) * stride];
+        for (int u = 0; u < 8; u++) v[u] = w[(int64_t)min(i + u, n - 1) * stride];
 #pragma unroll
-        for (int u = 0; u < 8; u++) sum += v[u];
+        for (int u = 0; u < 8; u++) sum = i + u < n ? sum + v[u] : sum;
     }
-    for (; i < n; i++) sum += w[(int64_t)i * stride];
     return sum;
 }
 

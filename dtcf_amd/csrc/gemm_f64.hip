@@ -27,7 +27,7 @@
 namespace dtcf {
 namespace {
 
-// CU count per device, and the tail-split workspace per (device, stream):
+// CU count per device, and the split workspace per (device, stream):
 // GEMMs enqueued on different streams never share a workspace; GEMMs on one
 // stream are ordered by it.
 std::mutex g_dev_mu;
@@ -79,39 +79,65 @@ int split_workspace(hipStream_t s, size_t need, double **ws)
 
 }  // namespace
 
-// How many of T tiles to cut into K slices (nsplit, the last ones) and
-// into how many (sk >= 2; sk < 2 means no split), for `slots` resident
-// workgroups and nk K steps per tile.  A last partial round of at most half
-// the slots: its tiles are cut to fill one round.  Under-filled grid (at
-// most half the slots): every tile is cut.  One partial round (more than
-// half the slots, at most all): every tile is cut into the sk <= 8 slices
-// that fill whole rounds best, within two rounds of slots, when that beats
-// the unsplit fill by 3% (a 340-tile GEMM on 512 slots: 3 slices, 1020
-// items in 2 rounds, 66% -> 99.6% of the slots busy).  In every case
-// nsplit * sk <= 2 * slots, and every slice is non-empty.
-void gemm_tail_split(uint32_t T, uint32_t slots, int64_t nk, uint32_t &nsplit, uint32_t &sk)
+TileRate tile_rate(int cfg)
 {
-    const uint32_t rem = T % slots;
-    nsplit = 0;
-    sk = 0;
-    if (T > slots && rem > 0 && rem <= slots / 2 && nk >= 32) {
-        nsplit = rem;
-        sk = std::min<uint32_t>(slots / rem, (uint32_t)(nk / 8));
-    } else if (T <= slots / 2 && nk >= 16) {
-        nsplit = T;
-        sk = std::min<uint32_t>(slots / T, (uint32_t)(nk / 4));
-    } else if (T <= slots && nk >= 32) {
-        double best = (double)T / slots;
-        for (uint32_t c = 2; c <= 8 && nk / c >= 8 && T * c <= 2 * slots; c++) {
-            const uint32_t items = T * c;
-            const double fill = (double)items / (double)(((items + slots - 1) / slots) * slots);
-            if (fill > best * 1.03) {
-                best = fill;
-                sk = c;
-            }
-        }
-        if (sk >= 2) nsplit = T;
+    // Measured with whole tiles, one to four workgroups on every CU: 256,
+    // 512 and 1024 tiles of 64 x 64 x 4096 in 195, 278 and 515 us, 256 and
+    // 512 tiles of 128 x 128 in 561 (x 4096) and 514 us (x 2048).
+    switch (cfg) {
+    case kCfg192x96: return {192, 96, 2, 2.25, {0.88, 1.0, 1.0, 1.0}};
+    case kCfg96x192: return {96, 192, 2, 2.25, {0.88, 1.0, 1.0, 1.0}};
+    case kCfg64x64: return {64, 64, 4, 0.50, {0.66, 0.925, 0.98, 1.0}};
+    case kCfg192x64: return {192, 64, 2, 1.52, {0.85, 1.0, 1.0, 1.0}};
+    case kCfg64x192: return {64, 192, 2, 1.52, {0.85, 1.0, 1.0, 1.0}};
+    default: return {128, 128, 2, 1.96, {0.895, 1.0, 1.0, 1.0}};
     }
+}
+
+SplitPlan gemm_split_plan(uint32_t T, int64_t nk, int64_t panel, int cus, const TileRate &t)
+{
+    const uint32_t slots = (uint32_t)cus * t.occ;
+    const double step = t.step_us;
+    // c workgroups on the busiest CU, each running `n` steps.  A step that
+    // reads `hbm` bytes no other tile reads (thin results with long K) is
+    // bound by HBM instead, or, with too few workgroups to hide it, by its
+    // latency: 32 x 32 x 524288 took 148 us in 256 runs and 104 in 512, 128 x
+    // 128 x 131072 105 and 92.
+    const double hbm = (double)panel * 16 * 8 / T, all = (double)(t.bm + t.bn) * 16 * 8;
+    auto run_us = [&](double n, uint32_t c) {
+        const double mfma = step * c / t.share[std::min<uint32_t>(c, 4) - 1];
+        const double lat = 2.5 * std::min(1.0, hbm / all);
+        return n * std::max({mfma, hbm * c * cus / 5.0e6, lat});
+    };
+    SplitPlan best;
+    const double whole = (double)(T / slots) * t.occ * nk * step;
+    const uint32_t R = T % slots;
+    best.us = whole;
+    if (R == 0) return best;
+    best.us += run_us((double)nk, (R + cus - 1) / cus);
+    const int64_t steps = (int64_t)R * nk;
+    // Starting workgroups takes about 12 ns each (1 / 8 of an XCD's 0.1 us).
+    // Splitting pays a second launch (4 us), writes and reads back its pieces
+    // (16 B per element at about 6 TB/s, L2 and the MALL helping) and waits
+    // for eight of a tile's pieces at a time.
+    best.us += 0.012 * R;
+    auto consider = [&](uint32_t W, double pieces) {
+        const double n = (double)((steps + W - 1) / W);
+        const double us = whole + run_us(n, (W + cus - 1) / cus) + 0.012 * W + 4.0 +
+                          pieces * t.bm * t.bn * 16.0 / 6.0e6 + 0.7 * (pieces / R / 8.0 + 1.0);
+        if (us < best.us) {
+            best.us = us;
+            best.nsplit = R;
+            best.sw = W;
+        }
+    };
+    // Runs of at least four steps: one, two, .. workgroups on every CU, and
+    // the even cuts of each tile, which leave fewer pieces.
+    for (int c = 1; c <= t.occ; c++)
+        if (steps >= 4 * (int64_t)cus * c) consider((uint32_t)cus * c, (double)R + (double)cus * c);
+    for (uint32_t c = 2; c <= 512 && (uint64_t)R * c <= slots && nk >= 4 * (int64_t)c; c++)
+        consider(R * c, (double)R * c);
+    return best;
 }
 
 int gemm_f64_group_launch(const GemmGroupArgs &ga, int cfg, int amode, int bmode, hipStream_t s)
@@ -137,13 +163,13 @@ int gemm_device_cus(int *cus) { return device_cus(cus); }
 
 int gemm_reserve_workspace(hipStream_t s)
 {
-    // nsplit * sk <= 2 * slots for every configuration, and slots <= 2 per
-    // CU for the tiles that split (Occ), so twice the largest tile area
-    // times two slots per CU bounds every request.
+    // Two slots of a tile per run and at most `occ` runs per CU
+    // (gemm_split_plan): twice the largest tile (192 x 96) times two runs per
+    // CU bounds every request.
     int cus = 0;
     int st = device_cus(&cus);
     if (st != DTCF_OK) return st;
-    const size_t tile = std::max<size_t>({128 * 128, 192 * 96, 96 * 192, 64 * 64, 192 * 64});
+    const size_t tile = std::max<size_t>({128 * 128, 192 * 96, 96 * 192, 2 * 64 * 64, 192 * 64});
     double *ws = nullptr;
     return split_workspace(s, (size_t)cus * 2 * 2 * tile * sizeof(double), &ws);
 }

@@ -57,11 +57,11 @@ struct GemmArgs {
     int32_t amode, bmode, cview;
     uint32_t tiles_m, tiles_n;
     int64_t nfast;  // K steps loaded without bounds checks (gemm_tile.hpp)
-    // Tail split: workgroups [0, t_full) own whole tiles; the remaining
-    // tiles t_full.. are split over K into `sk` slices of `kchunk` K steps
-    // each, written to `ws` and summed in slice order by a second kernel.
-    uint32_t t_full, sk;
-    int64_t kchunk;
+    // Split tiles: workgroups [0, t_full) own whole tiles; the K steps of the
+    // tiles from t_full on, `steps` in all, are cut into `sw` equal runs, one
+    // per workgroup (SplitPlan).
+    uint32_t t_full, sw;
+    int64_t steps;
     double *ws;
     // 0: C += alpha * A * B (every reference call site); 1: C = alpha * A * B
     // (C is neither cleared first nor read)
@@ -73,10 +73,10 @@ int gemm_f64_launch(GemmArgs g, int cfg, hipStream_t s);
 // Up to kGroupMax independent dense GEMMs C_p (+)= alpha * op(A_p) * op(B_p)
 // in one launch, every problem with the same operand layouts: A_p m x k
 // (kDK) or k x m (kDMN), B_p n x k (kDK) or k x n (kDMN); C_p row-major.
-// tiles_m, tiles_n, wg0, t_whole, tail0 and kchunk are filled in by the
+// tiles_m, tiles_n, wg0, t_whole, tail0 and step0 are filled in by the
 // launch: problem p's tiles [0, t_whole) run whole, its tiles [t_whole,
-// tiles) are tail tiles tail0.. of the launch, each cut into `sk` K slices
-// of kchunk steps (the tail split of a single GEMM, over the group).
+// tiles) are the split tiles tail0.. of the launch, whose K steps are the
+// steps step0.. of the `steps` that `sw` workgroups share (as in GemmArgs).
 constexpr int kGroupMax = 16;
 struct GemmGroupProb {
     int64_t m, n, k;
@@ -87,14 +87,15 @@ struct GemmGroupProb {
     int32_t vec2a, vec2b;
     uint32_t tiles_m, tiles_n, wg0;
     uint32_t t_whole, tail0;
-    int64_t kchunk, nfast;
+    int64_t step0, nfast;
 };
 struct GemmGroupArgs {
     double alpha;
     int32_t overwrite;
     int32_t np;
-    uint32_t wg_whole, sk;  // workgroups of whole tiles; K slices per tail tile
-    double *ws;             // tail slices, [tail tile][slice][BM][BN]
+    uint32_t wg_whole, sw;  // workgroups of whole tiles; runs of split tiles
+    int64_t steps;
+    double *ws;
     GemmGroupProb p[kGroupMax];
 };
 
@@ -109,8 +110,28 @@ int gemm_group_tile_128x128(const GemmGroupArgs &ga, int amode, int bmode, hipSt
 int gemm_group_tile_192x96(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s);
 int gemm_group_tile_96x192(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s);
 int gemm_group_tile_64x64(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s);
-// Which tiles a launch cuts over K (gemm_f64.hip).
-void gemm_tail_split(uint32_t T, uint32_t slots, int64_t nk, uint32_t &nsplit, uint32_t &sk);
+// How a launch of T tiles of nk K steps each fills the device: the last
+// `nsplit` tiles are cut over K.  Their nsplit * nk steps, tile after tile,
+// are dealt in `sw` equal runs to as many workgroups.  A run that covers a
+// whole tile writes C; the piece of a tile at the start of run w goes to
+// workspace slot 2 w, one at its end (when it is not also the start) to 2 w
+// + 1, and a second kernel adds each tile's pieces to C in K order.  `us` is
+// the predicted time, which also chooses between tiles (pick_config).
+struct SplitPlan {
+    uint32_t nsplit = 0, sw = 0;
+    double us = 0.0;
+};
+// What the prediction knows of a C tile: us per K step of a workgroup when
+// a CU's matrix cores are busy, workgroups per CU, and the share of the CU's
+// rate that 1, 2, .. workgroups reach.
+struct TileRate {
+    int bm, bn, occ;
+    double step_us, share[4];
+};
+TileRate tile_rate(int cfg);
+// panel: rows of A and B together that one K step of the whole product
+// reads (tiles_m bm + tiles_n bn, 0: much shared, as in a large product).
+SplitPlan gemm_split_plan(uint32_t T, int64_t nk, int64_t panel, int cus, const TileRate &t);
 
 int gemm_f64_group_launch(const GemmGroupArgs &ga, int cfg, int amode, int bmode, hipStream_t s);
 
@@ -152,7 +173,7 @@ constexpr int kThinDecline = 1;
 bool thin_shape(int64_t m, int64_t n, int64_t k, int64_t min_rows);
 int thin_f64_launch(const GemmArgs &g, hipStream_t s);
 
-// Allocates the tail-split workspace of stream `s` at the largest size any
+// Allocates the split workspace of stream `s` at the largest size any
 // GEMM on it can need, so later launches on `s` never allocate.
 int gemm_reserve_workspace(hipStream_t s);
 // The split workspace of stream `s` (grown to `need` bytes if smaller; work

@@ -162,6 +162,11 @@ struct Loader {
 #pragma unroll
         for (int i = 0; i < (DIRECT ? 0 : P); i++) stage[(w * P + i) * 64 + l] = reg[i];
     }
+    __device__ static inline int64_t addr(const OpArgs &o, int64_t r, int64_t c)
+    {
+        if constexpr (M::VIEW && DIRECT) return o.rofs[r] + o.cofs[c];  // no block table
+        else return op_addr<MODE>(o, r, c);
+    }
     // Loads and stores one K step element by element, zeros outside.
     __device__ inline void load_checked(const OpArgs &o, const double *base, d2 *stage, int64_t row0,
                                         int64_t rows, int64_t K, int64_t kt, int w, int l) const
@@ -172,8 +177,8 @@ struct Loader {
             const int64_t r = row0 + frag_row(f, l), c = kt * BK + frag_k(f, l);
             const int64_t r1 = M::KC ? r : r + 1, cc1 = M::KC ? c + 1 : c;
             d2 v = {0.0, 0.0};
-            if (r < rows && c < K) v.x = base[op_addr<MODE>(o, r, c)];
-            if (r1 < rows && cc1 < K) v.y = base[op_addr<MODE>(o, r1, cc1)];
+            if (r < rows && c < K) v.x = base[addr(o, r, c)];
+            if (r1 < rows && cc1 < K) v.y = base[addr(o, r1, cc1)];
             stage[f * 64 + l] = v;
         }
     }
@@ -193,7 +198,7 @@ __device__ inline void tile_coords(uint32_t q, uint32_t tiles_m, uint32_t tiles_
 }
 
 // One workgroup's share of a GEMM: logical tile q over K steps [kt0, kt1);
-// a split slice (split) writes raw partial sums to workspace slot sidx.
+// a piece of a split tile (split) writes raw sums to workspace slot sidx.
 template <int BM, int BN, int WM, int WN, int AMODE, int BMODE, bool DIRECT>
 __device__ __forceinline__ void gemm_tile(const GemmArgs &g, uint32_t q, int64_t kt0, int64_t kt1,
                                           bool split, uint32_t sidx)
@@ -296,6 +301,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, uint32_t q, int64_t
         if (!DIRECT && store_next) finish(s + 1);
     };
 
+    int s = -1;
     if (nf > 0) {
         la.init(g.a, g.A, m0, g.m, wave, lane);
         lb.init(g.b, g.B, n0, g.n, wave, lane);
@@ -303,27 +309,24 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, uint32_t q, int64_t
         lb.fetch(g.b, kt0, wave, lane);
         begin(0);
         finish(0);
-    } else if (n > 0) {
-        checked(0);
-    }
-    sync();
-    int s = 0;
-    for (; s + 1 < nf; s++) {
-        begin(s + 1);
-        compute(s, true);
         sync();
+        for (s = 0; s + 1 < nf; s++) {
+            begin(s + 1);
+            compute(s, true);
+            sync();
+        }
     }
     // the last unchecked step and the checked one, out of the loop's code
     for (; s < n; s++) {
         if (s + 1 < n) checked(s + 1);
-        compute(s, false);
+        if (s >= 0) compute(s, false);
         sync();
     }
 
     const int fr = lane & 15, fq = lane >> 4;
     if (split) {
-        // K slice of a remainder tile: raw partial sums to the workspace,
-        // laid out [slice index][BM][BN]; the reduce kernel adds them to C.
+        // raw sums to the workspace, [slot][BM][BN]; the reduce kernel adds
+        // the tile's pieces to C
         double *w = g.ws + (int64_t)sidx * BM * BN;
 #pragma unroll
         for (int i = 0; i < FM; i++)
@@ -392,35 +395,59 @@ inline int64_t fast_steps(int64_t k, bool odd_pairs, bool table)
     return (odd_pairs && k % BK == 0) ? k / BK - 1 : k / BK;
 }
 
+// Workgroups per CU: two of the large tiles (their LDS stages take 64-74
+// KiB each), four of 64 x 64 (32 KiB, 128 VGPRs).
 template <int BM, int BN>
 struct Occ {
-    // Two workgroups per CU (their LDS stages take 64-74 KiB each at the
-    // large tiles).
-    static constexpr int v = 2;
+    static constexpr int v = BM * BN <= 64 * 64 ? 4 : 2;
 };
+
+// First K step of run w of `sw` over `steps` (sw <= steps: no run is empty),
+// and the run that holds step s.
+// A 64-bit division is about a microsecond of a workgroup's start: 32 bits
+// where they hold.
+__device__ inline int64_t div_small(int64_t a, int64_t b)
+{
+    return ((a | b) >> 32) == 0 ? (int64_t)((uint32_t)a / (uint32_t)b) : a / b;
+}
+__device__ inline int64_t run_begin(uint32_t w, uint32_t sw, int64_t steps) { return div_small(w * steps, sw); }
+__device__ inline uint32_t run_of(int64_t s, uint32_t sw, int64_t steps)
+{
+    return (uint32_t)div_small((s + 1) * sw - 1, steps);
+}
+
+// Run index of a workgroup past the whole tiles: neighbouring runs, which
+// share tiles and operand panels, go to one XCD.
+__device__ inline uint32_t run_index(uint32_t i, uint32_t sw) { return (sw & 7u) ? i : (i & 7u) * (sw >> 3) + (i >> 3); }
 
 template <int BM, int BN, int WM, int WN, int AMODE, int BMODE, bool DIRECT>
 __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_kernel(GemmArgs g)
 {
     // Workgroups below t_full own whole tiles; their ids are first remapped
     // so consecutive tiles land on one XCD (its own L2).  Workgroups above
-    // own one K slice of a remainder tile.
+    // own one run of the split tiles' K steps each.
     const uint32_t bid = blockIdx.x;
-    const int64_t nk_all = (g.k + BK - 1) / BK;
-    uint32_t q, sidx = 0;
-    int64_t kt0 = 0, kt1 = nk_all;
-    bool split = false;
+    const int64_t nk = (g.k + BK - 1) / BK;
+    uint32_t q, slot = 0;
+    int64_t k0 = 0, left = nk;
     if (bid < g.t_full) {
         q = bid;
         if ((g.t_full & 7u) == 0) q = (bid & 7u) * (g.t_full >> 3) + (bid >> 3);
     } else {
-        split = true;
-        sidx = bid - g.t_full;
-        q = g.t_full + sidx / g.sk;
-        kt0 = (int64_t)(sidx % g.sk) * g.kchunk;
-        kt1 = min(nk_all, kt0 + g.kchunk);
+        const uint32_t w = run_index(bid - g.t_full, g.sw);
+        const int64_t s = run_begin(w, g.sw, g.steps), t = div_small(s, nk);
+        left = run_begin(w + 1, g.sw, g.steps) - s;
+        q = g.t_full + (uint32_t)t;
+        k0 = s - t * nk;
+        slot = 2 * w;
     }
-    gemm_tile<BM, BN, WM, WN, AMODE, BMODE, DIRECT>(g, q, kt0, kt1, split, sidx);
+    for (; left > 0; q++) {
+        const int64_t k1 = min(nk, k0 + left);
+        gemm_tile<BM, BN, WM, WN, AMODE, BMODE, DIRECT>(g, q, k0, k1, k0 > 0 || k1 < nk, slot);
+        left -= k1 - k0;
+        k0 = 0;
+        slot |= 1;
+    }
 }
 
 // Problem owning tail tile ti (tail tiles are numbered problem by problem).
@@ -442,15 +469,16 @@ __device__ inline int tail_problem(const GemmGroupArgs &ga, uint32_t ti)
 // work, one per XCD, was measured slower: 8 x 2048^3 55.0 against 56.6
 // TF/s, 2 x 4096 x 4096 x 2048 59.0 against 63.7.)  Workgroups past a
 // problem's last whole tile exit at once.  The workgroups after wg_whole
-// each own one K slice of a tail tile.
+// each own one run of the split tiles' K steps.
 template <int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
 __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_group_kernel(GemmGroupArgs ga)
 {
     const uint32_t bid = blockIdx.x;
     int p = 0;
-    uint32_t q, sidx = 0;
-    bool split = false;
-    if (bid < ga.wg_whole) {
+    uint32_t q = 0, w = 0;
+    int64_t s = 0, e = 1;
+    const bool whole = bid < ga.wg_whole;
+    if (whole) {
         for (int i = 1; i < ga.np; i++)
             if (bid >= ga.p[i].wg0) p = i;
         const GemmGroupProb &P = ga.p[p];
@@ -459,40 +487,89 @@ __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_group_kernel(Ge
         q = (local & 7u) * (T8 >> 3) + (local >> 3);
         if (q >= T) return;  // whole workgroup: no barrier has been reached
     } else {
-        split = true;
-        sidx = bid - ga.wg_whole;
-        const uint32_t ti = sidx / ga.sk;
-        p = tail_problem(ga, ti);
-        q = ga.p[p].t_whole + (ti - ga.p[p].tail0);
+        w = run_index(bid - ga.wg_whole, ga.sw);
+        s = run_begin(w, ga.sw, ga.steps);
+        e = run_begin(w + 1, ga.sw, ga.steps);
     }
-    const GemmGroupProb &P = ga.p[p];
-    const int64_t nk = (P.k + BK - 1) / BK;
-    int64_t kt0 = 0, kt1 = nk;
-    if (split) {
-        kt0 = min(nk, (int64_t)(sidx % ga.sk) * P.kchunk);
-        kt1 = min(nk, kt0 + P.kchunk);
+    for (uint32_t seg = 0; s < e; seg = 1) {
+        int64_t k0 = 0, k1;
+        if (!whole) {
+            p = 0;
+            for (int i = 1; i < ga.np; i++)  // problems without split tiles hold no steps
+                if (s >= ga.p[i].step0 && ga.p[i].t_whole < ga.p[i].tiles_m * ga.p[i].tiles_n) p = i;
+        }
+        const GemmGroupProb &P = ga.p[p];
+        const int64_t nk = (P.k + BK - 1) / BK;
+        if (whole) {
+            k1 = nk;
+            s = e;
+        } else {
+            const int64_t t = div_small(s - P.step0, nk);
+            q = P.t_whole + (uint32_t)t;
+            k0 = s - P.step0 - t * nk;
+            k1 = min(nk, k0 + (e - s));
+            s += k1 - k0;
+        }
+        GemmArgs g{};
+        g.m = P.m;
+        g.n = P.n;
+        g.k = P.k;
+        g.nfast = P.nfast;
+        g.alpha = ga.alpha;
+        g.A = P.A;
+        g.B = P.B;
+        g.C = P.C;
+        g.a.ld = P.lda;
+        g.b.ld = P.ldb;
+        g.c.ld = P.ldc;
+        g.tiles_m = P.tiles_m;
+        g.tiles_n = P.tiles_n;
+        g.overwrite = ga.overwrite;
+        g.ws = ga.ws;
+        gemm_tile<BM, BN, WM, WN, AM, BMD, DIRECT>(g, q, k0, k1, k0 > 0 || k1 < nk, 2 * w + seg);
     }
-    GemmArgs g{};
-    g.m = P.m;
-    g.n = P.n;
-    g.k = P.k;
-    g.nfast = P.nfast;
-    g.alpha = ga.alpha;
-    g.A = P.A;
-    g.B = P.B;
-    g.C = P.C;
-    g.a.ld = P.lda;
-    g.b.ld = P.ldb;
-    g.c.ld = P.ldc;
-    g.tiles_m = P.tiles_m;
-    g.tiles_n = P.tiles_n;
-    g.overwrite = ga.overwrite;
-    g.ws = ga.ws;
-    gemm_tile<BM, BN, WM, WN, AM, BMD, DIRECT>(g, q, kt0, kt1, split, sidx);
 }
 
-// Sums the K slices of each tail tile of a group in slice order and adds
-// alpha * sum to (or, overwriting, stores it in) the problem's C.
+// The pieces of a tile whose K steps are [s0, s0 + nk) of the split ones,
+// element e, added in K order (whole: one run covers the tile and wrote C).
+// One element per thread: the reduce is bound by the latency of its loads,
+// and four elements per thread (a quarter of the workgroups) took 15.7
+// instead of 13.3 us with the product at 1024 x 64 x 1024.
+__device__ inline double sum_pieces(const double *ws, int64_t s0, int64_t nk, uint32_t sw, int64_t steps,
+                                    int64_t tile, int e, bool &whole)
+{
+    const uint32_t w0 = run_of(s0, sw, steps), w1 = run_of(s0 + nk - 1, sw, steps);
+    whole = w0 == w1;
+    if (whole) return 0.0;
+    const double first = ws[(2 * (int64_t)w0 + (run_begin(w0, sw, steps) < s0)) * tile + e];
+    return sum_in_order(ws + 2 * ((int64_t)w0 + 1) * tile + e, w1 - w0, 2 * tile, first);
+}
+
+__device__ inline void put_sum(const GemmArgs &g, int64_t row, int64_t col, double sum)
+{
+    const int64_t addr = g.cview ? op_addr<kVK>(g.c, row, col) : row * g.c.ld + col;
+    if (g.overwrite) g.C[addr] = g.alpha * sum;
+    else g.C[addr] += g.alpha * sum;
+}
+
+// Adds alpha times the pieces of each split tile to (or, overwriting, stores
+// them in) C.
+template <int BM, int BN>
+__global__ __launch_bounds__(256) void split_reduce_kernel(GemmArgs g)
+{
+    const uint32_t t = blockIdx.y;  // split tile
+    uint32_t tm, tn;
+    tile_coords(g.t_full + t, g.tiles_m, g.tiles_n, tm, tn);
+    const int64_t nk = (g.k + BK - 1) / BK;
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    const int64_t row = (int64_t)tm * BM + e / BN, col = (int64_t)tn * BN + e % BN;
+    if (row >= g.m || col >= g.n) return;
+    bool whole;
+    const double sum = sum_pieces(g.ws, t * nk, nk, g.sw, g.steps, BM * BN, e, whole);
+    if (!whole) put_sum(g, row, col, sum);
+}
+
+// The same over a group.
 template <int BM, int BN>
 __global__ __launch_bounds__(256) void group_split_reduce_kernel(GemmGroupArgs ga)
 {
@@ -500,32 +577,19 @@ __global__ __launch_bounds__(256) void group_split_reduce_kernel(GemmGroupArgs g
     const GemmGroupProb &P = ga.p[tail_problem(ga, ti)];
     uint32_t tm, tn;
     tile_coords(P.t_whole + (ti - P.tail0), P.tiles_m, P.tiles_n, tm, tn);
-    for (int e = blockIdx.x * 256 + threadIdx.x; e < BM * BN; e += gridDim.x * 256) {
-        const int64_t row = (int64_t)tm * BM + e / BN, col = (int64_t)tn * BN + e % BN;
-        if (row >= P.m || col >= P.n) continue;
-        const double sum = sum_in_order(ga.ws + (int64_t)ti * ga.sk * BM * BN + e, ga.sk, BM * BN);
-        const int64_t addr = row * P.ldc + col;
-        if (ga.overwrite) P.C[addr] = ga.alpha * sum;
-        else P.C[addr] += ga.alpha * sum;
-    }
-}
-
-// Sums the K slices of each remainder tile in slice order and adds
-// alpha * sum to C (deterministic: the order does not depend on timing).
-template <int BM, int BN>
-__global__ __launch_bounds__(256) void split_reduce_kernel(GemmArgs g)
-{
-    const uint32_t t = blockIdx.y;  // remainder tile
-    uint32_t tm, tn;
-    tile_coords(g.t_full + t, g.tiles_m, g.tiles_n, tm, tn);
-    for (int e = blockIdx.x * 256 + threadIdx.x; e < BM * BN; e += gridDim.x * 256) {
-        const int64_t row = (int64_t)tm * BM + e / BN, col = (int64_t)tn * BN + e % BN;
-        if (row >= g.m || col >= g.n) continue;
-        const double sum = sum_in_order(g.ws + (int64_t)t * g.sk * BM * BN + e, g.sk, BM * BN);
-        const int64_t addr = g.cview ? op_addr<kVK>(g.c, row, col) : row * g.c.ld + col;
-        if (g.overwrite) g.C[addr] = g.alpha * sum;
-        else g.C[addr] += g.alpha * sum;
-    }
+    const int64_t nk = (P.k + BK - 1) / BK;
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    const int64_t row = (int64_t)tm * BM + e / BN, col = (int64_t)tn * BN + e % BN;
+    if (row >= P.m || col >= P.n) return;
+    bool whole;
+    const double sum = sum_pieces(ga.ws, P.step0 + (ti - P.tail0) * nk, nk, ga.sw, ga.steps, BM * BN, e, whole);
+    if (whole) return;
+    GemmArgs g{};
+    g.C = P.C;
+    g.c.ld = P.ldc;
+    g.alpha = ga.alpha;
+    g.overwrite = ga.overwrite;
+    put_sum(g, row, col, sum);
 }
 
 // Large dynamic LDS needs the attribute once per kernel.
@@ -541,7 +605,7 @@ int allow_lds(K kern, size_t lds, std::once_flag &once, hipError_t &err)
     return DTCF_OK;
 }
 
-template <int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
+template <int CFG, int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
 int launch_one(GemmArgs g, hipStream_t s)
 {
     auto kern = gemm_f64_kernel<BM, BN, WM, WN, AM, BMD, DIRECT>;
@@ -550,58 +614,45 @@ int launch_one(GemmArgs g, hipStream_t s)
     static hipError_t attr_err = hipSuccess;
     int st = allow_lds(kern, lds, once, attr_err);
     if (st != DTCF_OK) return st;
-    // Tail split: when the last wave of whole tiles would leave most slots
-    // idle, its tiles are cut into K slices that fill one wave instead.
     int cus = 0;
     st = gemm_device_cus(&cus);
     if (st != DTCF_OK) return st;
     const uint32_t T = g.tiles_m * g.tiles_n;
-    const uint32_t slots = (uint32_t)cus * (uint32_t)Occ<BM, BN>::v;
     const int64_t nk = (g.k + BK - 1) / BK;
-    g.t_full = T;
-    g.sk = 1;
-    g.kchunk = nk;
-    uint32_t nsplit = 0, sk = 0;
-    gemm_tail_split(T, slots, nk, nsplit, sk);
-    if (sk >= 2) {
-        const int64_t kchunk = (nk + sk - 1) / sk;
-        sk = (uint32_t)((nk + kchunk - 1) / kchunk);
-        double *ws = nullptr;
-        st = gemm_workspace(s, (size_t)nsplit * sk * BM * BN * sizeof(double), &ws);
+    const SplitPlan sp = gemm_split_plan(T, nk, (int64_t)g.tiles_m * BM + (int64_t)g.tiles_n * BN, cus, tile_rate(CFG));
+    g.t_full = T - sp.nsplit;
+    g.sw = sp.sw;
+    g.steps = (int64_t)sp.nsplit * nk;
+    if (sp.nsplit) {
+        st = gemm_workspace(s, (size_t)2 * sp.sw * BM * BN * sizeof(double), &g.ws);
         if (st != DTCF_OK) return st;
-        g.ws = ws;
-        g.t_full = T - nsplit;
-        g.sk = sk;
-        g.kchunk = kchunk;
     }
-    const unsigned grid = g.t_full + (T - g.t_full) * g.sk;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds, s, g);
+    hipLaunchKernelGGL(kern, dim3(g.t_full + g.sw), dim3(NT), lds, s, g);
     DTCF_HIP(hipGetLastError());
-    if (g.t_full < T) {
-        hipLaunchKernelGGL((split_reduce_kernel<BM, BN>), dim3((BM * BN + 255) / 256, T - g.t_full),
-                           dim3(256), 0, s, g);
+    if (sp.nsplit) {
+        hipLaunchKernelGGL((split_reduce_kernel<BM, BN>), dim3(BM * BN / 256, sp.nsplit), dim3(256), 0, s, g);
         DTCF_HIP(hipGetLastError());
     }
     return DTCF_OK;
 }
 
-template <int BM, int BN, int WM, int WN, bool DIRECT>
+template <int CFG, int BM, int BN, int WM, int WN, bool DIRECT>
 int launch_modes(const GemmArgs &g, hipStream_t s)
 {
     const int am = g.amode, bm = g.bmode;
-    if (am == kDK && bm == kDK) return launch_one<BM, BN, WM, WN, kDK, kDK, DIRECT>(g, s);
-    if (am == kDK && bm == kDMN) return launch_one<BM, BN, WM, WN, kDK, kDMN, DIRECT>(g, s);
-    if (am == kDMN && bm == kDK) return launch_one<BM, BN, WM, WN, kDMN, kDK, DIRECT>(g, s);
-    if (am == kDMN && bm == kDMN) return launch_one<BM, BN, WM, WN, kDMN, kDMN, DIRECT>(g, s);
-    if (am == kVK && bm == kVK) return launch_one<BM, BN, WM, WN, kVK, kVK, DIRECT>(g, s);
-    if (am == kVK && bm == kVMN) return launch_one<BM, BN, WM, WN, kVK, kVMN, DIRECT>(g, s);
-    if (am == kVMN && bm == kVK) return launch_one<BM, BN, WM, WN, kVMN, kVK, DIRECT>(g, s);
-    if (am == kVMN && bm == kVMN) return launch_one<BM, BN, WM, WN, kVMN, kVMN, DIRECT>(g, s);
+    if (am == kDK && bm == kDK) return launch_one<CFG, BM, BN, WM, WN, kDK, kDK, DIRECT>(g, s);
+    if (am == kDK && bm == kDMN) return launch_one<CFG, BM, BN, WM, WN, kDK, kDMN, DIRECT>(g, s);
+    if (am == kDMN && bm == kDK) return launch_one<CFG, BM, BN, WM, WN, kDMN, kDK, DIRECT>(g, s);
+    if (am == kDMN && bm == kDMN) return launch_one<CFG, BM, BN, WM, WN, kDMN, kDMN, DIRECT>(g, s);
+    if (am == kVK && bm == kVK) return launch_one<CFG, BM, BN, WM, WN, kVK, kVK, DIRECT>(g, s);
+    if (am == kVK && bm == kVMN) return launch_one<CFG, BM, BN, WM, WN, kVK, kVMN, DIRECT>(g, s);
+    if (am == kVMN && bm == kVK) return launch_one<CFG, BM, BN, WM, WN, kVMN, kVK, DIRECT>(g, s);
+    if (am == kVMN && bm == kVMN) return launch_one<CFG, BM, BN, WM, WN, kVMN, kVMN, DIRECT>(g, s);
     set_error("gemm: unsupported operand mode combination");
     return DTCF_ERR_INVALID;
 }
 
-template <int BM, int BN, int WM, int WN>
+template <int CFG, int BM, int BN, int WM, int WN>
 int launch_tile(GemmArgs g, hipStream_t s)
 {
     g.tiles_m = (uint32_t)((g.m + BM - 1) / BM);
@@ -609,11 +660,11 @@ int launch_tile(GemmArgs g, hipStream_t s)
     g.nfast = fast_steps(g.k, (g.amode == kDMN && g.m % 2) || (g.bmode == kDMN && g.n % 2),
                          (g.amode >= kVK && g.a.blk) || (g.bmode >= kVK && g.b.blk));
     // direct loads need every pair adjacent and 16-byte aligned
-    if (g.a.vec2 && g.b.vec2) return launch_modes<BM, BN, WM, WN, true>(g, s);
-    return launch_modes<BM, BN, WM, WN, false>(g, s);
+    if (g.a.vec2 && g.b.vec2) return launch_modes<CFG, BM, BN, WM, WN, true>(g, s);
+    return launch_modes<CFG, BM, BN, WM, WN, false>(g, s);
 }
 
-template <int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
+template <int CFG, int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
 int launch_group(GemmGroupArgs ga, hipStream_t s)
 {
     auto kern = gemm_f64_group_kernel<BM, BN, WM, WN, AM, BMD, DIRECT>;
@@ -623,80 +674,78 @@ int launch_group(GemmGroupArgs ga, hipStream_t s)
     int st = allow_lds(kern, lds, once, attr_err);
     if (st != DTCF_OK) return st;
     uint64_t total = 0;
-    int64_t nk_min = INT64_MAX;
+    int64_t steps = 0;
     for (int i = 0; i < ga.np; i++) {
         GemmGroupProb &P = ga.p[i];
         P.tiles_m = (uint32_t)((P.m + BM - 1) / BM);
         P.tiles_n = (uint32_t)((P.n + BN - 1) / BN);
         P.nfast = fast_steps(P.k, (AM == kDMN && P.m % 2) || (BMD == kDMN && P.n % 2), false);
         total += (uint64_t)P.tiles_m * P.tiles_n;
-        nk_min = std::min<int64_t>(nk_min, (P.k + BK - 1) / BK);
+        steps += (int64_t)P.tiles_m * P.tiles_n * ((P.k + BK - 1) / BK);
     }
     DTCF_REQUIRE(total + 8 * kGroupMax < (1ull << 31), "gemm group: too many tiles");
     if (total == 0) return DTCF_OK;
-    // Tail split over the whole group: the last tiles (of the last
-    // problems, the shortest in K) are cut into K slices as a single GEMM's
-    // would be, with the shortest K of the group bounding the slice count.
+    // The split is planned for the group's mean K and taken from the last
+    // problems (the shortest in K).
     int cus = 0;
     st = gemm_device_cus(&cus);
     if (st != DTCF_OK) return st;
-    uint32_t nsplit = 0, sk = 0;
-    gemm_tail_split((uint32_t)total, (uint32_t)cus * (uint32_t)Occ<BM, BN>::v, nk_min, nsplit, sk);
-    if (sk < 2) nsplit = 0;
-    ga.sk = sk < 2 ? 1 : sk;
-    ga.ws = nullptr;
-    if (nsplit) {
-        st = gemm_workspace(s, (size_t)nsplit * sk * BM * BN * sizeof(double), &ga.ws);
-        if (st != DTCF_OK) return st;
-    }
-    uint32_t left = nsplit;
+    const SplitPlan sp = gemm_split_plan((uint32_t)total, std::max<int64_t>(1, steps / (int64_t)total), 0, cus,
+                                         tile_rate(CFG));
+    uint32_t left = sp.nsplit;
     for (int i = ga.np - 1; i >= 0; i--) {
         GemmGroupProb &P = ga.p[i];
         const uint32_t T = P.tiles_m * P.tiles_n, take = std::min(left, T);
         P.t_whole = T - take;
         left -= take;
-        const int64_t nk = (P.k + BK - 1) / BK;
-        P.kchunk = (nk + ga.sk - 1) / ga.sk;
     }
     uint64_t wg = 0;
     uint32_t tail = 0;
+    ga.steps = 0;
     for (int i = 0; i < ga.np; i++) {
         GemmGroupProb &P = ga.p[i];
         P.wg0 = (uint32_t)wg;
         wg += ((uint64_t)P.t_whole + 7) & ~7ull;
         P.tail0 = tail;
-        tail += P.tiles_m * P.tiles_n - P.t_whole;
+        P.step0 = ga.steps;
+        const uint32_t cut = P.tiles_m * P.tiles_n - P.t_whole;
+        tail += cut;
+        ga.steps += cut * ((P.k + BK - 1) / BK);
     }
     ga.wg_whole = (uint32_t)wg;
-    const uint64_t grid = (uint64_t)ga.wg_whole + (uint64_t)nsplit * ga.sk;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NT), lds, s, ga);
+    ga.sw = (uint32_t)std::min<int64_t>(sp.sw, ga.steps);
+    ga.ws = nullptr;
+    if (ga.sw) {
+        st = gemm_workspace(s, (size_t)2 * ga.sw * BM * BN * sizeof(double), &ga.ws);
+        if (st != DTCF_OK) return st;
+    }
+    hipLaunchKernelGGL(kern, dim3(ga.wg_whole + ga.sw), dim3(NT), lds, s, ga);
     DTCF_HIP(hipGetLastError());
-    if (nsplit) {
-        hipLaunchKernelGGL((group_split_reduce_kernel<BM, BN>), dim3((BM * BN + 255) / 256, nsplit),
-                           dim3(256), 0, s, ga);
+    if (ga.sw) {
+        hipLaunchKernelGGL((group_split_reduce_kernel<BM, BN>), dim3(BM * BN / 256, sp.nsplit), dim3(256), 0, s, ga);
         DTCF_HIP(hipGetLastError());
     }
     return DTCF_OK;
 }
 
-template <int BM, int BN, int WM, int WN, bool DIRECT>
+template <int CFG, int BM, int BN, int WM, int WN, bool DIRECT>
 int launch_group_modes(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s)
 {
-    if (amode == kDK && bmode == kDK) return launch_group<BM, BN, WM, WN, kDK, kDK, DIRECT>(ga, s);
-    if (amode == kDK && bmode == kDMN) return launch_group<BM, BN, WM, WN, kDK, kDMN, DIRECT>(ga, s);
-    if (amode == kDMN && bmode == kDK) return launch_group<BM, BN, WM, WN, kDMN, kDK, DIRECT>(ga, s);
-    if (amode == kDMN && bmode == kDMN) return launch_group<BM, BN, WM, WN, kDMN, kDMN, DIRECT>(ga, s);
+    if (amode == kDK && bmode == kDK) return launch_group<CFG, BM, BN, WM, WN, kDK, kDK, DIRECT>(ga, s);
+    if (amode == kDK && bmode == kDMN) return launch_group<CFG, BM, BN, WM, WN, kDK, kDMN, DIRECT>(ga, s);
+    if (amode == kDMN && bmode == kDK) return launch_group<CFG, BM, BN, WM, WN, kDMN, kDK, DIRECT>(ga, s);
+    if (amode == kDMN && bmode == kDMN) return launch_group<CFG, BM, BN, WM, WN, kDMN, kDMN, DIRECT>(ga, s);
     set_error("gemm group: unsupported operand layout");
     return DTCF_ERR_INVALID;
 }
 
-template <int BM, int BN, int WM, int WN>
+template <int CFG, int BM, int BN, int WM, int WN>
 int launch_group_tile(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s)
 {
     bool direct = true;
     for (int i = 0; i < ga.np; i++) direct = direct && ga.p[i].vec2a && ga.p[i].vec2b;
-    if (direct) return launch_group_modes<BM, BN, WM, WN, true>(ga, amode, bmode, s);
-    return launch_group_modes<BM, BN, WM, WN, false>(ga, amode, bmode, s);
+    if (direct) return launch_group_modes<CFG, BM, BN, WM, WN, true>(ga, amode, bmode, s);
+    return launch_group_modes<CFG, BM, BN, WM, WN, false>(ga, amode, bmode, s);
 }
 
 }  // namespace

@@ -495,7 +495,7 @@ typedef struct dtcf_program_s *dtcf_program;
 /* Opens a server on the current device: one device arena of `budget`
  * bytes (resident tensors and request blocks are carved out of it) and
  * `nslots` (1..16) non-blocking streams of default priority.  Each slot
- * also keeps a GEMM tail-split workspace (under 80 MB) outside the arena. */
+ * also keeps a GEMM split workspace (at most 151 MB) outside the arena. */
 int dtcf_server_open(int64_t budget, int nslots, dtcf_server *out);
 /* Waits for every admitted request (queued requests that can no longer be
  * admitted fail with DTCF_ERR_BUDGET), then frees everything. */

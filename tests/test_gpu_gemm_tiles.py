@@ -94,3 +94,32 @@ def test_views_off_alignment(dev, cfg_reset, cfg, ka, kb):
         print("view", cfg, ka, kb, m, n, k, flush=True)
         ops.gemm_view(m, n, k, 1.0, A, ops.View(m, k, ra, ca), B, ops.View(n, k, rb, cb), C, cv, ldc=n)
         _close(C, ref, (ka, kb, m, n, k))
+
+
+# Grids where the last tiles' K steps are dealt in runs: fewer tiles than
+# workgroup slots, a little and a lot over whole rounds of slots, runs that
+# cover several pieces of tiles, and K with a checked last step.
+@pytest.mark.parametrize("cfg,m,n,k", [(3, 64, 64, 4096), (3, 500, 500, 500), (3, 130, 70, 3001),
+                                       (3, 2112, 2112, 80), (3, 2200, 2050, 333), (0, 128, 128, 9000),
+                                       (0, 1300, 1200, 700), (0, 2400, 2400, 171), (0, 2944, 2944, 100),
+                                       (4, 192, 48, 20001), (5, 48, 192, 20001), (1, 1000, 900, 800)])
+@pytest.mark.parametrize("overwrite_view", [False, True])
+def test_split_runs(dev, cfg_reset, cfg, m, n, k, overwrite_view):
+    ops.set_gemm_config(cfg)
+    A, B, C = _rand(m * k, 7, dev), _rand(n * k, 8, dev), _rand(m * n, 9, dev)
+    ref = C.view(m, n) - 2.0 * (A.view(m, k) @ B.view(n, k).t().contiguous())
+    print("split", cfg, m, n, k, overwrite_view, flush=True)
+    outs = []
+    for _ in range(2):
+        X = C.clone()
+        if overwrite_view:  # C through a view of its transpose
+            X = X.view(m, n).t().contiguous().reshape(-1)
+            v = ops.View(m, n, np.arange(m), np.arange(n) * m)
+            ops.gemm_view(m, n, k, -2.0, A, ops.View(m, k, np.arange(m) * k, np.arange(k)), B,
+                          ops.View(n, k, np.arange(n) * k, np.arange(k)), X, v)
+            outs.append(X.view(n, m).t().contiguous())
+        else:
+            ops.gemm(0, 1, m, n, k, -2.0, A, k, B, k, X, n)
+            outs.append(X.view(m, n))
+    _close(outs[0], ref, (cfg, m, n, k))
+    assert torch.equal(outs[0], outs[1])  # the order of the additions is fixed

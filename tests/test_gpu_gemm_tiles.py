@@ -123,3 +123,26 @@ def test_split_runs(dev, cfg_reset, cfg, m, n, k, overwrite_view):
             outs.append(X.view(m, n))
     _close(outs[0], ref, (cfg, m, n, k))
     assert torch.equal(outs[0], outs[1])  # the order of the additions is fixed
+
+
+@pytest.mark.parametrize("sizes", [{"Oa": 5, "Ob": 4, "Va": 23, "Vb": 22}, {"Oa": 4, "Ob": 7, "Va": 21, "Vb": 19}])
+def test_served_odd_extents_read_in_place(dev, sizes):
+    # operands with odd extents are read in place in runs, not copied; small
+    # enough for the einsum oracle, large enough (rows * K >= 65536) that the
+    # rule applies
+    import oracle
+    from dtcf_amd import serve, termlist
+
+    tl = termlist.load("t2")
+    with serve.Server(1 << 30, 4) as srv:
+        system = serve.System(srv, 0, 0, [tl], seed=3, sizes=sizes)
+        prog = serve.Program(srv, tl, system)
+        print("served", sizes, flush=True)
+        got = prog.run()
+        prog.destroy()
+        stms = [(s.lhs.name, s.kind, s.lhs.idx, [(t.name, t.idx) + ((t.coef,) if s.kind == "sum" else ())
+                                                 for t in s.terms]) for s in tl.statements]
+        ref = oracle.termlist_run(stms, {n: system.host(n) for n in tl.inputs()})
+    for n, x in got.items():
+        err = np.abs(x - ref[n]).max() / np.abs(ref[n]).max()
+        assert err <= TOL, (n, err)

@@ -133,7 +133,7 @@ SplitPlan gemm_split_plan(uint32_t T, int64_t nk, int64_t panel, int cus, const 
     };
     // Runs of at least four steps: one, two, .. workgroups on every CU, and
     // the even cuts of each tile, which leave fewer pieces.
-    for (int c = 1; c <= t.occ; c++)
+    for (int c = 1; c <= t.occ && !t.even; c++)
         if (steps >= 4 * (int64_t)cus * c) consider((uint32_t)cus * c, (double)R + (double)cus * c);
     for (uint32_t c = 2; c <= 512 && (uint64_t)R * c <= slots && nk >= 4 * (int64_t)c; c++)
         consider(R * c, (double)R * c);

@@ -123,10 +123,13 @@ struct SplitPlan {
 };
 // What the prediction knows of a C tile: us per K step of a workgroup when
 // a CU's matrix cores are busy, workgroups per CU, and the share of the CU's
-// rate that 1, 2, .. workgroups reach.
+// rate that 1, 2, .. workgroups reach.  even: only cuts of every split tile
+// into equal runs, which keep the workgroups on a few common K positions (a
+// kernel whose operand panels must be shared through the L2s).
 struct TileRate {
     int bm, bn, occ;
     double step_us, share[4];
+    bool even = false;
 };
 TileRate tile_rate(int cfg);
 // panel: rows of A and B together that one K step of the whole product

@@ -25,12 +25,14 @@
 // applications", Numer. Algorithms 59 (2012), with integer slices).
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <vector>
 
 #include <climits>
 
 #include "common.hpp"
 #include "gemm_f64.hpp"
+#include "runs.hpp"
 #include "view.hpp"
 
 namespace dtcf {
@@ -814,14 +816,13 @@ __global__ __launch_bounds__(256, 2) void lp_gemm_kernel(LPArgs g)
 // FP16 slices (64 bytes = 32 elements per step, the same fragment bytes and
 // lane order) sum in FP32 and reach C once.
 //
-// Workgroup: C tile 128 x 128 (wave layout below).  LDS holds K steps as
+// Workgroup: 8 waves (2 per SIMD) over one C tile; LDS holds two K steps as
 // fragments of 1 KiB ([operand digit][16-row block][lane][16 B], the order
 // of the digit planes themselves: lane = row % 16 + 16 * kq holds bytes
 // 16kq..16kq+15 of the 64-byte step of its row); each fragment is one
 // direct global->LDS load of 64 lanes x 16 B of one contiguous KiB.
-// `ozaki_kernel` keeps two full stages (16 * NS fragments each, loaded a
-// step ahead); `ozaki_ring_kernel` (NS <= 4) five half stages.
-constexpr int OZ_BM = 128, OZ_BN = 128, OZ_BK = 64;
+constexpr int OZ_BK = 64;
+constexpr int OZ_WAVES = 8;
 
 struct OzArgs {
     const unsigned char *A, *B;  // slice planes [NS][Mp][Kp bytes], [NS][Np][Kp bytes]
@@ -829,31 +830,34 @@ struct OzArgs {
     double alpha;
     int64_t M, N, Kp, Mp, Np;    // Kp: bytes of K per slice row (a multiple of 64)
     int64_t kchunk_steps;        // K steps between INT32 flushes
-    // K split: workgroups [0, t_full) own whole tiles; workgroup t_full + s
-    // computes tile t_full + s / sk over K steps [(s % sk) * kslice, +
-    // kslice) and leaves alpha * its sum in ws[s] (OZ_BM x OZ_BN);
-    // oz_split_reduce adds the slices of tiles t_full.. to C in order.
-    uint32_t t_full, sk;
-    int64_t kslice;
+    // Split tiles (SplitPlan): workgroups [0, t_full) own whole tiles, the
+    // others one run each of the K steps of the tiles from t_full on, leaving
+    // alpha times the pieces in ws; oz_split_reduce adds them to C in K order.
+    uint32_t t_full, sw;
+    int64_t steps;
     double *ws;
     double *C;
     ViewArgs cv;
     int64_t ldc;
     uint32_t tiles_m, tiles_n;
-    // 1: C = alpha * A B^T (the first write of each element stores, no read
-    // of C); 0: C += alpha * A B^T
-    int overwrite;
+    // cview: C through cv; overwrite 1: C = alpha * A B^T (the first write of
+    // each element stores, no read of C); 0: C += alpha * A B^T
+    int32_t cview, overwrite;
 };
 
-// Workgroup of 8 waves (2 per SIMD) as 4 x 2, each owning 32 x 64 of the
-// 128 x 128 tile as 2 x 4 MFMA blocks; the LDS stages take all 160 KiB (two
-// stages at NS = 5, five half stages at NS = 4).  The tile is as large as
-// the registers allow (L - 1 INT32 level sums per C element): every
-// workgroup streams 16 * NS KiB of digit planes per K step, the loads'
-// latency is the kernel's limit, and a 64 x 128 tile (1.5x the traffic per
-// product) ran 15-25% slower, two 64 x 64 workgroups per CU slower still.
-constexpr int OZ_WAVES = 8, OZ_WM = 32, OZ_WN = 64;
-constexpr int OZ_FM = OZ_WM / 16, OZ_FN = OZ_WN / 16;  // MFMA blocks per wave
+// C tile of each specialisation.  Every workgroup streams its NS planes of
+// BM + BN rows per step and reads each fragment BN / WN or BM / WM times from
+// LDS, so a larger tile per wave is worth its registers (L - 1 level sums
+// per C element).  Three products' levels (L = 4) fit 128 x 192 (64 x 48 per
+// wave) and 192 x 128 (48 x 64); 256 x 128 spills, and levels 5 and 6 have
+// registers for 128 x 128 (32 x 64) only.
+template <int BM_, int BN_>
+struct OzTile {
+    static constexpr int BM = BM_, BN = BN_;
+    static constexpr int WM = BM == 192 ? 48 : BN == 192 ? 64 : 32, WN = BM == 192 ? 64 : BN == 192 ? 48 : 64;
+    static constexpr int FM = WM / 16, FN = WN / 16;  // MFMA blocks per wave
+    static_assert((BM / WM) * (BN / WN) == OZ_WAVES, "eight waves per tile");
+};
 
 // Element traits of the fused kernels: the MFMA over one 16-byte fragment
 // per lane (64 bytes of K of 16 rows) and its accumulator.  A level's sum is
@@ -888,349 +892,272 @@ struct OzT<DTCF_PREC_F16X3> {
     }
 };
 
-template <int P, int NS, int L, bool CVIEW>
+// Level sums of one tile (or a piece of one: wsp) to C: scaled, added
+// smallest first.  Sixteen rows at a time: addresses, the old values in one
+// batch of loads, then the stores (the scheduling barriers keep one batch's
+// registers from piling on the next's).
+template <int P, int L, typename T>
 __device__ __forceinline__ void oz_flush(const OzArgs &g,
-                                         typename OzT<P>::Acc (&acc)[L - 1][OZ_FM][OZ_FN],
+                                         typename OzT<P>::Acc (&acc)[L - 1][T::FM][T::FN],
                                          int64_t m0, int64_t n0, int wm, int wn, int lane,
                                          double *wsp, bool first)
 {
+    // opaque to the compiler, which otherwise computes every address below
+    // before the K loop and spills them across it
+    asm volatile("" : "+v"(lane));
     const int fr = lane & 15, fq = lane >> 4;
+    const bool add = wsp ? !first : !(g.overwrite && first);
+    double *out = wsp ? wsp : g.C;
+    constexpr int JB = L > 4 && T::FN % 2 == 0 ? 2 : T::FN;  // columns of blocks per batch
 #pragma unroll
-    for (int j = 0; j < OZ_FN; j++) {
-        const int64_t col = n0 + wn * OZ_WN + j * 16 + fr;
-        if (col >= g.N) continue;
-        const int ebc = P == DTCF_PREC_BF16X3 ? 0 : g.eb[col];
-        int64_t cof;
-        if constexpr (CVIEW) cof = g.cv.cofs[col];
-        else cof = col;
+    for (int i = 0; i < T::FM; i++) {
+        int ea[4];
+        int64_t ro[4];
 #pragma unroll
-        for (int i = 0; i < OZ_FM; i++)
+        for (int r = 0; r < 4; r++) {
+            const int64_t row = m0 + wm * T::WM + i * 16 + 4 * fq + r, rc = min(row, g.M - 1);
+            ea[r] = P == DTCF_PREC_BF16X3 ? 0 : g.ea[rc];
+            ro[r] = wsp ? (row - m0) * T::BN : g.cview ? g.cv.rofs[rc] : rc * g.ldc;
+        }
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int64_t row = m0 + wm * OZ_WM + i * 16 + 4 * fq + r;
-                if (row >= g.M) continue;
-                const int e = P == DTCF_PREC_BF16X3 ? 0 : g.ea[row] + ebc;
-                double v = 0.0;
+        for (int jb = 0; jb < T::FN; jb += JB) {
+            __builtin_amdgcn_sched_barrier(0);
+            int eb[JB];
+            int64_t ad[JB][4];
+            double old[JB][4];
 #pragma unroll
-                for (int l = L - 2; l >= 0; l--) {  // smallest terms first
-                    if constexpr (P == DTCF_PREC_I8)
-                        v += ldexp((double)acc[l][i][j][r], e + 4 - 8 * (l + 2));
-                    else
-                        v += (double)acc[l][i][j][r];
+            for (int j = 0; j < JB; j++) {
+                const int64_t col = n0 + wn * T::WN + (jb + j) * 16 + fr, cc = min(col, g.N - 1);
+                eb[j] = P == DTCF_PREC_BF16X3 ? 0 : g.eb[cc];
+                const int64_t co = wsp ? col - n0 : g.cview ? g.cv.cofs[cc] : cc;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    ad[j][r] = ro[r] + co;
+                    if (!wsp && g.cview && g.cv.blk)
+                        ad[j][r] = vaddr(g.cv, min(m0 + wm * T::WM + i * 16 + 4 * fq + r, g.M - 1), cc);
                 }
-                if constexpr (P == DTCF_PREC_F16X3) v = ldexp(v, e);
-                if (wsp) {  // K slice: this workgroup's own tile of the workspace
-                    double *w = wsp + (row - m0) * OZ_BN + (col - n0);
-                    *w = first ? g.alpha * v : *w + g.alpha * v;
-                    continue;
-                }
-                int64_t addr;
-                if constexpr (CVIEW) addr = g.cv.blk ? vaddr(g.cv, row, col) : g.cv.rofs[row] + cof;
-                else addr = row * g.ldc + cof;
-                if (g.overwrite && first) g.C[addr] = g.alpha * v;
-                else g.C[addr] += g.alpha * v;
             }
-    }
-}
-
-// One K step of a workgroup: every product (di, dj), di + dj <= L, of the
-// A fragments in sa ([digit][16-row block][lane]) and the B fragments in sb,
-// added to the level sums.  B is taken digit by digit (the next one read
-// while this one is used); two updates of one accumulator -- (di, dj) and
-// (di - 1, dj + 1) -- are about 8 (NS - 1) MFMAs apart, and the SIMD's
-// second wave interleaves its own chains.
-template <int P, int NS, int L>
-__device__ __forceinline__ void oz_step(typename OzT<P>::Acc (&acc)[L - 1][OZ_FM][OZ_FN],
-                                        const i4 *sa, const i4 *sb, int wm, int wn, int lane)
-{
-    i4 af[NS][OZ_FM];
+            if (add) {
 #pragma unroll
-    for (int d = 0; d < NS; d++)
+                for (int j = 0; j < JB; j++)
 #pragma unroll
-        for (int i = 0; i < OZ_FM; i++)
-            af[d][i] = sa[(d * (OZ_BM / 16) + wm * (OZ_WM / 16) + i) * 64 + lane];
-    i4 bcur[OZ_FN], bnxt[OZ_FN];
+                    for (int r = 0; r < 4; r++) old[j][r] = out[ad[j][r]];
+            }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < OZ_FN; j++) bcur[j] = sb[(wn * (OZ_WN / 16) + j) * 64 + lane];
-    // Issue priority for the first B digit's MFMAs: the SIMD's two waves
-    // drift apart, so one's fragment reads and barrier wait overlap the
-    // other's MFMAs (1.8% on the int8x4/L6 ladder; priority while issuing
-    // the loads instead gained nothing).
-    __builtin_amdgcn_s_setprio(1);
+            for (int j = 0; j < JB; j++)
 #pragma unroll
-    for (int dj = 1; dj <= NS; dj++) {
-        if (dj == 2) __builtin_amdgcn_s_setprio(0);
-        if (dj < NS) {
+                for (int r = 0; r < 4; r++) {
+                    const int e = ea[r] + eb[j];
+                    double v = 0.0;
 #pragma unroll
-            for (int j = 0; j < OZ_FN; j++)
-                bnxt[j] = sb[(dj * (OZ_BN / 16) + wn * (OZ_WN / 16) + j) * 64 + lane];
+                    for (int l = L - 2; l >= 0; l--) {  // smallest terms first
+                        if constexpr (P == DTCF_PREC_I8)
+                            v += ldexp((double)acc[l][i][jb + j][r], e + 4 - 8 * (l + 2));
+                        else
+                            v += (double)acc[l][i][jb + j][r];
+                    }
+                    if constexpr (P == DTCF_PREC_F16X3) v = ldexp(v, e);
+                    if (m0 + wm * T::WM + i * 16 + 4 * fq + r < g.M && n0 + wn * T::WN + (jb + j) * 16 + fr < g.N)
+                        out[ad[j][r]] = add ? old[j][r] + g.alpha * v : g.alpha * v;
+                }
         }
-#pragma unroll
-        for (int di = 1; di <= NS; di++) {
-            if (di + dj > L) continue;
-#pragma unroll
-            for (int i = 0; i < OZ_FM; i++)
-#pragma unroll
-                for (int j = 0; j < OZ_FN; j++)
-                    acc[di + dj - 2][i][j] =
-                        OzT<P>::mfma(af[di - 1][i], bcur[j], acc[di + dj - 2][i][j]);
-        }
-#pragma unroll
-        for (int j = 0; j < OZ_FN; j++) bcur[j] = bnxt[j];
     }
 }
 
-// Tile, K steps [k0, k0 + nk) and workspace tile (null: C itself) of
-// workgroup blockIdx.x.  Whole tiles take an XCD-aware remap (consecutive
-// tiles on one XCD and its L2); every tile index then goes through groups of
-// 8 tile rows.
-__device__ __forceinline__ void oz_tile(const OzArgs &g, int64_t &m0, int64_t &n0, int64_t &k0,
-                                        int64_t &nk, double *&wsp)
+// What oz_flush reads of the kernel's arguments, loaded again from the
+// kernel argument segment (OzArgs is the only argument, at its start) behind
+// an opaque pointer: kept in scalar registers across the K loop they spilled,
+// and each step's loads then waited for reloads (7.4 instead of 4.9 ms for
+// the 9216^3 ring).
+__device__ __forceinline__ OzArgs flush_args()
 {
-    const int64_t nkall = g.Kp / OZ_BK;
-    uint32_t q;
-    if (blockIdx.x < g.t_full) {
-        q = blockIdx.x;
-        if ((g.t_full & 7u) == 0) q = (q & 7u) * (g.t_full >> 3) + (q >> 3);
-        k0 = 0;
-        nk = nkall;
-        wsp = nullptr;
-    } else {
-        const uint32_t sidx = blockIdx.x - g.t_full;
-        q = g.t_full + sidx / g.sk;
-        k0 = (int64_t)(sidx % g.sk) * g.kslice;
-        nk = min(nkall - k0, g.kslice);
-        wsp = g.ws + (int64_t)sidx * OZ_BM * OZ_BN;
-    }
-    const uint32_t width = 8 * g.tiles_n;
-    const uint32_t first = (q / width) * 8;
-    const uint32_t gsz = min(g.tiles_m - first, 8u);
-    const uint32_t tm = first + (q % width) % gsz, tn = (q % width) / gsz;
-    m0 = (int64_t)tm * OZ_BM;
-    n0 = (int64_t)tn * OZ_BN;
+    typedef const __attribute__((address_space(4))) OzArgs *Args;
+    Args a = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    OzArgs g;
+    g.ea = a->ea;
+    g.eb = a->eb;
+    g.alpha = a->alpha;
+    g.M = a->M;
+    g.N = a->N;
+    g.C = a->C;
+    g.ldc = a->ldc;
+    g.cview = a->cview;
+    g.overwrite = a->overwrite;
+    g.cv.rofs = a->cv.rofs;
+    g.cv.cofs = a->cv.cofs;
+    g.cv.blk = a->cv.blk;
+    g.cv.ncb = a->cv.ncb;
+    g.cv.div_rpb.d = a->cv.div_rpb.d;
+    g.cv.div_rpb.m = a->cv.div_rpb.m;
+    g.cv.div_rpb.l = a->cv.div_rpb.l;
+    g.cv.div_cpb.d = a->cv.div_cpb.d;
+    g.cv.div_cpb.m = a->cv.div_cpb.m;
+    g.cv.div_cpb.l = a->cv.div_cpb.l;
+    return g;
 }
 
-template <int NS, int L, bool CVIEW>
+// K steps [k0, k1) of tile q.  One step: every product (di, dj), di + dj <= L,
+// of the stage's A and B fragments, B digit by digit (the next one read while
+// this one is used); two updates of one accumulator -- (di, dj) and (di - 1,
+// dj + 1) -- are FM * FN * (NS - 1) MFMAs apart, and the SIMD's second wave
+// interleaves its own chains.  The next step's loads are issued first and
+// waited for before the last B digit's MFMAs, which then run across the
+// barrier and the next step's first reads: every fragment of the stage is
+// in registers by then (lgkmcnt 0), so the stage may be overwritten.
+// (9216^3, three digits to level 4, K loop of 128 x 192: 3.73 ms with the
+// wait after all MFMAs, 3.46 so.)  Bound by power (1.8-1.9 GHz under load)
+// and the LDS and L2 traffic of the digits.  A ring of five half steps,
+// unrolled by five, ran 128 x 128 tiles to level 6 in 7.70 ms (9216^3), this
+// loop in 7.10; three digits to level 4 in 4.61, this loop on its wide tiles
+// in 3.66-3.9.
+template <int P, int NS, int L, typename T>
+__device__ __forceinline__ void oz_run(const OzArgs &g, i4 *smem, uint32_t q, int64_t k0, int64_t k1, double *wsp)
+{
+    constexpr int FA = NS * (T::BM / 16), FB = NS * (T::BN / 16), NF = FA + FB;  // fragments per stage
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wv / (T::BN / T::WN), wn = wv % (T::BN / T::WN);
+    const uint32_t width = 8 * g.tiles_n;  // groups of 8 tile rows
+    const uint32_t first_row = (q / width) * 8;
+    const uint32_t gsz = min(g.tiles_m - first_row, 8u);
+    const int64_t m0 = (int64_t)(first_row + (q % width) % gsz) * T::BM;
+    const int64_t n0 = (int64_t)((q % width) / gsz) * T::BN;
+    const size_t pa = (size_t)g.Mp * g.Kp, pb = (size_t)g.Np * g.Kp;
+    const int64_t nk64 = g.Kp / OZ_BK;
+    // This wave's fragments of a stage, f = 8 c + wave (wave-uniform bases).
+    // Row blocks past the planes' last (planes are padded to 128 rows, tiles
+    // may be 192) repeat it: in range, and never stored.
+    constexpr int NC = (NF + OZ_WAVES - 1) / OZ_WAVES;
+    const unsigned char *src[NC];
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+        const int f = min(c * OZ_WAVES + wv, NF - 1);
+        const bool ina = f < FA;
+        const int h = ina ? f : f - FA, nb = ina ? T::BM / 16 : T::BN / 16, d = h / nb, b = h % nb;
+        const int64_t rb = min(((ina ? m0 : n0) >> 4) + b, ((ina ? g.Mp : g.Np) >> 4) - 1);
+        src[c] = (ina ? g.A + d * pa : g.B + d * pb) + rb * nk64 * 1024;
+    }
+    auto issue = [&](int64_t kt, int64_t s) __attribute__((always_inline)) {
+        i4 *stage = smem + (s & 1) * NF * 64;
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const int f = c * OZ_WAVES + wv;
+            if ((c + 1) * OZ_WAVES > NF && f >= NF) break;  // wave-uniform
+            __builtin_amdgcn_global_load_lds((const void *)(src[c] + kt * 1024 + 16 * lane),
+                                             (__attribute__((address_space(3))) void *)(stage + f * 64), 16, 0, 0);
+        }
+    };
+    auto sync = []() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(7 << 4);  // vmcnt 0, lgkmcnt 0
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    typedef typename OzT<P>::Acc Acc;
+    bool first = true;
+    // INT32 level sums stay exact for kchunk_steps steps
+    for (int64_t c0 = k0; c0 < k1; c0 += g.kchunk_steps) {
+        const int64_t c1 = g.kchunk_steps < k1 - c0 ? c0 + g.kchunk_steps : k1;
+        Acc acc[L - 1][T::FM][T::FN];
+#pragma unroll
+        for (int l = 0; l < L - 1; l++)
+#pragma unroll
+            for (int i = 0; i < T::FM; i++)
+#pragma unroll
+                for (int j = 0; j < T::FN; j++) acc[l][i][j] = (Acc){0, 0, 0, 0};
+        issue(c0, 0);
+        sync();
+        for (int64_t kt = c0; kt < c1; kt++) {
+            if (kt + 1 < c1) issue(kt + 1, kt + 1 - c0);
+            const i4 *sa = smem + ((kt - c0) & 1) * NF * 64, *sb = sa + FA * 64;
+            i4 af[NS][T::FM], bf[2][T::FN];
+#pragma unroll
+            for (int j = 0; j < T::FN; j++) bf[0][j] = sb[(wn * T::FN + j) * 64 + lane];
+#pragma unroll
+            for (int d = 0; d < NS; d++)
+#pragma unroll
+                for (int i = 0; i < T::FM; i++) af[d][i] = sa[(d * (T::BM / 16) + wm * T::FM + i) * 64 + lane];
+            // Issue priority for the first B digit's MFMAs: the SIMD's two
+            // waves drift apart, so one's fragment reads and barrier wait
+            // overlap the other's MFMAs.
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int dj = 1; dj <= NS; dj++) {
+                if (dj == 2) __builtin_amdgcn_s_setprio(0);
+                if (dj == NS) sync();
+                if (dj < NS) {
+#pragma unroll
+                    for (int j = 0; j < T::FN; j++)
+                        bf[dj & 1][j] = sb[(dj * (T::BN / 16) + wn * T::FN + j) * 64 + lane];
+                }
+#pragma unroll
+                for (int di = 1; di <= NS; di++) {
+                    if (di + dj > L) continue;
+#pragma unroll
+                    for (int i = 0; i < T::FM; i++)
+#pragma unroll
+                        for (int j = 0; j < T::FN; j++)
+                            acc[di + dj - 2][i][j] =
+                                OzT<P>::mfma(af[di - 1][i], bf[(dj - 1) & 1][j], acc[di + dj - 2][i][j]);
+                }
+            }
+        }
+        oz_flush<P, L, T>(flush_args(), acc, m0, n0, wm, wn, lane, wsp, first);
+        first = false;
+    }
+}
+
+template <int P, int NS, int L, typename T>
 __global__ __launch_bounds__(64 * OZ_WAVES, 1) void ozaki_kernel(OzArgs g)
 {
-    constexpr int FA = NS * (OZ_BM / 16), FB = NS * (OZ_BN / 16);
-    constexpr int NF = FA + FB;                          // fragments per stage
-    constexpr int PER = (NF + OZ_WAVES - 1) / OZ_WAVES;  // per wave (last may be short)
-    // Two stages as two objects: the direct loads into one stage provably do
-    // not alias the fragment reads of the other, so no wait is placed
-    // between them.
-    __shared__ i4 stage0[NF * 64];
-    __shared__ i4 stage1[NF * 64];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wv / (OZ_BN / OZ_WN), wn = wv % (OZ_BN / OZ_WN);
-
-    int64_t m0, n0, k0, nk;
-    double *wsp;
-    oz_tile(g, m0, n0, k0, nk, wsp);
-
-    const size_t pa = (size_t)g.Mp * g.Kp, pb = (size_t)g.Np * g.Kp;
-    // Fragment f = wave * PER + c comes from a wave-uniform base (scalar
-    // registers) plus one per-lane offset; it is loaded straight into LDS
-    // (16 bytes per lane, lane l at byte 16 l of the fragment).
-    // (fragment-major planes: fragment (row block, K step) is one KiB)
-    const int64_t nk64 = g.Kp / OZ_BK, lane_off = 16 * lane;
-    auto frag_base = [&](int f) __attribute__((always_inline)) -> const unsigned char * {
-        if (f < FA) {
-            const int d = f / (OZ_BM / 16), b = f % (OZ_BM / 16);
-            return g.A + d * pa + ((m0 >> 4) + b) * nk64 * 1024;
-        }
-        const int h = f - FA, d = h / (OZ_BN / 16), b = h % (OZ_BN / 16);
-        return g.B + d * pb + ((n0 >> 4) + b) * nk64 * 1024;
-    };
-    auto issue = [&](i4 *stage, int64_t kt) __attribute__((always_inline)) {
-#pragma unroll
-        for (int c = 0; c < PER; c++) {
-            const int f = wv * PER + c;
-            if (NF % OZ_WAVES != 0 && f >= NF) break;  // wave-uniform
-            __builtin_amdgcn_global_load_lds(
-                (const void *)(frag_base(f) + lane_off + kt * 1024),
-                (__attribute__((address_space(3))) void *)(stage + f * 64), 16, 0, 0);
-        }
-    };
-
-    i4 acc[L - 1][OZ_FM][OZ_FN];
-#pragma unroll
-    for (int l = 0; l < L - 1; l++)
-#pragma unroll
-        for (int i = 0; i < OZ_FM; i++)
-#pragma unroll
-            for (int j = 0; j < OZ_FN; j++) acc[l][i][j] = (i4){0, 0, 0, 0};
-
-    auto step = [&](const i4 *st) __attribute__((always_inline)) {
-        oz_step<DTCF_PREC_I8, NS, L>(acc, st, st + FA * 64, wm, wn, lane);
-    };
-    bool first = true;
-    int64_t since = 0;
-    auto after = [&](bool more) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's direct loads have landed
-        __syncthreads();                // ... and everyone's; stage reads done
-        if (++since == g.kchunk_steps && more) {
-            oz_flush<DTCF_PREC_I8, NS, L, CVIEW>(g, acc, m0, n0, wm, wn, lane, wsp, first);
-            first = false;
-#pragma unroll
-            for (int l = 0; l < L - 1; l++)
-#pragma unroll
-                for (int i = 0; i < OZ_FM; i++)
-#pragma unroll
-                    for (int j = 0; j < OZ_FN; j++) acc[l][i][j] = (i4){0, 0, 0, 0};
-            since = 0;
-        }
-    };
-
-    issue(stage0, k0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    for (int64_t kt = 0; kt < nk; kt += 2) {
-        if (kt + 1 < nk) issue(stage1, k0 + kt + 1);
-        step(stage0);
-        after(kt + 1 < nk);
-        if (kt + 1 >= nk) break;
-        if (kt + 2 < nk) issue(stage0, k0 + kt + 2);
-        step(stage1);
-        after(kt + 2 < nk);
-    }
-    oz_flush<DTCF_PREC_I8, NS, L, CVIEW>(g, acc, m0, n0, wm, wn, lane, wsp, first);
-}
-
-// The same computation with a deeper load pipeline, for NS <= 4: LDS holds
-// five half stages of NS * 8 fragments (32 KiB at NS = 4), one A or one B
-// tile of a K step each, as five objects h0..h4.  Half n of the stream
-// (A_k = half 2k, B_k = half 2k+1) sits in slot n mod 5; step k computes from
-// slots 2k, 2k+1 and issues B_{k+1} and A_{k+2} into the two slots step k-1
-// read, so A is loaded two steps ahead and B one (the two-stage kernel gives
-// both one).  The end-of-step wait leaves this wave's A_{k+2} loads in
-// flight (vmcnt = NS): direct loads complete in issue order.  The loop is
-// unrolled by five so every slot is a fixed object and the compiler sees
-// that loads into one slot never alias reads of another.
-template <int P, int NS, int L, bool CVIEW>
-__global__ __launch_bounds__(64 * OZ_WAVES, 1) void ozaki_ring_kernel(OzArgs g)
-{
-    static_assert(OZ_BM == OZ_BN, "A and B halves have the same size");
-    constexpr int FH = NS * (OZ_BM / 16);  // fragments per half stage
-    static_assert(FH % OZ_WAVES == 0 && NS <= 4, "five half stages fit LDS for NS <= 4");
-    constexpr int PH = FH / OZ_WAVES;      // direct loads per wave per half (= NS)
-    __shared__ i4 h0[FH * 64];
-    __shared__ i4 h1[FH * 64];
-    __shared__ i4 h2[FH * 64];
-    __shared__ i4 h3[FH * 64];
-    __shared__ i4 h4[FH * 64];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wv / (OZ_BN / OZ_WN), wn = wv % (OZ_BN / OZ_WN);
-    int64_t m0, n0, k0, nk;
-    double *wsp;
-    oz_tile(g, m0, n0, k0, nk, wsp);
-
-    const size_t pa = (size_t)g.Mp * g.Kp, pb = (size_t)g.Np * g.Kp;
-    const int64_t nk64 = g.Kp / OZ_BK, lane_off = 16 * lane;
-    // fragment f = wave * PH + c of a half: digit f / 8, 16-row block f % 8
-    // (fragment-major planes: fragment (row block, K step) is one KiB)
-    auto issue = [&](i4 *slot, const unsigned char *planes, size_t pstride, int64_t row0,
-                     int64_t kt) __attribute__((always_inline)) {
-#pragma unroll
-        for (int c = 0; c < PH; c++) {
-            const int f = wv * PH + c, d = f / (OZ_BM / 16), b = f % (OZ_BM / 16);
-            __builtin_amdgcn_global_load_lds(
-                (const void *)(planes + d * pstride + (((row0 >> 4) + b) * nk64 + kt) * 1024 + lane_off),
-                (__attribute__((address_space(3))) void *)(slot + f * 64), 16, 0, 0);
-        }
-    };
-
-    typedef typename OzT<P>::Acc Acc;
-    Acc acc[L - 1][OZ_FM][OZ_FN];
-#pragma unroll
-    for (int l = 0; l < L - 1; l++)
-#pragma unroll
-        for (int i = 0; i < OZ_FM; i++)
-#pragma unroll
-            for (int j = 0; j < OZ_FN; j++) acc[l][i][j] = (Acc){0, 0, 0, 0};
-
-    // s_waitcnt with vmcnt = PH and no expcnt / lgkmcnt wait (GFX9 encoding:
-    // vmcnt[3:0], expcnt[6:4], lgkmcnt[11:8], vmcnt[15:14])
-    constexpr int WAIT_PH = (PH & 15) | (7 << 4) | (15 << 8) | ((PH >> 4) << 14);
-    bool first = true;
-    int64_t since = 0;
-    // Workgroup barrier without __syncthreads' release fence, which would
-    // wait for every outstanding load (vmcnt 0) and so for A_{k+2} too.  The
-    // waits are explicit instead: before the barrier each wave has its own
-    // loads for the next step landed (s_waitcnt) and has consumed its reads
-    // of this step's slots (the MFMAs used them); the "memory" clobber keeps
-    // the compiler from moving LDS or load instructions across it.
-    auto barrier = []() __attribute__((always_inline)) { asm volatile("s_barrier" ::: "memory"); };
-    auto after = [&](int64_t k) __attribute__((always_inline)) {
-        if (k + 2 < nk) __builtin_amdgcn_s_waitcnt(WAIT_PH);  // A_{k+2} may stay in flight
-        else __builtin_amdgcn_s_waitcnt(0);
-        barrier();
-        if (++since == g.kchunk_steps && k + 1 < nk) {
-            oz_flush<P, NS, L, CVIEW>(g, acc, m0, n0, wm, wn, lane, wsp, first);
-            first = false;
-#pragma unroll
-            for (int l = 0; l < L - 1; l++)
-#pragma unroll
-                for (int i = 0; i < OZ_FM; i++)
-#pragma unroll
-                    for (int j = 0; j < OZ_FN; j++) acc[l][i][j] = (Acc){0, 0, 0, 0};
-            since = 0;
-        }
-    };
-
-    issue(h0, g.A, pa, m0, k0);
-    issue(h1, g.B, pb, n0, k0);
-    if (nk > 1) {
-        issue(h2, g.A, pa, m0, k0 + 1);
-        __builtin_amdgcn_s_waitcnt(WAIT_PH);
+    extern __shared__ i4 oz_smem[];  // two stages
+    const int64_t nk = g.Kp / OZ_BK;
+    uint32_t q, slot = 0;
+    int64_t k0 = 0, left = nk;
+    if (blockIdx.x < g.t_full) {
+        // XCD-aware remap: consecutive tiles on one XCD and its L2
+        q = blockIdx.x;
+        if ((g.t_full & 7u) == 0) q = (q & 7u) * (g.t_full >> 3) + (q >> 3);
     } else {
-        __builtin_amdgcn_s_waitcnt(0);
+        const uint32_t w = run_index(blockIdx.x - g.t_full, g.sw);
+        const int64_t s = run_begin(w, g.sw, g.steps), t = div_small(s, nk);
+        left = run_begin(w + 1, g.sw, g.steps) - s;
+        q = g.t_full + (uint32_t)t;
+        k0 = s - t * nk;
+        slot = 2 * w;
     }
-    barrier();
-#define OZ_RING_STEP(SA, SB, NB, NA, J)                   \
-    {                                                     \
-        const int64_t k = kt + (J);                       \
-        if (k >= nk) break;                               \
-        if (k + 1 < nk) issue(NB, g.B, pb, n0, k0 + k + 1); \
-        if (k + 2 < nk) issue(NA, g.A, pa, m0, k0 + k + 2); \
-        oz_step<P, NS, L>(acc, SA, SB, wm, wn, lane);     \
-        after(k);                                         \
+    for (; left > 0; q++) {
+        const int64_t k1 = min(nk, k0 + left);
+        oz_run<P, NS, L, T>(g, oz_smem, q, k0, k1,
+                            k0 > 0 || k1 < nk ? g.ws + (int64_t)slot * T::BM * T::BN : nullptr);
+        left -= k1 - k0;
+        k0 = 0;
+        slot |= 1;
     }
-    for (int64_t kt = 0; kt < nk; kt += 5) {
-        OZ_RING_STEP(h0, h1, h3, h4, 0)
-        OZ_RING_STEP(h2, h3, h0, h1, 1)
-        OZ_RING_STEP(h4, h0, h2, h3, 2)
-        OZ_RING_STEP(h1, h2, h4, h0, 3)
-        OZ_RING_STEP(h3, h4, h1, h2, 4)
-    }
-#undef OZ_RING_STEP
-    oz_flush<P, NS, L, CVIEW>(g, acc, m0, n0, wm, wn, lane, wsp, first);
 }
 
-// Adds the K slices of every tile (workspace slot tile * sk + slice, alpha
-// already applied) to C in slice order: deterministic.
-template <bool CVIEW>
+// Adds the pieces of every split tile (alpha already applied) to C in K
+// order: deterministic.
+template <typename T>
 __global__ __launch_bounds__(256) void oz_split_reduce(OzArgs g)
 {
-    const uint32_t ti = blockIdx.y, q = g.t_full + ti;  // split tile, in oz_tile's order
+    const uint32_t ti = blockIdx.y, q = g.t_full + ti;  // split tile, in oz_run's order
     const uint32_t width = 8 * g.tiles_n;
     const uint32_t first = (q / width) * 8;
     const uint32_t gsz = min(g.tiles_m - first, 8u);
-    const uint32_t tm = first + (q % width) % gsz, tn = (q % width) / gsz;
-    const int64_t m0 = (int64_t)tm * OZ_BM, n0 = (int64_t)tn * OZ_BN;
-    for (int e = blockIdx.x * 256 + threadIdx.x; e < OZ_BM * OZ_BN; e += gridDim.x * 256) {
-        const int64_t row = m0 + e / OZ_BN, col = n0 + e % OZ_BN;
-        if (row >= g.M || col >= g.N) continue;
-        const double sum = sum_in_order(g.ws + (int64_t)ti * g.sk * OZ_BM * OZ_BN + e, g.sk, OZ_BM * OZ_BN);
-        int64_t addr;
-        if constexpr (CVIEW)
-            addr = g.cv.blk ? vaddr(g.cv, row, col) : g.cv.rofs[row] + g.cv.cofs[col];
-        else addr = row * g.ldc + col;
-        if (g.overwrite) g.C[addr] = sum;
-        else g.C[addr] += sum;
-    }
+    const int64_t nk = g.Kp / OZ_BK;
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    const int64_t row = (int64_t)(first + (q % width) % gsz) * T::BM + e / T::BN;
+    const int64_t col = (int64_t)((q % width) / gsz) * T::BN + e % T::BN;
+    if (row >= g.M || col >= g.N) return;
+    bool whole;
+    const double sum = sum_pieces(g.ws, ti * nk, nk, g.sw, g.steps, T::BM * T::BN, e, whole);
+    if (whole) return;
+    const int64_t addr = g.cview ? vaddr(g.cv, row, col) : row * g.ldc + col;
+    if (g.overwrite) g.C[addr] = sum;
+    else g.C[addr] += sum;
 }
 
 int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
@@ -1239,49 +1166,101 @@ int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 // specialisation exists; 0: one launch per product.
 int g_fused_i8 = 1;
 
-template <int P, int NS, int L>
-int oz_launch(const OzArgs &g, bool cview, hipStream_t s)
+// One workgroup per CU.  rate: TOP/s of the tile's K loop on a large
+// product.  Every round of tiles also pays its epilogue, which nothing
+// overlaps (C read and written at about 5 TB/s).  Tiles are only cut evenly:
+// runs at 256 different K positions share no panels in L2, and at 9 TB/s of
+// digits the K loop then waits for HBM (2304 x 2304 x 9216, 216 tiles of 192 x
+// 128: 315 us in 256 equal runs, 253 uncut).
+template <typename T>
+SplitPlan oz_plan(const OzArgs &g, int products, int ns, double rate, int cus)
 {
-    const uint32_t T = g.tiles_m * g.tiles_n;
-    const unsigned grid = g.t_full + (T - g.t_full) * g.sk;
-    if constexpr (NS <= 4) {
-        if (cview) hipLaunchKernelGGL((ozaki_ring_kernel<P, NS, L, true>), dim3(grid), dim3(64 * OZ_WAVES), 0, s, g);
-        else hipLaunchKernelGGL((ozaki_ring_kernel<P, NS, L, false>), dim3(grid), dim3(64 * OZ_WAVES), 0, s, g);
-    } else {
-        static_assert(NS > 4 && P == DTCF_PREC_I8, "two full stages: INT8 with five digits only");
-        if (cview) hipLaunchKernelGGL((ozaki_kernel<NS, L, true>), dim3(grid), dim3(64 * OZ_WAVES), 0, s, g);
-        else hipLaunchKernelGGL((ozaki_kernel<NS, L, false>), dim3(grid), dim3(64 * OZ_WAVES), 0, s, g);
+    const int64_t tm = (g.M + T::BM - 1) / T::BM, tn = (g.N + T::BN - 1) / T::BN;
+    SplitPlan none;
+    none.us = 1e300;
+    if ((double)tm * tn >= 2147483648.0) return none;
+    const double step = 2.0 * T::BM * T::BN * OZ_BK * products / (rate * 1e6 / cus);
+    const TileRate t = {T::BM, T::BN, 1, step, {1.0, 1.0, 1.0, 1.0}, true};
+    // panel rows of 128 bytes, as an FP64 K step reads
+    SplitPlan p = gemm_split_plan((uint32_t)(tm * tn), g.Kp / OZ_BK, (tm * T::BM + tn * T::BN) * ns / 2, cus, t);
+    p.us += (double)((tm * tn + cus - 1) / cus) * T::BM * T::BN * 16.0 * cus / 5.0e6;
+    return p;
+}
+
+template <int P, int NS, int L, typename T>
+int oz_launch(OzArgs g, const SplitPlan &sp, hipStream_t s)
+{
+    auto kern = ozaki_kernel<P, NS, L, T>;
+    constexpr size_t lds = (size_t)2 * NS * (T::BM + T::BN) * OZ_BK;
+    static std::once_flag once;
+    static hipError_t attr_err = hipSuccess;
+    std::call_once(once, [&] {
+        attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    });
+    DTCF_HIP(attr_err);
+    g.tiles_m = (uint32_t)((g.M + T::BM - 1) / T::BM);
+    g.tiles_n = (uint32_t)((g.N + T::BN - 1) / T::BN);
+    const uint32_t tiles = g.tiles_m * g.tiles_n;
+    g.t_full = tiles - sp.nsplit;
+    g.sw = sp.sw;
+    g.steps = (int64_t)sp.nsplit * (g.Kp / OZ_BK);
+    g.ws = nullptr;
+    if (sp.nsplit) {
+        const int st = gemm_workspace(s, (size_t)2 * sp.sw * T::BM * T::BN * sizeof(double), &g.ws);
+        if (st != DTCF_OK) return st;
     }
+    hipLaunchKernelGGL(kern, dim3(g.t_full + g.sw), dim3(64 * OZ_WAVES), lds, s, g);
     DTCF_HIP(hipGetLastError());
-    if (g.t_full < T) {
-        const dim3 rg(OZ_BM * OZ_BN / 256, T - g.t_full);
-        if (cview) hipLaunchKernelGGL(oz_split_reduce<true>, rg, dim3(256), 0, s, g);
-        else hipLaunchKernelGGL(oz_split_reduce<false>, rg, dim3(256), 0, s, g);
+    if (sp.nsplit) {
+        hipLaunchKernelGGL(oz_split_reduce<T>, dim3(T::BM * T::BN / 256, sp.nsplit), dim3(256), 0, s, g);
         DTCF_HIP(hipGetLastError());
     }
     return DTCF_OK;
 }
 
+// The tile with the shortest predicted time: 192 x 128 or 128 x 192 where
+// the registers and LDS allow (`wide` TOP/s) unless the padding and the last
+// round cost it more than 128 x 128 (`square`).
+template <int P, int NS, int L>
+int oz_pick(const OzArgs &g, double square, double wide, hipStream_t s)
+{
+    int cus = 0;
+    const int st = gemm_device_cus(&cus);
+    if (st != DTCF_OK) return st;
+    int products = 0;
+    for (int i = 1; i <= NS; i++)
+        for (int j = 1; j <= NS; j++) products += i + j <= L;
+    const SplitPlan sq = oz_plan<OzTile<128, 128>>(g, products, NS, square, cus);
+    if constexpr (L == 4) {
+        const SplitPlan hi = oz_plan<OzTile<192, 128>>(g, products, NS, 0.97 * wide, cus);
+        const SplitPlan lo = oz_plan<OzTile<128, 192>>(g, products, NS, wide, cus);
+        if (hi.us <= lo.us && hi.us < sq.us) return oz_launch<P, NS, L, OzTile<192, 128>>(g, hi, s);
+        if (lo.us < sq.us) return oz_launch<P, NS, L, OzTile<128, 192>>(g, lo, s);
+    }
+    return oz_launch<P, NS, L, OzTile<128, 128>>(g, sq, s);
+}
+
 // Runs the fused kernel when (prec, ns, lev) has a specialisation; *done =
-// false otherwise.
-int oz_dispatch(int prec, int ns, int lev, const OzArgs &g, bool cview, hipStream_t s, bool *done)
+// false otherwise.  Rates: 9216^3 less the epilogue (three INT8 digits to
+// level 4: 4.23 ms on 128 x 128, 3.66 on 128 x 192, 3.76 on 192 x 128; four to
+// level 4: 4.68 / 4.04 / 4.15; BF16: 8.11 / 7.01 / 7.10).
+int oz_dispatch(int prec, int ns, int lev, const OzArgs &g, hipStream_t s, bool *done)
 {
     *done = true;
-    if (prec == DTCF_PREC_BF16X3 && ns == 3 && lev == 4)
-        return oz_launch<DTCF_PREC_BF16X3, 3, 4>(g, cview, s);
-    if (prec == DTCF_PREC_F16X3 && ns == 3 && lev == 4)
-        return oz_launch<DTCF_PREC_F16X3, 3, 4>(g, cview, s);
+    if (prec == DTCF_PREC_BF16X3 && ns == 3 && lev == 4) return oz_pick<DTCF_PREC_BF16X3, 3, 4>(g, 1200, 1390, s);
+    if (prec == DTCF_PREC_F16X3 && ns == 3 && lev == 4) return oz_pick<DTCF_PREC_F16X3, 3, 4>(g, 1200, 1390, s);
     if (prec != DTCF_PREC_I8) {
         *done = false;
         return DTCF_OK;
     }
     switch (ns * 16 + lev) {
-    case 3 * 16 + 4: return oz_launch<DTCF_PREC_I8, 3, 4>(g, cview, s);
-    case 4 * 16 + 4: return oz_launch<DTCF_PREC_I8, 4, 4>(g, cview, s);
-    case 4 * 16 + 5: return oz_launch<DTCF_PREC_I8, 4, 5>(g, cview, s);
-    case 4 * 16 + 6: return oz_launch<DTCF_PREC_I8, 4, 6>(g, cview, s);
-    case 5 * 16 + 5: return oz_launch<DTCF_PREC_I8, 5, 5>(g, cview, s);
-    case 5 * 16 + 6: return oz_launch<DTCF_PREC_I8, 5, 6>(g, cview, s);
+    case 3 * 16 + 4: return oz_pick<DTCF_PREC_I8, 3, 4>(g, 2370, 2770, s);
+    case 4 * 16 + 4: return oz_pick<DTCF_PREC_I8, 4, 4>(g, 2130, 2490, s);
+    case 4 * 16 + 5: return oz_pick<DTCF_PREC_I8, 4, 5>(g, 2800, 0, s);
+    case 4 * 16 + 6: return oz_pick<DTCF_PREC_I8, 4, 6>(g, 2970, 0, s);
+    case 5 * 16 + 5: return oz_pick<DTCF_PREC_I8, 5, 5>(g, 2580, 0, s);
+    case 5 * 16 + 6: return oz_pick<DTCF_PREC_I8, 5, 6>(g, 2860, 0, s);
     default: *done = false; return DTCF_OK;
     }
 }
@@ -1569,8 +1548,7 @@ int gemm_split_f64_impl(int prec, int nslice, int64_t m, int64_t n, int64_t k, d
         o.C = C;
         o.cv = g.cv;
         o.ldc = ldc;
-        o.tiles_m = (uint32_t)(g.Mp / OZ_BM);
-        o.tiles_n = (uint32_t)(g.Np / OZ_BN);
+        o.cview = cv != nullptr;
         o.overwrite = overwrite;
         // Level l = i + j sums the products q_i q_j, |q_1| <= 65, |q_i| <= 128
         // otherwise; INT32 stays exact while K times the largest level's
@@ -1585,47 +1563,12 @@ int gemm_split_f64_impl(int prec, int nslice, int64_t m, int64_t n, int64_t k, d
             worst = std::max(worst, s);
         }
         const int64_t kmax = ((int64_t(1) << 31) - 1) / worst;
-        o.kchunk_steps = prec == DTCF_PREC_I8 ? std::max<int64_t>(1, kmax / OZ_BK) : INT64_MAX;
-        // K split (one workgroup per CU): when the tiles fill under half the
-        // CUs, every tile is cut into sk slices of >= 16 K steps with sk *
-        // tiles <= CUs; when the last round of whole tiles fills at most half
-        // the CUs, its tiles alone are cut so that they fill one round (the
-        // 324 tiles of a 2304^2 result: 68 tail tiles x 3 slices after 256
-        // whole ones, instead of a second round 27% full).  nsplit * sk <=
-        // CUs, so the slices (alpha * partial C tiles) fit the stream's GEMM
-        // split workspace.
-        const uint32_t tiles = o.tiles_m * o.tiles_n;
-        const int64_t nkall = o.Kp / OZ_BK;
-        o.t_full = tiles;
-        o.sk = 1;
-        o.kslice = nkall;
-        o.ws = nullptr;
-        int cus = 0;
-        int sst = gemm_device_cus(&cus);
-        if (sst != DTCF_OK) return sst;
-        const uint32_t rem = tiles % (uint32_t)cus;
-        uint32_t nsplit = 0;
-        int64_t sk = 0;
-        if (tiles < (uint32_t)cus / 2 && nkall >= 32) {
-            nsplit = tiles;
-            sk = std::min<int64_t>(cus / tiles, nkall / 16);
-        } else if (tiles > (uint32_t)cus && rem > 0 && rem <= (uint32_t)cus / 2 && nkall >= 32) {
-            nsplit = rem;
-            sk = std::min<int64_t>(cus / rem, nkall / 16);
-        }
-        if (sk >= 2) {
-            const int64_t ks = (nkall + sk - 1) / sk;
-            sk = (nkall + ks - 1) / ks;
-            double *ws = nullptr;
-            sst = gemm_workspace(s, (size_t)nsplit * sk * OZ_BM * OZ_BN * sizeof(double), &ws);
-            if (sst != DTCF_OK) return sst;
-            o.t_full = tiles - nsplit;
-            o.sk = (uint32_t)sk;
-            o.kslice = ks;
-            o.ws = ws;
-        }
+        // (never past the tile's steps, so the kernel's step index cannot overflow)
+        o.kchunk_steps = o.Kp / OZ_BK;
+        if (prec == DTCF_PREC_I8)
+            o.kchunk_steps = std::min<int64_t>(o.kchunk_steps, std::max<int64_t>(1, kmax / OZ_BK));
         bool done = false;
-        int st = oz_dispatch(prec, ns, lev, o, cv != nullptr, s, &done);
+        int st = oz_dispatch(prec, ns, lev, o, s, &done);
         if (st != DTCF_OK || done) return st;
     }
     if (prec == DTCF_PREC_I8)

@@ -1,0 +1,52 @@
+"""Fused slice products at the sizes where their C tile and split change:
+square and wide tiles with ragged edges (planes are padded to 128 rows, the
+wide tiles are 192), whole rounds of tiles and tiles cut over K, C dense,
+through a view, accumulated twice.  INT8 digits against the one-GEMM-per-
+product path (the same exact integers, recombined in FP64 in another order:
+1e-13 of the largest result, as test_gpu_mixed); BF16 and FP16 against FP64
+(5e-6, the bound stated for their FP32 sums)."""
+import numpy as np
+import pytest
+import torch
+
+from dtcf_amd import mixed, ops
+
+pytestmark = pytest.mark.gpu
+
+SIZES = ((2304, 2304, 1000), (3000, 2400, 700), (2400, 3000, 300), (193, 5000, 260), (5000, 193, 260),
+         (130, 190, 6000), (1537, 129, 2100), (64, 64, 64))
+MODES = ((mixed.I8, 3, 4), (mixed.I8, 4, 4), (mixed.I8, 4, 6), (mixed.I8, 5, 6), (mixed.BF16X3, 3, 4),
+         (mixed.F16X3, 3, 4))
+
+
+@pytest.mark.parametrize("prec,ns,lev", MODES)
+@pytest.mark.parametrize("m,n,k", SIZES)
+def test_fused_tiles(dev, prec, ns, lev, m, n, k):
+    A, B = mixed.fill_normal(m * k, 1, 1.0), mixed.fill_normal(n * k, 2, 1.0)
+    sa = mixed.Split(prec, A, mixed.dense_view(m, k), ns)
+    sb = mixed.Split(prec, B, mixed.dense_view(n, k), ns)
+    C0 = mixed.fill_normal(m * n, 3, 1.0)
+    print("slices", prec, ns, lev, m, n, k, flush=True)
+    got = C0.clone()
+    for _ in range(2):
+        mixed.gemm_split(sa, sb, got, alpha=0.5, ldc=n, max_level=lev)
+    if prec == mixed.I8:
+        mixed.set_fused(False)
+        try:
+            ref = C0.clone()
+            for _ in range(2):
+                mixed.gemm_split(sa, sb, ref, alpha=0.5, ldc=n, max_level=lev)
+        finally:
+            mixed.set_fused(True)
+        tol = 1e-13
+    else:
+        ref = C0 + (A.view(m, k) @ B.view(n, k).t().contiguous()).reshape(-1)
+        tol = 5e-6
+    scale = ref.abs().max()
+    assert ((got - ref).abs().max() / scale).item() <= tol
+    # C through a view of its transpose: the same values, element for element
+    view = ops.View(m, n, np.arange(m), np.arange(n) * m)
+    gv = C0.view(m, n).t().contiguous().reshape(-1)
+    for _ in range(2):
+        mixed.gemm_split(sa, sb, gv, alpha=0.5, cview=view, max_level=lev)
+    assert torch.equal(gv.view(n, m).t().contiguous().reshape(-1), got)

@@ -8,10 +8,11 @@
 //   q = the dim with the smallest output stride (output-fastest),
 //   p = the dim with unit input stride (input-fastest) when it differs from q.
 // TRANSPOSE tiles (p != q) go through LDS so that reads run along p and
-// writes run along q, both coalesced; DIRECT tiles (q is fastest on both
-// sides) copy straight through with lanes along q.  All other dims and the
-// tile batch index are decoded once per workgroup.
+// writes run along q, both coalesced; straight tiles (q is fastest on both
+// sides) copy through registers with lanes along q.  All other dims and the
+// tile batch index are decoded once per plane.
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -38,96 +39,154 @@ struct PermParams {
     double alpha, beta;
 };
 
+// 8-byte form, for any extents, offsets and alignment.  A plane is the p x q
+// extents at one index of every other dim and batch entry; a work item is
+// one Pt x Qt tile of up to `np` consecutive planes, and its threads take its
+// elements flat, p fastest to read and q fastest to write (TRANSPOSE, through
+// LDS) or q fastest for both.  So short extents fill the waves (tiles of a
+// fixed 32 x 32 left 13 of 32 lanes working on a 13 x 47 plane), a plane that
+// is contiguous in the output is written in one run, and eight loads per
+// thread are in flight.  HBM-bound: 256 tiles of 11 x 13 x 45 x 47, order
+// 2,0,3,1: 438 -> 257 us; 12 ns of start-up per workgroup are spread over
+// up to 4096 elements.
+constexpr int kPlaneElems = 4096;
+constexpr int kMaxPlanes = 64;
+struct PlaneParams {
+    uint32_t Pt, Qt, np;
+    FastDiv div_pt, div_qt, div_pq;  // by Pt, Qt, Pt * Qt
+    uint64_t planes, items;
+    uint32_t others;                 // planes per batch entry
+};
+
 template <bool TRANSPOSE>
 __global__ __launch_bounds__(256) void permute_kernel(const double *__restrict__ in,
-                                                      double *__restrict__ out, PermParams P,
+                                                      double *__restrict__ out, PermParams P, PlaneParams L,
                                                       const int64_t *__restrict__ src_off,
                                                       const int64_t *__restrict__ dst_off)
 {
-    constexpr int TP = TRANSPOSE ? 32 : 16;   // tile rows along p
-    constexpr int TQ = TRANSPOSE ? 32 : 64;   // tile cols along q
-    __shared__ double lds[TRANSPOSE ? 32 : 1][TRANSPOSE ? 33 : 1];
-    const int tid = threadIdx.x;
-
-    for (uint64_t blk = blockIdx.x; blk < P.total; blk += gridDim.x) {
-        const uint64_t t = blk / P.per_tile;
-        uint32_t rem = (uint32_t)(blk - t * P.per_tile);
-        const uint32_t qt_div = P.div_ntq.div(rem);
-        const uint32_t qt = rem - qt_div * P.ntq;
-        rem = qt_div;
-        const uint32_t pt_div = P.div_ntp.div(rem);
-        const uint32_t pt = rem - pt_div * P.ntp;
-        rem = pt_div;
-        int64_t src = src_off ? src_off[t] : (int64_t)t * P.src_step;
-        int64_t dst = dst_off ? dst_off[t] : (int64_t)t * P.dst_step;
-        for (int d = P.n_other - 1; d >= 0; d--) {
-            const uint32_t q = P.other_div[d].div(rem);
-            const uint32_t x = rem - q * P.other_ext[d];
-            rem = q;
-            src += (int64_t)x * P.other_istr[d];
-            dst += (int64_t)x * P.other_ostr[d];
+    __shared__ double lds[TRANSPOSE ? kPlaneElems : 1];
+    __shared__ int64_t soff[kMaxPlanes], doff[kMaxPlanes];
+    const uint32_t tid = threadIdx.x, PS = L.Pt | 1, PQ = L.Pt * L.Qt;  // odd LDS pitch
+    for (uint64_t it = blockIdx.x; it < L.items; it += gridDim.x) {
+        const uint64_t pg = it / ((uint64_t)P.ntp * P.ntq);
+        const uint32_t rem = (uint32_t)(it - pg * P.ntp * P.ntq);
+        const uint32_t pt = P.div_ntq.div(rem), qt = rem - pt * P.ntq;
+        const uint64_t plane0 = pg * L.np;
+        const uint32_t np = (uint32_t)min((uint64_t)L.np, L.planes - plane0);
+        if (tid < np) {
+            const uint64_t t = (plane0 + tid) / L.others;
+            uint32_t x = (uint32_t)(plane0 + tid - t * L.others);
+            int64_t src = src_off ? src_off[t] : (int64_t)t * P.src_step;
+            int64_t dst = dst_off ? dst_off[t] : (int64_t)t * P.dst_step;
+            for (int d = P.n_other - 1; d >= 0; d--) {
+                const uint32_t q = P.other_div[d].div(x), r = x - q * P.other_ext[d];
+                x = q;
+                src += (int64_t)r * P.other_istr[d];
+                dst += (int64_t)r * P.other_ostr[d];
+            }
+            const int64_t p0 = (int64_t)pt * L.Pt, q0 = (int64_t)qt * L.Qt;
+            soff[tid] = src + p0 * P.istr_p + q0 * P.istr_q;
+            doff[tid] = dst + p0 * P.ostr_p + q0 * P.ostr_q;
         }
-        const int64_t p0 = (int64_t)pt * TP;
-        const int64_t q0 = (int64_t)qt * TQ;
-
+        __syncthreads();
+        const uint32_t pn = (uint32_t)min((int64_t)L.Pt, P.ext_p - (int64_t)pt * L.Pt);
+        const uint32_t qn = (uint32_t)min((int64_t)L.Qt, P.ext_q - (int64_t)qt * L.Qt);
+        const uint32_t total = np * PQ;
+        // element e of the item: plane, and (slow, fast) of its tile
+        auto split = [&](uint32_t e, const FastDiv &fast, uint32_t &pl, uint32_t &hi, uint32_t &lo) {
+            pl = L.div_pq.div(e);
+            const uint32_t r = e - pl * PQ;
+            hi = fast.div(r);
+            lo = r - hi * fast.d;
+        };
+        // Elements outside are clamped to one of the item and not stored: loads
+        // under a branch wait one by one (368 us where this form takes 257)
+        auto locate = [&](uint32_t e, bool p_fast, uint32_t &pl, uint32_t &pp, uint32_t &qq) {
+            const uint32_t c = min(e, total - 1);
+            if (p_fast) split(c, L.div_pt, pl, qq, pp);
+            else split(c, L.div_qt, pl, pp, qq);
+            const bool ok = e < total && pp < pn && qq < qn;
+            pp = min(pp, pn - 1);
+            qq = min(qq, qn - 1);
+            return ok;
+        };
+        auto put = [&](auto count, const double *v, double *const *to, uint32_t ok) {
+            constexpr int U = decltype(count)::value;
+            if (P.beta == 0.0) {
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (ok >> u & 1) *to[u] = (P.alpha == 1.0) ? v[u] : P.alpha * v[u];
+            } else {
+                double w[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) w[u] = *to[u];
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (ok >> u & 1) *to[u] = P.alpha * v[u] + P.beta * w[u];
+            }
+        };
+        // in -> LDS (TRANSPOSE) or out, `U` elements of this thread from e0 on
+        auto fetch = [&](auto count, uint32_t e0) {
+            constexpr int U = decltype(count)::value;
+            double v[U];
+            double *to[U];
+            uint32_t at[U], ok = 0;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                uint32_t pl, pp, qq;
+                if (locate(e0 + 256 * u + tid, TRANSPOSE, pl, pp, qq)) ok |= 1u << u;
+                if constexpr (TRANSPOSE) at[u] = (pl * L.Qt + qq) * PS + pp;
+                else to[u] = out + doff[pl] + (int64_t)qq * P.ostr_q + (int64_t)pp * P.ostr_p;
+                v[u] = in[soff[pl] + (int64_t)pp * P.istr_p + (int64_t)qq * P.istr_q];
+            }
+            if constexpr (TRANSPOSE) {
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (ok >> u & 1) lds[at[u]] = v[u];
+            } else {
+                put(count, v, to, ok);
+            }
+        };
+        auto store = [&](auto count, uint32_t e0) {  // LDS -> out
+            constexpr int U = decltype(count)::value;
+            double v[U];
+            double *to[U];
+            uint32_t ok = 0;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                uint32_t pl, pp, qq;
+                if (locate(e0 + 256 * u + tid, false, pl, pp, qq)) ok |= 1u << u;
+                to[u] = out + doff[pl] + (int64_t)qq * P.ostr_q + (int64_t)pp * P.ostr_p;
+                v[u] = lds[(pl * L.Qt + qq) * PS + pp];
+            }
+            put(count, v, to, ok);
+        };
+        // eight per thread, fewer for the rest: the clamped ones cost as much
+        auto sweep = [&](auto &&step) {
+            uint32_t e0 = 0;
+            for (; e0 + 1024 < total; e0 += 2048) step(std::integral_constant<int, 8>(), e0);
+            if (e0 + 512 < total) step(std::integral_constant<int, 4>(), e0);
+            else if (e0 < total) step(std::integral_constant<int, 2>(), e0);
+        };
+        sweep(fetch);
+        __syncthreads();
         if constexpr (TRANSPOSE) {
-            const int tx = tid & 31, ty = tid >> 5;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t pp = p0 + tx, qq = q0 + ty + 8 * i;
-                if (pp < P.ext_p && qq < P.ext_q)
-                    lds[ty + 8 * i][tx] = in[src + pp * P.istr_p + qq * P.istr_q];
-            }
+            sweep(store);
             __syncthreads();
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t qq = q0 + tx, pp = p0 + ty + 8 * i;
-                if (pp < P.ext_p && qq < P.ext_q) {
-                    double *o = out + dst + qq * P.ostr_q + pp * P.ostr_p;
-                    const double v = lds[tx][ty + 8 * i];
-                    if (P.beta == 0.0)
-                        *o = (P.alpha == 1.0) ? v : P.alpha * v;
-                    else
-                        *o = P.alpha * v + P.beta * (*o);
-                }
-            }
-            __syncthreads();
-        } else {
-            const int tx = tid & 63, ty = tid >> 6;
-            double v[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t qq = q0 + tx, pp = p0 + ty + 4 * i;
-                if (pp < P.ext_p && qq < P.ext_q) v[i] = in[src + qq * P.istr_q + pp * P.istr_p];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t qq = q0 + tx, pp = p0 + ty + 4 * i;
-                if (pp < P.ext_p && qq < P.ext_q) {
-                    double *o = out + dst + qq * P.ostr_q + pp * P.ostr_p;
-                    if (P.beta == 0.0)
-                        *o = (P.alpha == 1.0) ? v[i] : P.alpha * v[i];
-                    else
-                        *o = P.alpha * v[i] + P.beta * (*o);
-                }
-            }
         }
     }
 }
 
-// 16-byte forms of the two tiles, taken when the tile's fast strides are 1
-// on their side, the extents and every other offset even and the buffers
-// 16-byte aligned (no per-tile offset tables): TRANSPOSE 64 x 64 through
-// LDS, 16 elements per thread, reads two consecutive p and writes two
-// consecutive q per access; DIRECT 16 x 128, 8 elements per thread, q
-// contiguous on both sides.  Same values as permute_kernel.
-template <bool TRANSPOSE>
+// 16-byte form of the TRANSPOSE tile, taken when the fast strides are 1 on
+// their side, the extents and every other offset even, the buffers 16-byte
+// aligned (no per-tile offset tables) and the tile filled to a fifth:
+// 64 x 64 through LDS, 16 elements per thread, reads two consecutive p and
+// writes two consecutive q per access.  Same values as permute_kernel.
 __global__ __launch_bounds__(256) void permute_vec_kernel(const double *__restrict__ in,
                                                           double *__restrict__ out, PermParams P)
 {
-    constexpr int TP = TRANSPOSE ? 64 : 16;
-    constexpr int TQ = TRANSPOSE ? 64 : 128;
-    __shared__ double lds[TRANSPOSE ? 64 : 1][TRANSPOSE ? 65 : 1];
+    constexpr int TP = 64, TQ = 64;
+    __shared__ double lds[64][65];
     const int tid = threadIdx.x;
     for (uint64_t blk = blockIdx.x; blk < P.total; blk += gridDim.x) {
         const uint64_t t = blk / P.per_tile;
@@ -160,46 +219,29 @@ __global__ __launch_bounds__(256) void permute_vec_kernel(const double *__restri
             }
             *reinterpret_cast<double2 *>(o) = v;
         };
-        if constexpr (TRANSPOSE) {
-            const int tx = tid & 31, ty = tid >> 5;
-            double2 v[8];
+        const int tx = tid & 31, ty = tid >> 5;
+        double2 v[8];
 #pragma unroll
-            for (int i = 0; i < 8; i++) {  // rows q, pairs of p (unit input stride)
-                const int64_t pp = p0 + 2 * tx, qq = q0 + ty + 8 * i;
-                v[i] = (pp < P.ext_p && qq < P.ext_q)
-                           ? *reinterpret_cast<const double2 *>(in + src + pp + qq * P.istr_q)
-                           : make_double2(0.0, 0.0);
-            }
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                lds[ty + 8 * i][2 * tx] = v[i].x;
-                lds[ty + 8 * i][2 * tx + 1] = v[i].y;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < 8; i++) {  // rows p, pairs of q (unit output stride)
-                const int64_t qq = q0 + 2 * tx, pp = p0 + ty + 8 * i;
-                if (pp < P.ext_p && qq < P.ext_q)
-                    put(out + dst + qq + pp * P.ostr_p,
-                        make_double2(lds[2 * tx][ty + 8 * i], lds[2 * tx + 1][ty + 8 * i]));
-            }
-            __syncthreads();
-        } else {
-            const int tx = tid & 63, ty = tid >> 6;
-            double2 v[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t qq = q0 + 2 * tx, pp = p0 + ty + 4 * i;
-                v[i] = (pp < P.ext_p && qq < P.ext_q)
-                           ? *reinterpret_cast<const double2 *>(in + src + qq + pp * P.istr_p)
-                           : make_double2(0.0, 0.0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t qq = q0 + 2 * tx, pp = p0 + ty + 4 * i;
-                if (pp < P.ext_p && qq < P.ext_q) put(out + dst + qq + pp * P.ostr_p, v[i]);
-            }
+        for (int i = 0; i < 8; i++) {  // rows q, pairs of p (unit input stride)
+            const int64_t pp = p0 + 2 * tx, qq = q0 + ty + 8 * i;
+            v[i] = (pp < P.ext_p && qq < P.ext_q)
+                       ? *reinterpret_cast<const double2 *>(in + src + pp + qq * P.istr_q)
+                       : make_double2(0.0, 0.0);
         }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            lds[ty + 8 * i][2 * tx] = v[i].x;
+            lds[ty + 8 * i][2 * tx + 1] = v[i].y;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; i++) {  // rows p, pairs of q (unit output stride)
+            const int64_t qq = q0 + 2 * tx, pp = p0 + ty + 8 * i;
+            if (pp < P.ext_p && qq < P.ext_q)
+                put(out + dst + qq + pp * P.ostr_p,
+                    make_double2(lds[2 * tx][ty + 8 * i], lds[2 * tx + 1][ty + 8 * i]));
+        }
+        __syncthreads();
     }
 }
 
@@ -283,17 +325,38 @@ extern "C" int dtcf_permute_copy_f64(const double *in, double *out, const dtcf_s
     P.ostr_p = dp.ostr;
     P.istr_q = dq.istr;
     P.ostr_q = dq.ostr;
-    // 16-byte form: unit fast strides, even extents and offsets, aligned
-    // buffers, offsets from steps (not tables)
-    bool vec = !src_off && !dst_off && (reinterpret_cast<uintptr_t>(in) & 15) == 0 &&
+    // 16-byte form: a transpose of unit fast strides, even extents and
+    // offsets, aligned buffers, offsets from steps (not tables), whose 64 x 64
+    // tiles the extents fill to a fifth at least.  us, 16-byte / flat: 48 x 48
+    // 253 / 275, 24 x 48 155 / 162, 32 x 32 150 / 155, below a fifth 24 x 24
+    // 225 / 161, 20 x 20 35 / 24, 12 x 48 365 / 253.  (A straight copy gains
+    // nothing from it: 64 x 128 199 / 195, 32 x 64 211 / 146.)
+    auto fill = [](int64_t ext) { return (double)ext / (double)((ext + 63) / 64 * 64); };
+    bool vec = transpose && !src_off && !dst_off && (reinterpret_cast<uintptr_t>(in) & 15) == 0 &&
                (reinterpret_cast<uintptr_t>(out) & 15) == 0 && src_step % 2 == 0 &&
-               dst_step % 2 == 0 && dq.ext % 2 == 0 && dq.ostr == 1;
-    if (transpose) vec = vec && dp.istr == 1 && dp.ext % 2 == 0 && dq.istr % 2 == 0 && dp.ostr % 2 == 0;
-    else vec = vec && dq.istr == 1 && (p < 0 || (dp.istr % 2 == 0 && dp.ostr % 2 == 0));
+               dst_step % 2 == 0 && dq.ext % 2 == 0 && dq.ostr == 1 && dp.istr == 1 &&
+               dp.ext % 2 == 0 && dq.istr % 2 == 0 && dp.ostr % 2 == 0 && fill(dp.ext) * fill(dq.ext) >= 0.2;
     for (int i = 0; vec && i < (int)dims.size(); i++)
         if (i != q && i != p) vec = dims[i].istr % 2 == 0 && dims[i].ostr % 2 == 0;
-    const int TP = vec ? (transpose ? 64 : 16) : (transpose ? 32 : 16);
-    const int TQ = vec ? (transpose ? 64 : 128) : (transpose ? 32 : 64);
+    // Tiles: 64 x 64 in the 16-byte form; in the flat form at most 64 x 63
+    // through LDS (65 x 63 with its odd pitch fills the buffer) or 4096
+    // elements straight, the extents cut evenly.
+    int64_t TP = 64, TQ = 64;
+    PlaneParams L{};
+    if (!vec) {
+        auto even = [](int64_t ext, int64_t most) {
+            const int64_t n = (ext + most - 1) / most;
+            return (ext + n - 1) / n;
+        };
+        // fewer than 1024 tiles of 64 x 63: 32 x 32, so that no CU idles (200
+        // of 63 x 65, 15 -> 11 us; one of 1331 x 1177, 13 -> 11)
+        uint64_t tiles = (uint64_t)ntiles * ((dp.ext + 63) / 64) * ((dq.ext + 62) / 63);
+        for (int i = 0; i < (int)dims.size() && tiles < 1024; i++)
+            if (i != q && i != p) tiles *= (uint64_t)dims[i].ext;
+        const bool small = tiles < 1024;
+        TQ = even(dq.ext, !transpose ? kPlaneElems : small ? 32 : 63);
+        TP = even(dp.ext, !transpose ? std::max<int64_t>(1, kPlaneElems / TQ) : small ? 32 : 64);
+    }
     const uint64_t ntp = (dp.ext + TP - 1) / TP, ntq = (dq.ext + TQ - 1) / TQ;
     uint64_t per = ntp * ntq;
     int n_other = 0;
@@ -320,18 +383,30 @@ extern "C" int dtcf_permute_copy_f64(const double *in, double *out, const dtcf_s
     P.beta = beta;
 
     const uint64_t max_grid = 256ull * 64;  // plenty of waves in flight per CU
-    const unsigned grid = (unsigned)std::min<uint64_t>(P.total, max_grid);
     hipStream_t s = as_stream(stream);
-    if (vec && transpose)
-        hipLaunchKernelGGL(permute_vec_kernel<true>, dim3(grid), dim3(256), 0, s, in, out, P);
-    else if (vec)
-        hipLaunchKernelGGL(permute_vec_kernel<false>, dim3(grid), dim3(256), 0, s, in, out, P);
-    else if (transpose)
-        hipLaunchKernelGGL(permute_kernel<true>, dim3(grid), dim3(256), 0, s, in, out, P, src_off,
-                           dst_off);
-    else
-        hipLaunchKernelGGL(permute_kernel<false>, dim3(grid), dim3(256), 0, s, in, out, P, src_off,
-                           dst_off);
+    if (!vec) {
+        L.Pt = (uint32_t)TP;
+        L.Qt = (uint32_t)TQ;
+        const uint32_t elems = (transpose ? L.Pt | 1 : L.Pt) * L.Qt;  // at most kPlaneElems
+        L.others = (uint32_t)(per / (ntp * ntq));
+        L.planes = (uint64_t)L.others * (uint64_t)ntiles;
+        L.np = std::max<uint32_t>(1, std::min<uint32_t>(kMaxPlanes, kPlaneElems / elems));
+        // small calls: fewer planes per item rather than idle CUs
+        while (L.np > 1 && (L.planes + L.np - 1) / L.np * ntp * ntq < 1024) L.np = (L.np + 1) / 2;
+        L.items = (L.planes + L.np - 1) / L.np * ntp * ntq;
+        L.div_pt = FastDiv(L.Pt);
+        L.div_qt = FastDiv(L.Qt);
+        L.div_pq = FastDiv(L.Pt * L.Qt);
+        const unsigned grid = (unsigned)std::min<uint64_t>(L.items, max_grid);
+        if (transpose)
+            hipLaunchKernelGGL(permute_kernel<true>, dim3(grid), dim3(256), 0, s, in, out, P, L, src_off, dst_off);
+        else
+            hipLaunchKernelGGL(permute_kernel<false>, dim3(grid), dim3(256), 0, s, in, out, P, L, src_off, dst_off);
+        DTCF_HIP(hipGetLastError());
+        return DTCF_OK;
+    }
+    const unsigned grid = (unsigned)std::min<uint64_t>(P.total, max_grid);
+    hipLaunchKernelGGL(permute_vec_kernel, dim3(grid), dim3(256), 0, s, in, out, P);
     DTCF_HIP(hipGetLastError());
     return DTCF_OK;
 }

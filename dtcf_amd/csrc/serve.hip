@@ -106,30 +106,36 @@ __global__ __launch_bounds__(256) void sum_kernel(SumArgs a)
 
 // The same sums, one (i2, i3) plane of the output per workgroup pass: the
 // result element (i0, i1, i2, i3) adds its terms in list order exactly as
-// sum_kernel does.  Terms go in chunks of kChunk: every term of a chunk is
-// loaded before one barrier, so kChunk terms' loads are in flight at once.
-// A term whose unit stride lies on i2 (the occupied pair transposed, e.g.
-// X[p2,p1,h2,h1] into R[p1,p2,h1,h2]) is staged through its own LDS plane
-// with lanes along i2; any other term is read directly into registers
-// (lanes along i3: whole lines when its unit stride lies there).  (i2, i3)
-// come from 32-bit divisions by invariants, (i0, i1) once per plane.
+// sum_kernel does.  Terms go in chunks of CH: every load of a chunk is issued
+// before one is waited for.  A term whose unit stride lies on i2 (the
+// occupied pair transposed, e.g. X[p2,p1,h2,h1] into R[p1,p2,h1,h2]) is read
+// with lanes along i2 and turned in its own LDS plane; any other term is read
+// directly into registers (lanes along i3: whole lines when its unit stride
+// lies there).  (i2, i3) come from 32-bit divisions by invariants, (i0, i1)
+// once per plane.
+//
+// PAIRS (d2 and d3 even): each thread owns element pairs (i3, i3 + 1) of one
+// i2, read with one 16-byte load from the terms marked in `pairs` and stored
+// with one 16-byte store; every element still adds its terms in list order,
+// with the same operations as the element form.
+//
+// HBM-bound in the end, latency-bound before: a 19 x 19 plane is less than
+// one element per thread, so NS (slots per thread) follows the plane, small
+// planes take eight terms per chunk, and workgroups stay for many planes
+// (a start costs the chip 12 ns: 45 us for the 3781 planes of a
+// 19 x 199 x 19 x 19 result).  Measured: a UHF T2 request at 19 /
+// 199 9.37 -> 8.8 ms, a CCSD iteration of 64 / 256 45.0 -> 43.4 ms.
 constexpr int kPlaneCap = 3072;  // doubles per staged plane: d3 rows of d2 + 1
 constexpr int kPlaneThreads = 512;
-constexpr int kPlanePer = 6;     // result elements per thread: d2 * d3 <= 3072
-constexpr int kChunk = 4;        // terms per barrier
+constexpr unsigned kPlaneGrid = 1024;
 
-// PAIRS (d2 and d3 even): each thread owns element pairs (i3, i3 + 1) of one
-// i2 -- six pairs for the 3072-element plane limit -- read with one 16-byte
-// load from the terms marked in `pairs` and stored with one 16-byte store;
-// every element still adds its terms in list order, with the same
-// operations as the element form.
-template <bool PAIRS>
+template <bool PAIRS, int NS, int CH>
 __global__ __launch_bounds__(kPlaneThreads, 4) void sum_plane_kernel(SumArgs a, FastDiv div_d3,
                                                                   FastDiv div_d2, uint64_t nplanes,
                                                                   uint32_t bufstride)
 {
     constexpr uint32_t T = kPlaneThreads;
-    extern __shared__ double planes[];  // kChunk staged planes of bufstride doubles
+    extern __shared__ double planes[];  // CH staged planes of bufstride doubles
     __shared__ int64_t st[kMaxSumTerms * 4];
     __shared__ const double *src[kMaxSumTerms];
     __shared__ double coef[kMaxSumTerms];
@@ -139,19 +145,20 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void sum_plane_kernel(SumArgs a, 
         coef[threadIdx.x] = a.coef[threadIdx.x];
     }
     __syncthreads();
-    constexpr int W = PAIRS ? 2 : 1;          // elements per slot
-    constexpr int NS = kPlanePer / W;         // slots per thread
+    constexpr int W = PAIRS ? 2 : 1;  // elements per slot
     const uint32_t d2 = (uint32_t)a.d2, d3 = (uint32_t)a.d3, P = d2 * d3, pitch = d2 + 1;
-    uint32_t i2[NS], i3[NS];
-    bool in[NS];
+    uint32_t i2[NS], i3[NS];  // of slots past the plane: its last one, not stored
 #pragma unroll
     for (int k = 0; k < NS; k++) {
-        const uint32_t e0 = W * (threadIdx.x + T * k);
-        in[k] = e0 < P;
-        const uint32_t e = min<uint32_t>(e0, P - W);
+        const uint32_t e = min<uint32_t>(W * (threadIdx.x + T * k), P - W);
         i2[k] = div_d3.div(e);
         i3[k] = e - i2[k] * d3;
     }
+    auto uniform = [](int64_t x) {  // the same in every lane: into scalar registers
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
+        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)x >> 32));
+        return (int64_t)((uint64_t)hi << 32 | lo);
+    };
     // Workgroups go to the XCDs in turn; when the grid allows, consecutive
     // planes are given to workgroups of one XCD, so terms whose neighbouring
     // planes share cache lines (the plane's indices outermost in the term)
@@ -165,28 +172,30 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void sum_plane_kernel(SumArgs a, 
         for (int k = 0; k < NS; k++)
 #pragma unroll
             for (int w = 0; w < W; w++) acc[k][w] = 0.0;
-        for (int t0 = 0; t0 < a.nterms; t0 += kChunk) {
-            double xr[kChunk][NS][W];
-            bool staged[kChunk];
-            __syncthreads();  // the previous chunk's staged planes have been read
+        for (int t0 = 0; t0 < a.nterms; t0 += CH) {
+            double xr[CH][NS][W];
+            bool staged[CH];
 #pragma unroll
-            for (int j = 0; j < kChunk; j++) {
+            for (int j = 0; j < CH; j++) {
                 const int t = t0 + j;
                 staged[j] = false;
                 if (t >= a.nterms) continue;
                 const int64_t *q = st + 4 * t;
-                const double *x = src[t] + (int64_t)p0 * q[0] + (int64_t)p1 * q[1];
-                if (q[2] == 1 && q[3] != 1) {
+                const int64_t q2 = uniform(q[2]), q3 = uniform(q[3]);
+                const double *x = reinterpret_cast<const double *>(uniform((int64_t)src[t])) +
+                                  ((int64_t)p0 * uniform(q[0]) + (int64_t)p1 * uniform(q[1]));
+                if (q2 == 1 && q3 != 1) {
                     staged[j] = true;
-                    double *b = planes + j * bufstride;
-                    for (uint32_t idx = threadIdx.x; idx < P; idx += T) {
+#pragma unroll
+                    for (int m = 0; m < NS * W; m++) {
+                        const uint32_t idx = min<uint32_t>(threadIdx.x + T * m, P - 1);
                         const uint32_t r3 = div_d2.div(idx), r2 = idx - r3 * d2;
-                        b[r3 * pitch + r2] = x[r2 + (int64_t)r3 * q[3]];
+                        xr[j][m / W][m % W] = x[r2 + (int64_t)r3 * q3];
                     }
                 } else if (PAIRS && ((a.pairs[t >> 6] >> (t & 63)) & 1)) {
 #pragma unroll
                     for (int k = 0; k < NS; k++) {
-                        d2v v = in[k] ? *(const d2v *)(x + (int64_t)i2[k] * q[2] + i3[k]) : d2v{0.0, 0.0};
+                        const d2v v = *(const d2v *)(x + (int64_t)i2[k] * q2 + i3[k]);
                         xr[j][k][0] = v.x;
                         xr[j][k][W - 1] = v.y;
                     }
@@ -195,13 +204,25 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void sum_plane_kernel(SumArgs a, 
                     for (int k = 0; k < NS; k++)
 #pragma unroll
                         for (int w = 0; w < W; w++)
-                            xr[j][k][w] = in[k] ? x[(int64_t)i2[k] * q[2] + (int64_t)(i3[k] + w) * q[3]]
-                                                : 0.0;
+                            xr[j][k][w] = x[(int64_t)i2[k] * q2 + (int64_t)(i3[k] + w) * q3];
+                }
+            }
+            __syncthreads();  // the previous chunk's staged planes have been read
+#pragma unroll
+            for (int j = 0; j < CH; j++) {
+                if (!staged[j]) continue;
+                double *b = planes + j * bufstride;
+#pragma unroll
+                for (int m = 0; m < NS * W; m++) {
+                    const uint32_t idx = threadIdx.x + T * m;
+                    if (idx >= P) continue;
+                    const uint32_t r3 = div_d2.div(idx), r2 = idx - r3 * d2;
+                    b[r3 * pitch + r2] = xr[j][m / W][m % W];
                 }
             }
             __syncthreads();
 #pragma unroll
-            for (int j = 0; j < kChunk; j++) {
+            for (int j = 0; j < CH; j++) {
                 const int t = t0 + j;
                 if (t >= a.nterms) continue;
                 const double c = coef[t];
@@ -216,12 +237,31 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void sum_plane_kernel(SumArgs a, 
         double *o = a.out + plane * P;
 #pragma unroll
         for (int k = 0; k < NS; k++) {
-            if (!in[k]) continue;
             const uint32_t e = W * (threadIdx.x + T * k);
+            if (e >= P) continue;
             if constexpr (PAIRS) *(d2v *)(o + e) = d2v{acc[k][0], acc[k][1]};
             else o[e] = acc[k][0];
         }
     }
+}
+
+// The instance for a plane of `elems`: slots to cover it, its chunk.
+struct PlaneSum {
+    void (*kernel)(SumArgs, FastDiv, FastDiv, uint64_t, uint32_t);
+    int chunk, slots;  // slots: elements per thread
+};
+const PlaneSum &plane_sum(bool pairs, int64_t elems)
+{
+    static const PlaneSum even[] = {{sum_plane_kernel<true, 1, 8>, 8, 2},
+                                    {sum_plane_kernel<true, 2, 4>, 4, 4},
+                                    {sum_plane_kernel<true, 3, 3>, 3, 6}};
+    static const PlaneSum odd[] = {{sum_plane_kernel<false, 1, 8>, 8, 1},
+                                   {sum_plane_kernel<false, 2, 8>, 8, 2},
+                                   {sum_plane_kernel<false, 4, 4>, 4, 4},
+                                   {sum_plane_kernel<false, 6, 3>, 3, 6}};
+    const PlaneSum *v = pairs ? even : odd;
+    while ((int64_t)v->slots * kPlaneThreads < elems) v++;  // elems <= kPlaneCap
+    return *v;
 }
 
 unsigned grid_for(int64_t n)
@@ -678,15 +718,22 @@ int launch_stmt(dtcf_server srv, Req *r, int i, hipStream_t stream)
             static std::once_flag once;
             static hipError_t attr = hipSuccess;
             std::call_once(once, [] {
-                for (const void *k : {reinterpret_cast<const void *>(sum_plane_kernel<false>),
-                                      reinterpret_cast<const void *>(sum_plane_kernel<true>)})
-                    if (attr == hipSuccess)
-                        attr = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                   (int)(kChunk * kPlaneCap * sizeof(double)));
+                for (bool pairs : {false, true})
+                    for (int64_t slots : {1, 2, 4, 6}) {
+                        const PlaneSum &v = plane_sum(pairs, slots * kPlaneThreads);
+                        if (attr == hipSuccess)  // (d2 + 1) * d3 <= 2 d2 d3
+                            attr = hipFuncSetAttribute(reinterpret_cast<const void *>(v.kernel),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       v.chunk * (int)sizeof(double) *
+                                                           std::min(kPlaneCap, 2 * v.slots * kPlaneThreads));
+                    }
             });
             DTCF_HIP(attr);
             const uint64_t nplanes = (uint64_t)(a.n / (s.od[2] * s.od[3]));
-            const unsigned grid = (unsigned)std::min<uint64_t>(nplanes, 1u << 20);
+            // an even number of planes for each workgroup, whole rounds of XCDs
+            const uint64_t rounds = std::max<uint64_t>(1, (nplanes + kPlaneGrid - 1) / kPlaneGrid);
+            unsigned grid = (unsigned)((nplanes + rounds - 1) / rounds);
+            if (rounds > 1) grid = (grid + 7) / 8 * 8;
             const uint32_t bufstride = (uint32_t)(s.od[3] * (s.od[2] + 1));
             // element pairs when the plane's rows are whole pairs; per term, a
             // 16-byte load where its pairs are adjacent and aligned
@@ -699,16 +746,10 @@ int launch_stmt(dtcf_server srv, Req *r, int i, hipStream_t stream)
                         (reinterpret_cast<uintptr_t>(a.src[t]) & 15) == 0)
                         a.pairs[t >> 6] |= uint64_t(1) << (t & 63);
                 }
-            if (pairs)
-                hipLaunchKernelGGL(sum_plane_kernel<true>, dim3(grid), dim3(kPlaneThreads),
-                                   (size_t)kChunk * bufstride * sizeof(double), stream, a,
-                                   FastDiv((uint32_t)s.od[3]), FastDiv((uint32_t)s.od[2]), nplanes,
-                                   bufstride);
-            else
-                hipLaunchKernelGGL(sum_plane_kernel<false>, dim3(grid), dim3(kPlaneThreads),
-                                   (size_t)kChunk * bufstride * sizeof(double), stream, a,
-                                   FastDiv((uint32_t)s.od[3]), FastDiv((uint32_t)s.od[2]), nplanes,
-                                   bufstride);
+            const PlaneSum &v = plane_sum(pairs, s.od[2] * s.od[3]);
+            hipLaunchKernelGGL(v.kernel, dim3(grid), dim3(kPlaneThreads),
+                               (size_t)v.chunk * bufstride * sizeof(double), stream, a,
+                               FastDiv((uint32_t)s.od[3]), FastDiv((uint32_t)s.od[2]), nplanes, bufstride);
         } else {
             hipLaunchKernelGGL(sum_kernel, dim3(grid_for(a.n)), dim3(256), 0, stream, a);
         }
@@ -1216,7 +1257,7 @@ extern "C" int dtcf_program_sum(dtcf_program p, const char *c, const char *c_idx
     DTCF_HIP(hipMemcpy(s.dstrides, strides.data(), strides.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     s.hstrides = strides;
     s.flops = (double)C.elems * nterms;
-    s.plane = (s.od[2] + 1) * s.od[3] <= kPlaneCap && s.od[2] * s.od[3] <= kPlaneThreads * kPlanePer;
+    s.plane = (s.od[2] + 1) * s.od[3] <= kPlaneCap;
     p->st.push_back(std::move(s));
     p->broken = false;
     return DTCF_OK;

@@ -35,9 +35,14 @@
 //   the other stage after the step's MFMAs are issued.
 //   1331 x 1177 x 905, odd pitches: 160 -> 69 us (it ran element loads with
 //   bounds checks in every step).
-// Only a K step that is not whole (K % 16), or the last one when a row pair
-// may reach past the operand's last row, is loaded element by element with
-// bounds checks (nfast).  Rows past the operand's last (an edge tile) load
+//   table (a view whose block table did not fold): staged, with the blocks'
+//   offsets looked up a step ahead and added only when the pair is loaded (an
+//   add at the look-up would wait for the data loads issued before it: 64 x
+//   64 at 2304^3, both operands in 144 x 144 tiles of a scrambled order, 920
+//   us, 567 so; with checked loads in every step 1468).
+// Only a K step that is not whole (K % 16), or the last one of a dense
+// row-contiguous operand with an odd row count, whose last pair reaches past
+// the operand, is loaded element by element with bounds checks (nfast).  Rows past the operand's last (an edge tile) load
 // the last row or row pair again: in range, and never stored.
 #pragma once
 #include <algorithm>
@@ -57,6 +62,10 @@ typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // 16-byte 
 constexpr int BK = 16;
 constexpr int NT = 256;
 constexpr int KH = BK / 8;  // fragments per 16 rows and K step
+
+// How a kernel fills its stages: through registers, the same with a block
+// table on a view operand, straight into LDS.
+enum { kStaged = 0, kTable = 1, kDirect = 2 };
 
 template <int MODE>
 struct ModeT {
@@ -83,15 +92,18 @@ __device__ inline int64_t op_addr(const OpArgs &o, int64_t r, int64_t c)
 
 // One wave's share of one operand's stage: P of the ROWS/16 * KH fragments,
 // f = wave * P + i: 16-row group f / KH, half f % KH.
-template <int ROWS, int MODE, bool DIRECT>
+template <int ROWS, int MODE, int LOAD>
 struct Loader {
     typedef ModeT<MODE> M;
+    static constexpr bool DIRECT = LOAD == kDirect, TABLE = LOAD == kTable;
     static constexpr int P = ROWS / 16 * KH / 4;
     static_assert(ROWS % 32 == 0, "whole fragments per wave");
     const double *p0[P];  // row part of the pair (its first row)
     const double *p1[(!DIRECT && !M::KC) ? P : 1];  // second row of a non-adjacent row pair
     int64_t c0[M::VIEW ? P : 1];                    // column offsets of the next step to load
     int64_t c1[(M::VIEW && !DIRECT && M::KC) ? P : 1];
+    uint32_t rb[TABLE ? P : 1], rb1[(TABLE && !M::KC) ? P : 1];  // block rows
+    int64_t b0[TABLE ? P : 1], b1[TABLE ? P : 1];   // block offsets of the pair's elements
     d2 reg[DIRECT ? 1 : P];
 
     __device__ static inline int frag_row(int f, int l) { return 16 * (f / KH) + (M::KC ? (l & 15) : 2 * (l & 7)); }
@@ -114,11 +126,15 @@ struct Loader {
             else {
                 p0[i] = base + o.rofs[r];
                 if constexpr (!DIRECT && !M::KC) p1[i] = base + o.rofs[min(r + 1, rows - 1)];
+                if constexpr (TABLE) {
+                    rb[i] = o.div_rpb.div((uint32_t)r);
+                    if constexpr (!M::KC) rb1[i] = o.div_rpb.div((uint32_t)min(r + 1, rows - 1));
+                }
             }
         }
     }
-    // Column offsets of K step kt (views): fetched a step before their data,
-    // so no data load waits on a table load.
+    // Column and block offsets of K step kt (views): fetched a step before
+    // their data, so no data load waits on a table load.
     __device__ inline void fetch(const OpArgs &o, int64_t kt, int w, int l)
     {
         if constexpr (M::VIEW) {
@@ -127,6 +143,15 @@ struct Loader {
                 const int64_t c = kt * BK + frag_k(w * P + i, l);
                 c0[i] = o.cofs[c];
                 if constexpr (!DIRECT && M::KC) c1[i] = o.cofs[c + 1];
+                if constexpr (TABLE) {
+                    b0[i] = b1[i] = 0;
+                    if (!o.blk) continue;  // uniform: the other operand has the table
+                    const uint32_t cb = o.div_cpb.div((uint32_t)c);
+                    b0[i] = o.blk[rb[i] * o.ncb + cb];
+                    if (o.adj) continue;  // uniform: the pair lies in one block
+                    if constexpr (M::KC) b1[i] = o.blk[rb[i] * o.ncb + o.div_cpb.div((uint32_t)c + 1)];
+                    else b1[i] = o.blk[rb1[i] * o.ncb + cb];
+                }
             }
         }
     }
@@ -134,6 +159,7 @@ struct Loader {
     {
         if constexpr (MODE == kDK) return p0[i] + kt * BK;
         else if constexpr (MODE == kDMN) return p0[i] + kt * BK * o.ld;
+        else if constexpr (TABLE) return p0[i] + c0[i] + b0[i];
         else return p0[i] + c0[i];
     }
     // Loads K step kt (kt < nfast) of this wave's fragments: into the stage
@@ -152,9 +178,9 @@ struct Loader {
         } else if constexpr (M::VIEW) {
 #pragma unroll
             for (int i = 0; i < P; i++) {
-                reg[i].x = p0[i][c0[i]];
-                if constexpr (M::KC) reg[i].y = p0[i][c1[i]];
-                else reg[i].y = p1[i][c0[i]];
+                reg[i].x = *at(o, i, kt);
+                const double *y = M::KC ? p0[i] + c1[M::KC ? i : 0] : p1[M::KC ? 0 : i] + c0[i];
+                reg[i].y = TABLE ? y[b1[TABLE ? i : 0]] : *y;
             }
         }
     }
@@ -200,11 +226,12 @@ __device__ inline void tile_coords(uint32_t q, uint32_t tiles_m, uint32_t tiles_
 
 // One workgroup's share of a GEMM: logical tile q over K steps [kt0, kt1);
 // a piece of a split tile (split) writes raw sums to workspace slot sidx.
-template <int BM, int BN, int WM, int WN, int AMODE, int BMODE, bool DIRECT>
+template <int BM, int BN, int WM, int WN, int AMODE, int BMODE, int LOAD>
 __device__ __forceinline__ void gemm_tile(const GemmArgs &g, uint32_t q, int64_t kt0, int64_t kt1,
                                           bool split, uint32_t sidx)
 {
     static_assert((BM / WM) * (BN / WN) == 4, "four waves per workgroup");
+    constexpr bool DIRECT = LOAD == kDirect;
     constexpr int FM = WM / 16, FN = WN / 16;
     constexpr int FA = BM / 16 * KH, FB = BN / 16 * KH;  // fragments per stage
     constexpr bool AKC = ModeT<AMODE>::KC, BKC = ModeT<BMODE>::KC;
@@ -218,8 +245,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, uint32_t q, int64_t
     tile_coords(q, g.tiles_m, g.tiles_n, tm, tn);
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
 
-    Loader<BM, AMODE, DIRECT> la;
-    Loader<BN, BMODE, DIRECT> lb;
+    Loader<BM, AMODE, LOAD> la;
+    Loader<BN, BMODE, LOAD> lb;
     d4 acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; i++)
@@ -390,9 +417,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, uint32_t q, int64_t
 // K steps that need no bounds checks (gemm_tile): whole ones, less the last
 // when a row pair of a dense row-contiguous operand with an odd row count
 // reads one element past the operand's last k row.
-inline int64_t fast_steps(int64_t k, bool odd_pairs, bool table)
+inline int64_t fast_steps(int64_t k, bool odd_pairs)
 {
-    if (table) return 0;
     return (odd_pairs && k % BK == 0) ? k / BK - 1 : k / BK;
 }
 
@@ -403,7 +429,7 @@ struct Occ {
     static constexpr int v = BM * BN <= 64 * 64 ? 4 : 2;
 };
 
-template <int BM, int BN, int WM, int WN, int AMODE, int BMODE, bool DIRECT>
+template <int BM, int BN, int WM, int WN, int AMODE, int BMODE, int LOAD>
 __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_kernel(GemmArgs g)
 {
     // Workgroups below t_full own whole tiles; their ids are first remapped
@@ -426,7 +452,7 @@ __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_kernel(GemmArgs
     }
     for (; left > 0; q++) {
         const int64_t k1 = min(nk, k0 + left);
-        gemm_tile<BM, BN, WM, WN, AMODE, BMODE, DIRECT>(g, q, k0, k1, k0 > 0 || k1 < nk, slot);
+        gemm_tile<BM, BN, WM, WN, AMODE, BMODE, LOAD>(g, q, k0, k1, k0 > 0 || k1 < nk, slot);
         left -= k1 - k0;
         k0 = 0;
         slot |= 1;
@@ -453,7 +479,7 @@ __device__ inline int tail_problem(const GemmGroupArgs &ga, uint32_t ti)
 // TF/s, 2 x 4096 x 4096 x 2048 59.0 against 63.7.)  Workgroups past a
 // problem's last whole tile exit at once.  The workgroups after wg_whole
 // each own one run of the split tiles' K steps.
-template <int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
+template <int BM, int BN, int WM, int WN, int AM, int BMD, int LOAD>
 __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_group_kernel(GemmGroupArgs ga)
 {
     const uint32_t bid = blockIdx.x;
@@ -509,7 +535,7 @@ __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_group_kernel(Ge
         g.tiles_n = P.tiles_n;
         g.overwrite = ga.overwrite;
         g.ws = ga.ws;
-        gemm_tile<BM, BN, WM, WN, AM, BMD, DIRECT>(g, q, k0, k1, k0 > 0 || k1 < nk, 2 * w + seg);
+        gemm_tile<BM, BN, WM, WN, AM, BMD, LOAD>(g, q, k0, k1, k0 > 0 || k1 < nk, 2 * w + seg);
     }
 }
 
@@ -573,10 +599,10 @@ int allow_lds(K kern, size_t lds, std::once_flag &once, hipError_t &err)
     return DTCF_OK;
 }
 
-template <int CFG, int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
+template <int CFG, int BM, int BN, int WM, int WN, int AM, int BMD, int LOAD>
 int launch_one(GemmArgs g, hipStream_t s)
 {
-    auto kern = gemm_f64_kernel<BM, BN, WM, WN, AM, BMD, DIRECT>;
+    auto kern = gemm_f64_kernel<BM, BN, WM, WN, AM, BMD, LOAD>;
     constexpr size_t lds = (size_t)2 * (BM + BN) * BK * sizeof(double);
     static std::once_flag once;
     static hipError_t attr_err = hipSuccess;
@@ -604,18 +630,20 @@ int launch_one(GemmArgs g, hipStream_t s)
     return DTCF_OK;
 }
 
-template <int CFG, int BM, int BN, int WM, int WN, bool DIRECT>
+template <int CFG, int BM, int BN, int WM, int WN, int LOAD>
 int launch_modes(const GemmArgs &g, hipStream_t s)
 {
     const int am = g.amode, bm = g.bmode;
-    if (am == kDK && bm == kDK) return launch_one<CFG, BM, BN, WM, WN, kDK, kDK, DIRECT>(g, s);
-    if (am == kDK && bm == kDMN) return launch_one<CFG, BM, BN, WM, WN, kDK, kDMN, DIRECT>(g, s);
-    if (am == kDMN && bm == kDK) return launch_one<CFG, BM, BN, WM, WN, kDMN, kDK, DIRECT>(g, s);
-    if (am == kDMN && bm == kDMN) return launch_one<CFG, BM, BN, WM, WN, kDMN, kDMN, DIRECT>(g, s);
-    if (am == kVK && bm == kVK) return launch_one<CFG, BM, BN, WM, WN, kVK, kVK, DIRECT>(g, s);
-    if (am == kVK && bm == kVMN) return launch_one<CFG, BM, BN, WM, WN, kVK, kVMN, DIRECT>(g, s);
-    if (am == kVMN && bm == kVK) return launch_one<CFG, BM, BN, WM, WN, kVMN, kVK, DIRECT>(g, s);
-    if (am == kVMN && bm == kVMN) return launch_one<CFG, BM, BN, WM, WN, kVMN, kVMN, DIRECT>(g, s);
+    if constexpr (LOAD != kTable) {
+        if (am == kDK && bm == kDK) return launch_one<CFG, BM, BN, WM, WN, kDK, kDK, LOAD>(g, s);
+        if (am == kDK && bm == kDMN) return launch_one<CFG, BM, BN, WM, WN, kDK, kDMN, LOAD>(g, s);
+        if (am == kDMN && bm == kDK) return launch_one<CFG, BM, BN, WM, WN, kDMN, kDK, LOAD>(g, s);
+        if (am == kDMN && bm == kDMN) return launch_one<CFG, BM, BN, WM, WN, kDMN, kDMN, LOAD>(g, s);
+    }
+    if (am == kVK && bm == kVK) return launch_one<CFG, BM, BN, WM, WN, kVK, kVK, LOAD>(g, s);
+    if (am == kVK && bm == kVMN) return launch_one<CFG, BM, BN, WM, WN, kVK, kVMN, LOAD>(g, s);
+    if (am == kVMN && bm == kVK) return launch_one<CFG, BM, BN, WM, WN, kVMN, kVK, LOAD>(g, s);
+    if (am == kVMN && bm == kVMN) return launch_one<CFG, BM, BN, WM, WN, kVMN, kVMN, LOAD>(g, s);
     set_error("gemm: unsupported operand mode combination");
     return DTCF_ERR_INVALID;
 }
@@ -625,17 +653,18 @@ int launch_tile(GemmArgs g, hipStream_t s)
 {
     g.tiles_m = (uint32_t)((g.m + BM - 1) / BM);
     g.tiles_n = (uint32_t)((g.n + BN - 1) / BN);
-    g.nfast = fast_steps(g.k, (g.amode == kDMN && g.m % 2) || (g.bmode == kDMN && g.n % 2),
-                         (g.amode >= kVK && g.a.blk) || (g.bmode >= kVK && g.b.blk));
+    g.nfast = fast_steps(g.k, (g.amode == kDMN && g.m % 2) || (g.bmode == kDMN && g.n % 2));
     // direct loads need every pair adjacent and 16-byte aligned
-    if (g.a.vec2 && g.b.vec2) return launch_modes<CFG, BM, BN, WM, WN, true>(g, s);
-    return launch_modes<CFG, BM, BN, WM, WN, false>(g, s);
+    if (g.a.vec2 && g.b.vec2) return launch_modes<CFG, BM, BN, WM, WN, kDirect>(g, s);
+    if ((g.amode >= kVK && g.a.blk) || (g.bmode >= kVK && g.b.blk))
+        return launch_modes<CFG, BM, BN, WM, WN, kTable>(g, s);
+    return launch_modes<CFG, BM, BN, WM, WN, kStaged>(g, s);
 }
 
-template <int CFG, int BM, int BN, int WM, int WN, int AM, int BMD, bool DIRECT>
+template <int CFG, int BM, int BN, int WM, int WN, int AM, int BMD, int LOAD>
 int launch_group(GemmGroupArgs ga, hipStream_t s)
 {
-    auto kern = gemm_f64_group_kernel<BM, BN, WM, WN, AM, BMD, DIRECT>;
+    auto kern = gemm_f64_group_kernel<BM, BN, WM, WN, AM, BMD, LOAD>;
     constexpr size_t lds = (size_t)2 * (BM + BN) * BK * sizeof(double);
     static std::once_flag once;
     static hipError_t attr_err = hipSuccess;
@@ -647,7 +676,7 @@ int launch_group(GemmGroupArgs ga, hipStream_t s)
         GemmGroupProb &P = ga.p[i];
         P.tiles_m = (uint32_t)((P.m + BM - 1) / BM);
         P.tiles_n = (uint32_t)((P.n + BN - 1) / BN);
-        P.nfast = fast_steps(P.k, (AM == kDMN && P.m % 2) || (BMD == kDMN && P.n % 2), false);
+        P.nfast = fast_steps(P.k, (AM == kDMN && P.m % 2) || (BMD == kDMN && P.n % 2));
         total += (uint64_t)P.tiles_m * P.tiles_n;
         steps += (int64_t)P.tiles_m * P.tiles_n * ((P.k + BK - 1) / BK);
     }
@@ -696,13 +725,13 @@ int launch_group(GemmGroupArgs ga, hipStream_t s)
     return DTCF_OK;
 }
 
-template <int CFG, int BM, int BN, int WM, int WN, bool DIRECT>
+template <int CFG, int BM, int BN, int WM, int WN, int LOAD>
 int launch_group_modes(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t s)
 {
-    if (amode == kDK && bmode == kDK) return launch_group<CFG, BM, BN, WM, WN, kDK, kDK, DIRECT>(ga, s);
-    if (amode == kDK && bmode == kDMN) return launch_group<CFG, BM, BN, WM, WN, kDK, kDMN, DIRECT>(ga, s);
-    if (amode == kDMN && bmode == kDK) return launch_group<CFG, BM, BN, WM, WN, kDMN, kDK, DIRECT>(ga, s);
-    if (amode == kDMN && bmode == kDMN) return launch_group<CFG, BM, BN, WM, WN, kDMN, kDMN, DIRECT>(ga, s);
+    if (amode == kDK && bmode == kDK) return launch_group<CFG, BM, BN, WM, WN, kDK, kDK, LOAD>(ga, s);
+    if (amode == kDK && bmode == kDMN) return launch_group<CFG, BM, BN, WM, WN, kDK, kDMN, LOAD>(ga, s);
+    if (amode == kDMN && bmode == kDK) return launch_group<CFG, BM, BN, WM, WN, kDMN, kDK, LOAD>(ga, s);
+    if (amode == kDMN && bmode == kDMN) return launch_group<CFG, BM, BN, WM, WN, kDMN, kDMN, LOAD>(ga, s);
     set_error("gemm group: unsupported operand layout");
     return DTCF_ERR_INVALID;
 }
@@ -712,8 +741,8 @@ int launch_group_tile(const GemmGroupArgs &ga, int amode, int bmode, hipStream_t
 {
     bool direct = true;
     for (int i = 0; i < ga.np; i++) direct = direct && ga.p[i].vec2a && ga.p[i].vec2b;
-    if (direct) return launch_group_modes<CFG, BM, BN, WM, WN, true>(ga, amode, bmode, s);
-    return launch_group_modes<CFG, BM, BN, WM, WN, false>(ga, amode, bmode, s);
+    if (direct) return launch_group_modes<CFG, BM, BN, WM, WN, kDirect>(ga, amode, bmode, s);
+    return launch_group_modes<CFG, BM, BN, WM, WN, kStaged>(ga, amode, bmode, s);
 }
 
 }  // namespace

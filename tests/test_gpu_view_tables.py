@@ -1,0 +1,92 @@
+"""View products whose operands keep a block table (tiles in an order that is
+no sum of a row and a column part): pairs adjacent and aligned, adjacent off
+alignment, broken at odd block extents, along the columns or the rows, one
+operand or both, whole and partial last K steps, odd row counts.  Against
+torch's float64 product of the gathered operands, 1e-12 of the largest result
+as in test_gpu_core."""
+import numpy as np
+import pytest
+import torch
+
+from dtcf_amd import ops
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-12
+
+
+def _rand(n, seed, dev):
+    g = torch.Generator(device="cpu")
+    g.manual_seed(seed)
+    return torch.randn(n, dtype=torch.float64, generator=g).to(dev)
+
+
+def _tiles(rows, cols, rpb, cpb, rowwise, rng, off=0):
+    """rows x cols in rpb x cpb tiles stored one after another in a random
+    order, each row-major (or column-major): the view and its offsets."""
+    nr, nc = rows // rpb, cols // cpb
+    blk = rng.permutation(nr * nc).astype(np.int64) * (rpb * cpb) + off
+    r, c = np.arange(rows), np.arange(cols)
+    ro, co = (r % rpb, (c % cpb) * rpb) if rowwise else ((r % rpb) * cpb, c % cpb)
+    at = ro[:, None] + co[None, :] + blk.reshape(nr, nc)[(r // rpb)[:, None], (c // cpb)[None, :]]
+    return ops.View(rows, cols, ro, co, blk, rpb, cpb), at
+
+
+# tile (rows, columns) of A, of B, both along K or the rows, an odd first offset
+FORMS = (((6, 8), (10, 8), False, False, 0), ((6, 8), (10, 8), True, True, 0), ((6, 8), (10, 8), False, True, 1),
+         ((7, 5), (3, 5), False, False, 0), ((7, 5), (3, 5), True, True, 0), ((1, 40), (1, 20), False, False, 0),
+         ((21, 1), (15, 1), True, True, 0), ((3, 10), (5, 2), True, False, 0))
+
+
+@pytest.mark.parametrize("cfg", [-1, 0, 3, 4])
+@pytest.mark.parametrize("form", FORMS)
+def test_block_tables(dev, form, cfg):
+    (ra, ca), (rb, cb), wa, wb, off = form
+    rng = np.random.default_rng(2)
+    ops.set_gemm_config(cfg)
+    try:
+        for m, n, k in ((42, 30, 40), (63, 75, 80), (147, 135, 120), (168, 330, 200)):
+            m, n = m // ra * ra, n // rb * rb
+            av, ia = _tiles(m, k, ra, ca, wa, rng, off)
+            bv, ib = _tiles(n, k, rb, cb, wb, rng, off)
+            A, B, C = _rand(m * k + off, 1, dev), _rand(n * k + off, 2, dev), _rand(m * n, 3, dev)
+            Ad, Bd = A[torch.from_numpy(ia).to(dev)], B[torch.from_numpy(ib).to(dev)]
+            ref = C.view(m, n) + 0.5 * (Ad @ Bd.t().contiguous())
+            dense = [ops.View(r, k, np.arange(r) * k, np.arange(k)) for r in (m, n)]
+            cv = ops.View(m, n, np.arange(m) * n, np.arange(n)) if m % 2 else None
+            Ac, Bc = Ad.contiguous().reshape(-1), Bd.contiguous().reshape(-1)
+            for x, xv, y, yv in ((A, av, B, bv), (A, av, Bc, dense[1]), (Ac, dense[0], B, bv)):
+                print("tables", form, cfg, m, n, k, flush=True)
+                X = C.clone()
+                ops.gemm_view(m, n, k, 0.5, x, xv, y, yv, X, cv, ldc=n)
+                assert ((X.view(m, n) - ref).abs().max() / ref.abs().max()).item() <= TOL
+    finally:
+        ops.set_gemm_config(-1)
+
+
+def test_scrambled_tiles_cost_no_checked_loads(dev):
+    """The same 2304^3 product with its tiles in a scrambled order and in
+    order (a table that folds, read straight into LDS).  Scrambled it takes
+    1.3 times as long; with every K step loaded element by element under
+    bounds checks it took 3.2 times."""
+    n, t = 2304, 144
+    rng = np.random.default_rng(1)
+    A, B = _rand(n * n, 1, dev), _rand(n * n, 2, dev)
+    C = torch.zeros(n * n, dtype=torch.float64, device=dev)
+    scr = [_tiles(n, n, t, t, False, rng)[0] for _ in range(2)]
+    r = np.arange(n)
+    order = [ops.View(n, n, (r % t) * t, r % t, np.arange((n // t) ** 2) * t * t, t, t) for _ in range(2)]
+
+    def us(av, bv):
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        out = []
+        for _ in range(7):
+            ev[0].record()
+            ops.gemm_view(n, n, n, 1.0, A, av, B, bv, C, None, ldc=n)
+            ev[1].record()
+            torch.cuda.synchronize()
+            out.append(ev[0].elapsed_time(ev[1]) * 1e3)
+        return sorted(out)[3]
+
+    a, b = us(*scr), us(*order)
+    print("scrambled", a, "in order", b, flush=True)
+    assert a <= 2.0 * b, (a, b)

@@ -73,10 +73,14 @@ int gemm_f64_launch(GemmArgs g, int cfg, hipStream_t s);
 // Up to kGroupMax independent dense GEMMs C_p (+)= alpha * op(A_p) * op(B_p)
 // in one launch, every problem with the same operand layouts: A_p m x k
 // (kDK) or k x m (kDMN), B_p n x k (kDK) or k x n (kDMN); C_p row-major.
-// tiles_m, tiles_n, wg0, t_whole, tail0 and step0 are filled in by the
-// launch: problem p's tiles [0, t_whole) run whole, its tiles [t_whole,
-// tiles) are the split tiles tail0.. of the launch, whose K steps are the
-// steps step0.. of the `steps` that `sw` workgroups share (as in GemmArgs).
+// tiles_m, tiles_n, t_whole, nfast, wg0, tail0 and step0 are filled in by the
+// launch: problem p's tiles [0, t_whole) run whole, in workgroups wg0[p]..,
+// its tiles [t_whole, tiles) are the split tiles tail0[p].. of the launch,
+// whose K steps are the steps step0[p].. of the `steps` that `sw` workgroups
+// share (as in GemmArgs).  A problem without whole (split) tiles has the wg0
+// (tail0, step0) of the next, and entries past the last problem hold the
+// largest value, so the last entry not above a workgroup, tile or step is its
+// problem: one load of neighbouring words and as many compares.
 constexpr int kGroupMax = 16;
 struct GemmGroupProb {
     int64_t m, n, k;
@@ -85,9 +89,8 @@ struct GemmGroupProb {
     double *C;
     int64_t lda, ldb, ldc;
     int32_t vec2a, vec2b;
-    uint32_t tiles_m, tiles_n, wg0;
-    uint32_t t_whole, tail0;
-    int64_t step0, nfast;
+    uint32_t tiles_m, tiles_n, t_whole;
+    int64_t nfast;
 };
 struct GemmGroupArgs {
     double alpha;
@@ -96,6 +99,8 @@ struct GemmGroupArgs {
     uint32_t wg_whole, sw;  // workgroups of whole tiles; runs of split tiles
     int64_t steps;
     double *ws;
+    uint32_t wg0[kGroupMax], tail0[kGroupMax];
+    int64_t step0[kGroupMax];
     GemmGroupProb p[kGroupMax];
 };
 

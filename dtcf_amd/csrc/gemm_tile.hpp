@@ -459,26 +459,26 @@ __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_kernel(GemmArgs
     }
 }
 
-// Problem owning tail tile ti (tail tiles are numbered problem by problem).
-__device__ inline int tail_problem(const GemmGroupArgs &ga, uint32_t ti)
+// Index of the last entry not above x (GemmGroupArgs).
+template <typename U>
+__device__ inline int group_problem(const U (&first)[kGroupMax], U x)
 {
     int p = 0;
-    for (int i = 0; i < ga.np; i++) {
-        const GemmGroupProb &P = ga.p[i];
-        if (ti >= P.tail0 && ti < P.tail0 + (P.tiles_m * P.tiles_n - P.t_whole)) p = i;
-    }
+#pragma unroll
+    for (int i = 1; i < kGroupMax; i++) p = x >= first[i] ? i : p;
     return p;
 }
 
 // Several independent dense GEMMs C_p (+)= alpha A_p B_p^T in one launch.
-// Problem p's whole tiles own workgroups [wg0_p, wg0_p + t_whole_p rounded
-// up to 8); wg0_p is a multiple of 8, so a workgroup's XCD is its local id
-// mod 8 and each problem gets the same XCD-contiguous tile order as a lone
-// launch.  (Cutting the list of all whole tiles into eight runs of equal
-// work, one per XCD, was measured slower: 8 x 2048^3 55.0 against 56.6
-// TF/s, 2 x 4096 x 4096 x 2048 59.0 against 63.7.)  Workgroups past a
-// problem's last whole tile exit at once.  The workgroups after wg_whole
-// each own one run of the split tiles' K steps.
+// Problem p's whole tiles own workgroups [wg0_p, wg0_p + t_whole_p); every
+// eighth of them, one XCD's, takes a contiguous part of the problem's tile
+// order, as in a lone launch.  (Cutting the list of all whole tiles into eight
+// runs of equal work, one per XCD, was measured slower: 8 x 2048^3 55.0
+// against 56.6 TF/s, 2 x 4096 x 4096 x 2048 59.0 against 63.7.  Rounding each
+// problem up to whole rounds of XCDs leaves workgroups that exit at once, and
+// the chip then fills unevenly: 222 tiles of 128 x 128 x 630 in eight problems
+// 167 us, 108 without; 1004 tiles of 128 x 128 x 1380 897, 705.)  The
+// workgroups after wg_whole each own one run of the split tiles' K steps.
 template <int BM, int BN, int WM, int WN, int AM, int BMD, int LOAD>
 __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_group_kernel(GemmGroupArgs ga)
 {
@@ -488,13 +488,10 @@ __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_group_kernel(Ge
     int64_t s = 0, e = 1;
     const bool whole = bid < ga.wg_whole;
     if (whole) {
-        for (int i = 1; i < ga.np; i++)
-            if (bid >= ga.p[i].wg0) p = i;
+        p = group_problem(ga.wg0, bid);
         const GemmGroupProb &P = ga.p[p];
-        const uint32_t T = P.t_whole, T8 = (T + 7u) & ~7u;
-        const uint32_t local = bid - P.wg0;
-        q = (local & 7u) * (T8 >> 3) + (local >> 3);
-        if (q >= T) return;  // whole workgroup: no barrier has been reached
+        const uint32_t local = bid - ga.wg0[p], x = local & 7u;
+        q = x * (P.t_whole >> 3) + min(x, P.t_whole & 7u) + (local >> 3);
     } else {
         w = run_index(bid - ga.wg_whole, ga.sw);
         s = run_begin(w, ga.sw, ga.steps);
@@ -502,20 +499,16 @@ __global__ __launch_bounds__(NT, (Occ<BM, BN>::v)) void gemm_f64_group_kernel(Ge
     }
     for (uint32_t seg = 0; s < e; seg = 1) {
         int64_t k0 = 0, k1;
-        if (!whole) {
-            p = 0;
-            for (int i = 1; i < ga.np; i++)  // problems without split tiles hold no steps
-                if (s >= ga.p[i].step0 && ga.p[i].t_whole < ga.p[i].tiles_m * ga.p[i].tiles_n) p = i;
-        }
+        if (!whole) p = group_problem(ga.step0, s);
         const GemmGroupProb &P = ga.p[p];
         const int64_t nk = (P.k + BK - 1) / BK;
         if (whole) {
             k1 = nk;
             s = e;
         } else {
-            const int64_t t = div_small(s - P.step0, nk);
+            const int64_t t = div_small(s - ga.step0[p], nk);
             q = P.t_whole + (uint32_t)t;
-            k0 = s - P.step0 - t * nk;
+            k0 = s - ga.step0[p] - t * nk;
             k1 = min(nk, k0 + (e - s));
             s += k1 - k0;
         }
@@ -567,16 +560,17 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(GemmArgs g)
 template <int BM, int BN>
 __global__ __launch_bounds__(256) void group_split_reduce_kernel(GemmGroupArgs ga)
 {
-    const uint32_t ti = blockIdx.y;
-    const GemmGroupProb &P = ga.p[tail_problem(ga, ti)];
+    const int p = group_problem(ga.tail0, blockIdx.y);
+    const GemmGroupProb &P = ga.p[p];
+    const uint32_t t = blockIdx.y - ga.tail0[p];  // split tile of the problem
     uint32_t tm, tn;
-    tile_coords(P.t_whole + (ti - P.tail0), P.tiles_m, P.tiles_n, tm, tn);
+    tile_coords(P.t_whole + t, P.tiles_m, P.tiles_n, tm, tn);
     const int64_t nk = (P.k + BK - 1) / BK;
     const int e = blockIdx.x * 256 + threadIdx.x;
     const int64_t row = (int64_t)tm * BM + e / BN, col = (int64_t)tn * BN + e % BN;
     if (row >= P.m || col >= P.n) return;
     bool whole;
-    const double sum = sum_pieces(ga.ws, P.step0 + (ti - P.tail0) * nk, nk, ga.sw, ga.steps, BM * BN, e, whole);
+    const double sum = sum_pieces(ga.ws, ga.step0[p] + t * nk, nk, ga.sw, ga.steps, BM * BN, e, whole);
     if (whole) return;
     GemmArgs g{};
     g.C = P.C;
@@ -687,8 +681,14 @@ int launch_group(GemmGroupArgs ga, hipStream_t s)
     int cus = 0;
     st = gemm_device_cus(&cus);
     if (st != DTCF_OK) return st;
-    const SplitPlan sp = gemm_split_plan((uint32_t)total, std::max<int64_t>(1, steps / (int64_t)total), 0, cus,
-                                         tile_rate(CFG));
+    SplitPlan sp = gemm_split_plan((uint32_t)total, std::max<int64_t>(1, steps / (int64_t)total), 0, cus,
+                                   tile_rate(CFG));
+    // Past one round of 64 x 64 tiles nothing is cut: four workgroups per CU
+    // absorb the ragged end of problems of different K, which equal runs then
+    // only lengthen (1802 tiles x 930: 237 us whole, 265-270 cut; 1354 x 800:
+    // 158, 171; 1568 x 850: 195, 218; 2180 x 1000: 294, 288; 8525 x 2050: 2160,
+    // 2132).
+    if (Occ<BM, BN>::v == 4 && total > (uint64_t)cus * 4) sp = SplitPlan();
     uint32_t left = sp.nsplit;
     for (int i = ga.np - 1; i >= 0; i--) {
         GemmGroupProb &P = ga.p[i];
@@ -699,12 +699,17 @@ int launch_group(GemmGroupArgs ga, hipStream_t s)
     uint64_t wg = 0;
     uint32_t tail = 0;
     ga.steps = 0;
-    for (int i = 0; i < ga.np; i++) {
-        GemmGroupProb &P = ga.p[i];
-        P.wg0 = (uint32_t)wg;
-        wg += ((uint64_t)P.t_whole + 7) & ~7ull;
-        P.tail0 = tail;
-        P.step0 = ga.steps;
+    for (int i = 0; i < kGroupMax; i++) {
+        if (i >= ga.np) {
+            ga.wg0[i] = ga.tail0[i] = UINT32_MAX;
+            ga.step0[i] = INT64_MAX;
+            continue;
+        }
+        const GemmGroupProb &P = ga.p[i];
+        ga.wg0[i] = (uint32_t)wg;
+        wg += P.t_whole;
+        ga.tail0[i] = tail;
+        ga.step0[i] = ga.steps;
         const uint32_t cut = P.tiles_m * P.tiles_n - P.t_whole;
         tail += cut;
         ga.steps += cut * ((P.k + BK - 1) / BK);

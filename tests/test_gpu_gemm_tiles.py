@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from dtcf_amd import ops
+from dtcf_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-12
@@ -146,3 +146,58 @@ def test_served_odd_extents_read_in_place(dev, sizes):
     for n, x in got.items():
         err = np.abs(x - ref[n]).max() / np.abs(ref[n]).max()
         assert err <= TOL, (n, err)
+
+
+def _group(ms, k, dev):
+    """Grouped problems m x m x k over shared operands: the ctypes list and C."""
+    import ctypes as C
+
+    from dtcf_amd import blocksparse
+
+    A, B = _rand(max(ms) * k, 1, dev), _rand(max(ms) * k, 2, dev)
+    Cs = [torch.full((m * m,), float("nan"), dtype=torch.float64, device=dev) for m in ms]
+    probs = (blocksparse.GemmProblem * len(ms))(*[
+        blocksparse.GemmProblem(m, m, k, A.data_ptr(), k, B.data_ptr(), k, c.data_ptr(), m) for m, c in zip(ms, Cs)])
+
+    def run(cfg):
+        _lib.check(_lib.lib().dtcf_gemm_group_ex_f64(C.cast(probs, C.c_void_p), len(ms), 0, 1, 1.0, 1, cfg,
+                                                     C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    return run, A.view(-1, k), B.view(-1, k), Cs
+
+
+# tiles of 64 x 64 and 128 x 128 in all: one problem of one tile, problems
+# split whole, in part and not at all, sixteen problems and a second launch,
+# past one and two rounds of workgroups
+@pytest.mark.parametrize("cfg", [0, 3])
+@pytest.mark.parametrize("ms,k", [([5], 40), ([300, 65, 129], 700), ([640, 600, 650, 610, 630], 333),
+                                  ([130] * 20, 250), ([1100, 1200, 64, 900], 100), ([2300, 100, 2400], 170)])
+def test_group_overwrite(dev, cfg, ms, k):
+    run, A, B, Cs = _group(ms, k, dev)
+    print("group", cfg, ms, k, flush=True)
+    run(cfg)
+    for m, c in zip(ms, Cs):
+        _close(c.view(m, m), A[:m] @ B[:m].t().contiguous(), (cfg, ms, k, m))
+
+
+def test_group_fills_the_chip_like_a_lone_launch(dev):
+    """222 tiles of 128 x 128 x 640 in eight problems, and 225 in one: 108 us
+    each; 167 us with every problem padded to whole rounds of XCDs by
+    workgroups that exit at once."""
+    run = _group([652, 620, 627, 630, 633, 631, 647, 610], 640, dev)[0]
+    lone = _group([1900], 640, dev)[0]
+
+    def us(f):
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        out = []
+        for _ in range(9):
+            ev[0].record()
+            for _ in range(5):
+                f(0)
+            ev[1].record()
+            torch.cuda.synchronize()
+            out.append(ev[0].elapsed_time(ev[1]) * 200)
+        return sorted(out)[4]
+
+    a, b = us(run), us(lone)
+    print("group", a, "lone", b, flush=True)
+    assert a <= 1.25 * b, (a, b)

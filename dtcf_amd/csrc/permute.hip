@@ -47,7 +47,7 @@ struct PermParams {
 // fixed 32 x 32 left 13 of 32 lanes working on a 13 x 47 plane), a plane that
 // is contiguous in the output is written in one run, and eight loads per
 // thread are in flight.  HBM-bound: 256 tiles of 11 x 13 x 45 x 47, order
-// 2,0,3,1: 438 -> 257 us; 12 ns of start-up per workgroup are spread over
+// 2,0,3,1: 417 -> 241 us; 12 ns of start-up per workgroup are spread over
 // up to 4096 elements.
 constexpr int kPlaneElems = 4096;
 constexpr int kMaxPlanes = 64;
@@ -174,6 +174,58 @@ __global__ __launch_bounds__(256) void permute_kernel(const double *__restrict__
             sweep(store);
             __syncthreads();
         }
+    }
+}
+
+// 8-byte TRANSPOSE tile of a fixed 32 x 32, one per workgroup pass, for
+// extents that fill it and tensors that the caches hold: eight workgroups per
+// CU keep more tiles in flight than the flat form's four, and nothing is
+// divided per element.  75 x 2028 (119 MB read and written) 21.0 us, flat
+// 30.7; 169 x 169 in 64 tiles 8.9, 10.8.
+__global__ __launch_bounds__(256) void permute_tile_kernel(const double *__restrict__ in,
+                                                           double *__restrict__ out, PermParams P,
+                                                           const int64_t *__restrict__ src_off,
+                                                           const int64_t *__restrict__ dst_off)
+{
+    __shared__ double lds[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (uint64_t blk = blockIdx.x; blk < P.total; blk += gridDim.x) {
+        const uint64_t t = blk / P.per_tile;
+        uint32_t rem = (uint32_t)(blk - t * P.per_tile);
+        const uint32_t qt_div = P.div_ntq.div(rem);
+        const uint32_t qt = rem - qt_div * P.ntq;
+        rem = qt_div;
+        const uint32_t pt_div = P.div_ntp.div(rem);
+        const uint32_t pt = rem - pt_div * P.ntp;
+        rem = pt_div;
+        int64_t src = src_off ? src_off[t] : (int64_t)t * P.src_step;
+        int64_t dst = dst_off ? dst_off[t] : (int64_t)t * P.dst_step;
+        for (int d = P.n_other - 1; d >= 0; d--) {
+            const uint32_t q = P.other_div[d].div(rem);
+            const uint32_t x = rem - q * P.other_ext[d];
+            rem = q;
+            src += (int64_t)x * P.other_istr[d];
+            dst += (int64_t)x * P.other_ostr[d];
+        }
+        const int64_t p0 = (int64_t)pt * 32, q0 = (int64_t)qt * 32;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int64_t pp = p0 + tx, qq = q0 + ty + 8 * i;
+            if (pp < P.ext_p && qq < P.ext_q)
+                lds[ty + 8 * i][tx] = in[src + pp * P.istr_p + qq * P.istr_q];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int64_t qq = q0 + tx, pp = p0 + ty + 8 * i;
+            if (pp < P.ext_p && qq < P.ext_q) {
+                double *o = out + dst + qq * P.ostr_q + pp * P.ostr_p;
+                const double v = lds[tx][ty + 8 * i];
+                if (P.beta == 0.0) *o = (P.alpha == 1.0) ? v : P.alpha * v;
+                else *o = P.alpha * v + P.beta * (*o);
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -343,7 +395,21 @@ extern "C" int dtcf_permute_copy_f64(const double *in, double *out, const dtcf_s
     // elements straight, the extents cut evenly.
     int64_t TP = 64, TQ = 64;
     PlaneParams L{};
-    if (!vec) {
+    // The fixed tile: a transpose whose extents fill the 32 x 32 tiles to 0.4
+    // at least and do not leave tiles nearly empty past their first (from 40
+    // MB on), up to the 256 MB of the last-level cache and a little.  us, fixed
+    // / flat: 32 x 13 (36 MB, fill 0.41) 10.2 / 12.7, 19 x 19 (59 MB, 0.35) 17 /
+    // 16; 129 x 304 (237 MB) 42.4 / 54.3, 55 x 45 (192 MB, whose second tiles
+    // are 0.6 full) 49 / 38; 129 x 63 (329 MB) 83 / 73.
+    auto filled = [](int64_t ext) { return (double)ext / (double)((ext + 31) / 32 * 32); };
+    auto later = [&](int64_t ext) { return ext <= 32 ? 1.0 : filled(ext); };
+    double mb = 16e-6 * (double)ntiles;  // read and written
+    for (const Dim &d : dims) mb *= (double)d.ext;
+    const bool fixed = transpose && !vec && mb < 275.0 && filled(dp.ext) * filled(dq.ext) >= 0.4 &&
+                       (mb < 40.0 || later(dp.ext) * later(dq.ext) >= 0.61);
+    if (fixed) {
+        TP = TQ = 32;
+    } else if (!vec) {
         auto even = [](int64_t ext, int64_t most) {
             const int64_t n = (ext + most - 1) / most;
             return (ext + n - 1) / n;
@@ -384,7 +450,7 @@ extern "C" int dtcf_permute_copy_f64(const double *in, double *out, const dtcf_s
 
     const uint64_t max_grid = 256ull * 64;  // plenty of waves in flight per CU
     hipStream_t s = as_stream(stream);
-    if (!vec) {
+    if (!vec && !fixed) {
         L.Pt = (uint32_t)TP;
         L.Qt = (uint32_t)TQ;
         const uint32_t elems = (transpose ? L.Pt | 1 : L.Pt) * L.Qt;  // at most kPlaneElems
@@ -406,7 +472,8 @@ extern "C" int dtcf_permute_copy_f64(const double *in, double *out, const dtcf_s
         return DTCF_OK;
     }
     const unsigned grid = (unsigned)std::min<uint64_t>(P.total, max_grid);
-    hipLaunchKernelGGL(permute_vec_kernel, dim3(grid), dim3(256), 0, s, in, out, P);
+    if (fixed) hipLaunchKernelGGL(permute_tile_kernel, dim3(grid), dim3(256), 0, s, in, out, P, src_off, dst_off);
+    else hipLaunchKernelGGL(permute_vec_kernel, dim3(grid), dim3(256), 0, s, in, out, P);
     DTCF_HIP(hipGetLastError());
     return DTCF_OK;
 }

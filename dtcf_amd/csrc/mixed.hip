@@ -1030,9 +1030,18 @@ __device__ __forceinline__ void oz_run(const OzArgs &g, i4 *smem, uint32_t q, in
     // Row blocks past the planes' last (planes are padded to 128 rows, tiles
     // may be 192) repeat it: in range, and never stored.
     constexpr int NC = (NF + OZ_WAVES - 1) / OZ_WAVES;
-    const unsigned char *src[NC];
+    // 128 x 128: fragment c of a wave is its own row block in plane c of A, then
+    // of B.  Only the two row blocks are kept: ten addresses of five digits
+    // spilled, and each of a tile's first loads waited for its reload and so
+    // for the load before it.
+    constexpr bool SQUARE = T::BM / 16 == OZ_WAVES && T::BN / 16 == OZ_WAVES;
+    const unsigned char *src[SQUARE ? 2 : NC];
+    if constexpr (SQUARE) {
+        src[0] = g.A + ((m0 >> 4) + wv) * nk64 * 1024;  // in range: planes are padded to 128 rows
+        src[1] = g.B + ((n0 >> 4) + wv) * nk64 * 1024;
+    }
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
+    for (int c = 0; c < (SQUARE ? 0 : NC); c++) {
         const int f = min(c * OZ_WAVES + wv, NF - 1);
         const bool ina = f < FA;
         const int h = ina ? f : f - FA, nb = ina ? T::BM / 16 : T::BN / 16, d = h / nb, b = h % nb;
@@ -1041,11 +1050,16 @@ __device__ __forceinline__ void oz_run(const OzArgs &g, i4 *smem, uint32_t q, in
     }
     auto issue = [&](int64_t kt, int64_t s) __attribute__((always_inline)) {
         i4 *stage = smem + (s & 1) * NF * 64;
+        const unsigned char *pl[2] = {src[0], src[1]};
+        if constexpr (SQUARE) asm volatile("" : "+s"(pl[0]), "+s"(pl[1]));  // the planes' addresses are made here
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             const int f = c * OZ_WAVES + wv;
             if ((c + 1) * OZ_WAVES > NF && f >= NF) break;  // wave-uniform
-            __builtin_amdgcn_global_load_lds((const void *)(src[c] + kt * 1024 + 16 * lane),
+            const unsigned char *x;
+            if constexpr (SQUARE) x = c < NS ? pl[0] + c * pa : pl[1] + (c - NS) * pb;
+            else x = src[c];
+            __builtin_amdgcn_global_load_lds((const void *)(x + kt * 1024 + 16 * lane),
                                              (__attribute__((address_space(3))) void *)(stage + f * 64), 16, 0, 0);
         }
     };
@@ -1056,6 +1070,8 @@ __device__ __forceinline__ void oz_run(const OzArgs &g, i4 *smem, uint32_t q, in
         __builtin_amdgcn_sched_barrier(0);
     };
     typedef typename OzT<P>::Acc Acc;
+    constexpr int LAST = NS < L - 1 ? NS : L - 1;  // last B digit with a product
+    constexpr int SYNC_AT = L >= 5 ? LAST - 1 : LAST;
     bool first = true;
     // INT32 level sums stay exact for kchunk_steps steps
     for (int64_t c0 = k0; c0 < k1; c0 += g.kchunk_steps) {
@@ -1084,14 +1100,15 @@ __device__ __forceinline__ void oz_run(const OzArgs &g, i4 *smem, uint32_t q, in
             // overlap the other's MFMAs.
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int dj = 1; dj <= NS; dj++) {
+            for (int dj = 1; dj <= LAST; dj++) {
                 if (dj == 2) __builtin_amdgcn_s_setprio(0);
-                if (dj == NS) sync();
-                if (dj < NS) {
+                if (dj == SYNC_AT && SYNC_AT == LAST) sync();
+                if (dj < LAST) {
 #pragma unroll
                     for (int j = 0; j < T::FN; j++)
                         bf[dj & 1][j] = sb[(dj * (T::BN / 16) + wn * T::FN + j) * 64 + lane];
                 }
+                if (dj == SYNC_AT && SYNC_AT < LAST) sync();
 #pragma unroll
                 for (int di = 1; di <= NS; di++) {
                     if (di + dj > L) continue;

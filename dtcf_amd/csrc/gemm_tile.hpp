@@ -552,7 +552,7 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(GemmArgs g)
     const int64_t row = (int64_t)tm * BM + e / BN, col = (int64_t)tn * BN + e % BN;
     if (row >= g.m || col >= g.n) return;
     bool whole;
-    const double sum = sum_pieces(g.ws, t * nk, nk, g.sw, g.steps, BM * BN, e, whole);
+    const double sum = sum_pieces(g.ws, t, gridDim.y, nk, g.sw, g.steps, BM * BN, e, whole);
     if (!whole) put_sum(g, row, col, sum);
 }
 
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(256) void group_split_reduce_kernel(GemmGroupArgs g
     const int64_t row = (int64_t)tm * BM + e / BN, col = (int64_t)tn * BN + e % BN;
     if (row >= P.m || col >= P.n) return;
     bool whole;
-    const double sum = sum_pieces(ga.ws, ga.step0[p] + t * nk, nk, ga.sw, ga.steps, BM * BN, e, whole);
+    const double sum = sum_runs(ga.ws, ga.step0[p] + t * nk, nk, ga.sw, ga.steps, BM * BN, e, whole);
     if (whole) return;
     GemmArgs g{};
     g.C = P.C;

@@ -1170,7 +1170,7 @@ __global__ __launch_bounds__(256) void oz_split_reduce(OzArgs g)
     const int64_t col = (int64_t)((q % width) / gsz) * T::BN + e % T::BN;
     if (row >= g.M || col >= g.N) return;
     bool whole;
-    const double sum = sum_pieces(g.ws, ti * nk, nk, g.sw, g.steps, T::BM * T::BN, e, whole);
+    const double sum = sum_pieces(g.ws, ti, gridDim.y, nk, g.sw, g.steps, T::BM * T::BN, e, whole);
     if (whole) return;
     const int64_t addr = g.cview ? vaddr(g.cv, row, col) : row * g.ldc + col;
     if (g.overwrite) g.C[addr] = sum;

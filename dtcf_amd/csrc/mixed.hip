@@ -1183,20 +1183,21 @@ int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 // specialisation exists; 0: one launch per product.
 int g_fused_i8 = 1;
 
-// One workgroup per CU.  rate: TOP/s of the tile's K loop on a large
+// One workgroup per CU.  rate: TOP/s (TF/s) of the tile's K loop on a large
 // product.  Every round of tiles also pays its epilogue, which nothing
 // overlaps (C read and written at about 5 TB/s).  Tiles are only cut evenly:
 // runs at 256 different K positions share no panels in L2, and at 9 TB/s of
 // digits the K loop then waits for HBM (2304 x 2304 x 9216, 216 tiles of 192 x
 // 128: 315 us in 256 equal runs, 253 uncut).
-template <typename T>
+template <int P, typename T>
 SplitPlan oz_plan(const OzArgs &g, int products, int ns, double rate, int cus)
 {
     const int64_t tm = (g.M + T::BM - 1) / T::BM, tn = (g.N + T::BN - 1) / T::BN;
     SplitPlan none;
     none.us = 1e300;
     if ((double)tm * tn >= 2147483648.0) return none;
-    const double step = 2.0 * T::BM * T::BN * OZ_BK * products / (rate * 1e6 / cus);
+    const int elems = P == DTCF_PREC_I8 ? OZ_BK : OZ_BK / 2;  // of K in a step
+    const double step = 2.0 * T::BM * T::BN * elems * products / (rate * 1e6 / cus);
     const TileRate t = {T::BM, T::BN, 1, step, {1.0, 1.0, 1.0, 1.0}, true};
     // panel rows of 128 bytes, as an FP64 K step reads
     SplitPlan p = gemm_split_plan((uint32_t)(tm * tn), g.Kp / OZ_BK, (tm * T::BM + tn * T::BN) * ns / 2, cus, t);
@@ -1248,10 +1249,10 @@ int oz_pick(const OzArgs &g, double square, double wide, hipStream_t s)
     int products = 0;
     for (int i = 1; i <= NS; i++)
         for (int j = 1; j <= NS; j++) products += i + j <= L;
-    const SplitPlan sq = oz_plan<OzTile<128, 128>>(g, products, NS, square, cus);
+    const SplitPlan sq = oz_plan<P, OzTile<128, 128>>(g, products, NS, square, cus);
     if constexpr (L == 4) {
-        const SplitPlan hi = oz_plan<OzTile<192, 128>>(g, products, NS, 0.97 * wide, cus);
-        const SplitPlan lo = oz_plan<OzTile<128, 192>>(g, products, NS, wide, cus);
+        const SplitPlan hi = oz_plan<P, OzTile<192, 128>>(g, products, NS, 0.97 * wide, cus);
+        const SplitPlan lo = oz_plan<P, OzTile<128, 192>>(g, products, NS, wide, cus);
         if (hi.us <= lo.us && hi.us < sq.us) return oz_launch<P, NS, L, OzTile<192, 128>>(g, hi, s);
         if (lo.us < sq.us) return oz_launch<P, NS, L, OzTile<128, 192>>(g, lo, s);
     }

@@ -50,3 +50,22 @@ def test_fused_tiles(dev, prec, ns, lev, m, n, k):
     for _ in range(2):
         mixed.gemm_split(sa, sb, gv, alpha=0.5, cview=view, max_level=lev)
     assert torch.equal(gv.view(n, m).t().contiguous().reshape(-1), got)
+
+
+
+@pytest.mark.parametrize("prec", [mixed.BF16X3, mixed.F16X3])
+def test_fp32_sums_stay_short(dev, prec):
+    """The FP32 level sums run over half of K at most where 128 x 128 tiles
+    would leave a short last round, whatever tile the plan takes.  One product
+    of 2^30 at the start and 1310 of 1 in the second half (K padded to 2688, 84
+    steps of 32): added to 2^30 in FP32 a step's 32 is below half a unit in the
+    last place and is lost, in a sum of its own every one counts."""
+    m, n, k = 5954, 928, 2654
+    row = torch.zeros(k, dtype=torch.float64, device=dev)
+    row[0], row[1344:] = 2.0 ** 15, 1.0
+    sa = mixed.Split(prec, row.repeat(m), mixed.dense_view(m, k), 3)
+    sb = mixed.Split(prec, row.repeat(n), mixed.dense_view(n, k), 3)
+    C = torch.zeros(m * n, dtype=torch.float64, device=dev)
+    print("fp32 sums", prec, flush=True)
+    mixed.gemm_split(sa, sb, C, ldc=n, max_level=4)
+    assert (C == 2.0 ** 30 + (k - 1344)).all()

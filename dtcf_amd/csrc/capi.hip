@@ -29,7 +29,7 @@ int ccsd_scratch_setup(int dev);  // ccsd.hip
 
 // Tile-shape choice when no explicit configuration is set.  (192 x 96 and 96
 // x 192 were never the fastest and are used only when forced.)
-int pick_config(int64_t m, int64_t n, int64_t k)
+int pick_config(int64_t m, int64_t n, int64_t k, bool gather)
 {
     const int forced = g_cfg.load();
     if (forced >= 0) return forced;
@@ -54,7 +54,9 @@ int pick_config(int64_t m, int64_t n, int64_t k)
     // columns, so 128 x 128 unless its padding costs more than 12% over 64 x
     // 64's (10000 x 100 x 10000: 424 against 471 us).
     auto padded = [&](int64_t t) { return (double)((m + t - 1) / t * t) * (double)((n + t - 1) / t * t); };
-    if (std::min(m, n) <= 128) return padded(128) <= 1.12 * padded(64) ? kCfg128x128 : kCfg64x64;
+    // (Likewise where an operand is gathered, whose loads bound the step: 2242 x
+    // 1920 x 2436 1159 against 1453, 2365 x 1056 x 2940 637 / 780.)
+    if (gather || std::min(m, n) <= 128) return padded(128) <= 1.12 * padded(64) ? kCfg128x128 : kCfg64x64;
     // Otherwise the shorter predicted time (gemm_split_plan): 128 x 128 runs 70
     // TF/s on a large product, 64 x 64 62 to 64, but a quarter of the tile
     // fills the last round and the edges better (2048^3: 286 / 265 us, 2400^3:
@@ -283,6 +285,7 @@ int dtcf_view_create(int64_t rows, int64_t cols, const int64_t *rofs, const int6
     v->coladj = coladj;
     v->rowadj = rowadj;
     v->rowwise = (double)runit * cols > (double)cunit * rows;
+    v->gather = 2 * cunit < cols && 2 * runit < rows;
     v->rowrun16 = !blk;
     for (int64_t r = 0; v->rowrun16 && r < rows; r++) v->rowrun16 = rofs[r] == rofs[r & ~15ll] + (r & 15);
     hipError_t e = hipMalloc(&v->rofs, rows * sizeof(int64_t));
@@ -371,6 +374,7 @@ static int operand_mode(const dtcf_view_s *v, const double *X, OpArgs &o)
                                                    : v->rowwise;
     o.vec2 = al && (v->colpairs || v->rowpairs) && !v->blk;
     o.adj = rows ? v->rowadj : v->coladj;
+    o.gather = v->gather && !o.adj;
     return rows ? kVMN : kVK;
 }
 
@@ -429,7 +433,7 @@ static int gemm_view_impl(int64_t m, int64_t n, int64_t k, double alpha, const d
     fill_op(g.b, bv);
     g.amode = operand_mode(av, A, g.a);
     g.bmode = operand_mode(bv, B, g.b);
-    int cfg = pick_config(m, n, k);
+    int cfg = pick_config(m, n, k, g.a.gather || g.b.gather);
     // 128 x 128 has no registers left for the block offsets of a table (48 to
     // 128 spills): 4608^3 with tables on both operands 5.06 ms, 4.19 on 64 x 64.
     if ((av->blk || bv->blk) && cfg == kCfg128x128 && g_cfg.load() < 0) cfg = kCfg64x64;

@@ -79,19 +79,32 @@ int split_workspace(hipStream_t s, size_t need, double **ws)
 
 }  // namespace
 
-TileRate tile_rate(int cfg)
+TileRate tile_rate(int cfg, bool gather)
 {
     // Measured with whole tiles, one to four workgroups on every CU: 256,
     // 512 and 1024 tiles of 64 x 64 x 4096 in 195, 278 and 515 us, 256 and
     // 512 tiles of 128 x 128 in 561 (x 4096) and 514 us (x 2048).
+    TileRate t;
     switch (cfg) {
-    case kCfg192x96: return {192, 96, 2, 2.25, {0.88, 1.0, 1.0, 1.0}};
-    case kCfg96x192: return {96, 192, 2, 2.25, {0.88, 1.0, 1.0, 1.0}};
-    case kCfg64x64: return {64, 64, 4, 0.50, {0.66, 0.925, 0.98, 1.0}};
-    case kCfg192x64: return {192, 64, 2, 1.52, {0.85, 1.0, 1.0, 1.0}};
-    case kCfg64x192: return {64, 192, 2, 1.52, {0.85, 1.0, 1.0, 1.0}};
-    default: return {128, 128, 2, 1.96, {0.895, 1.0, 1.0, 1.0}};
+    case kCfg192x96: t = {192, 96, 2, 2.25, {0.88, 1.0, 1.0, 1.0}}; break;
+    case kCfg96x192: t = {96, 192, 2, 2.25, {0.88, 1.0, 1.0, 1.0}}; break;
+    case kCfg64x64: t = {64, 64, 4, 0.50, {0.66, 0.925, 0.98, 1.0}}; break;
+    case kCfg192x64: t = {192, 64, 2, 1.52, {0.85, 1.0, 1.0, 1.0}}; break;
+    case kCfg64x192: t = {64, 192, 2, 1.52, {0.85, 1.0, 1.0, 1.0}}; break;
+    default: t = {128, 128, 2, 1.96, {0.895, 1.0, 1.0, 1.0}}; break;
     }
+    // An operand read element by element from lines of its own: the CU's loads
+    // bound the step, 1.4 us on 64 x 64 tiles from two workgroups on and 4.5 on
+    // 128 x 128, and lines serve several steps and tiles only from the L2s, so
+    // the cuts are even (SplitPlan).  us, rated as pairs / so: 152 x 1295 x
+    // 756 41.3 / 27.5, 782 x 700 x 450 49.4 / 33.1, 176 x 630 x 910 29.5 / 21.8.
+    if (gather) {
+        t.step_us *= t.bm * t.bn <= 64 * 64 ? 2.8 : 2.3;
+        t.share[0] = t.bm * t.bn <= 64 * 64 ? 0.7 : 1.0;
+        for (int c = 1; c < 4; c++) t.share[c] = 1.0;
+        t.even = true;
+    }
+    return t;
 }
 
 SplitPlan gemm_split_plan(uint32_t T, int64_t nk, int64_t panel, int cus, const TileRate &t)

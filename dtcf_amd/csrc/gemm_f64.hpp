@@ -33,7 +33,7 @@ enum {
     kCfgGroupCount = 4
 };
 // The C tile configuration dtcf_gemm_* uses for an m x n x k GEMM.
-int pick_config(int64_t m, int64_t n, int64_t k);
+int pick_config(int64_t m, int64_t n, int64_t k, bool gather = false);
 
 struct OpArgs {
     int64_t ld;
@@ -45,6 +45,7 @@ struct OpArgs {
     int32_t vec2;  // 1: (r,c),(r,c+1) [k-mode] or (r,c),(r+1,c) [mn-mode] are adjacent
                    //    and 16-byte aligned wherever both are in range (c or r even)
     int32_t adj;   // views: 1: they are adjacent, at any alignment
+    int32_t gather;  // views: 1: single elements whose neighbours lie elsewhere
 };
 
 struct GemmArgs {
@@ -136,7 +137,7 @@ struct TileRate {
     double step_us, share[4];
     bool even = false;
 };
-TileRate tile_rate(int cfg);
+TileRate tile_rate(int cfg, bool gather = false);
 // panel: rows of A and B together that one K step of the whole product
 // reads (tiles_m bm + tiles_n bn, 0: much shared, as in a large product).
 SplitPlan gemm_split_plan(uint32_t T, int64_t nk, int64_t panel, int cus, const TileRate &t);

@@ -607,7 +607,8 @@ int launch_one(GemmArgs g, hipStream_t s)
     if (st != DTCF_OK) return st;
     const uint32_t T = g.tiles_m * g.tiles_n;
     const int64_t nk = (g.k + BK - 1) / BK;
-    const SplitPlan sp = gemm_split_plan(T, nk, (int64_t)g.tiles_m * BM + (int64_t)g.tiles_n * BN, cus, tile_rate(CFG));
+    const SplitPlan sp = gemm_split_plan(T, nk, (int64_t)g.tiles_m * BM + (int64_t)g.tiles_n * BN, cus,
+                                         tile_rate(CFG, g.a.gather || g.b.gather));
     g.t_full = T - sp.nsplit;
     g.sw = sp.sw;
     g.steps = (int64_t)sp.nsplit * nk;

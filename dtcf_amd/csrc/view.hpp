@@ -11,6 +11,7 @@ struct dtcf_view_s {
     // the same at any alignment; and whether adjacent rows are more often
     // one element apart than adjacent columns
     bool coladj = false, rowadj = false, rowwise = false;
+    bool gather = false;  // neighbours mostly not adjacent in either direction
     bool rowrun16 = false;  // no block table and rofs[r] = rofs[r & ~15] + (r & 15)
     bool owner = true;  // sub-views share their parent's tables
 };

@@ -90,3 +90,40 @@ def test_scrambled_tiles_cost_no_checked_loads(dev):
     a, b = us(*scr), us(*order)
     print("scrambled", a, "in order", b, flush=True)
     assert a <= 2.0 * b, (a, b)
+
+
+@pytest.mark.parametrize("dims,oa,ob", [((23, 34, 20, 35, 30, 15), (2, 0, 3, 1), (1, 2, 3, 0)),
+                                        ((11, 16, 18, 35, 26, 35), (2, 0, 3, 1), (0, 3, 1, 2))])
+def test_gathered_operands_fill_the_chip(dev, dims, oa, ob):
+    """(a, b) x (c, d) summed over (e, f) with B's (or A's) last memory index
+    no neighbour along rows or columns, so B is read element by element,
+    against the same product with both stored rows first: 1.06 and 1.15 times
+    its time; cut over K as if it were read in pairs it took 1.55 times."""
+    a, b, c, d, e, f = dims
+    m, n, k = a * b, c * d, e * f
+
+    def view(x, order):
+        st, s = [0] * 4, 1
+        for q in reversed(order):
+            st[q], s = s, s * x[q]
+        i = [np.arange(v) * t for v, t in zip(x, st)]
+        return ops.View(x[0] * x[1], x[2] * x[3], (i[0][:, None] + i[1]).ravel(), (i[2][:, None] + i[3]).ravel())
+
+    A, B, C = _rand(m * k, 1, dev), _rand(n * k, 2, dev), torch.zeros(m * n, dtype=torch.float64, device=dev)
+
+    def us(av, bv):
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        out = []
+        for _ in range(7):
+            ev[0].record()
+            for _ in range(30):
+                ops.gemm_view(m, n, k, 1.0, A, av, B, bv, C, None, ldc=n)
+            ev[1].record()
+            torch.cuda.synchronize()
+            out.append(ev[0].elapsed_time(ev[1]) / 30 * 1e3)
+        return sorted(out)[3]
+
+    x, y = (a, b, e, f), (c, d, e, f)
+    p, q = us(view(x, oa), view(y, ob)), us(view(x, (0, 1, 2, 3)), view(y, (0, 1, 2, 3)))
+    print("gathered", p, "rows first", q, flush=True)
+    assert p <= 1.3 * q, (p, q)

@@ -187,7 +187,14 @@ int thin_f64_launch(const GemmArgs &g, hipStream_t s);
 int gemm_reserve_workspace(hipStream_t s);
 // The split workspace of stream `s` (grown to `need` bytes if smaller; work
 // on one stream shares it in stream order), and the device's CU count.
-int gemm_workspace(hipStream_t s, size_t need, double **ws);
+// A capturing stream cannot grow its own: with at least `uncut` bytes *ws is
+// null and the launch runs without cuts, with less the call is refused.
+int gemm_workspace(hipStream_t s, size_t need, double **ws, size_t uncut = SIZE_MAX);
+// The `uncut` of T tiles (tile elements each) of nk K steps on `slots`
+// resident workgroups: 0 where whole tiles fill most of every round, else what
+// filling them by even cuts takes, since uncut such a product leaves up to
+// nearly all of the device idle.
+size_t gemm_uncut_bytes(uint32_t T, uint32_t slots, int64_t nk, size_t tile);
 int gemm_device_cus(int *cus);
 
 // dtcf_gemm_view_f64 with C = alpha * A * B instead of C += (capi.hip).

@@ -593,6 +593,16 @@ int allow_lds(K kern, size_t lds, std::once_flag &once, hipError_t &err)
     return DTCF_OK;
 }
 
+// gemm_uncut_bytes of a product on the tiles that its shape alone would take,
+// two workgroups per CU.
+inline size_t uncut_bytes(const GemmArgs &g, int cus)
+{
+    const int cfg = pick_config(g.m, g.n, g.k, true);
+    const TileRate t = tile_rate(cfg == kCfgThin ? kCfg64x64 : cfg);
+    const int64_t T = ((g.m + t.bm - 1) / t.bm) * ((g.n + t.bn - 1) / t.bn);
+    return gemm_uncut_bytes((uint32_t)T, 2 * cus, (g.k + BK - 1) / BK, (size_t)t.bm * t.bn);
+}
+
 template <int CFG, int BM, int BN, int WM, int WN, int AM, int BMD, int LOAD>
 int launch_one(GemmArgs g, hipStream_t s)
 {
@@ -607,15 +617,16 @@ int launch_one(GemmArgs g, hipStream_t s)
     if (st != DTCF_OK) return st;
     const uint32_t T = g.tiles_m * g.tiles_n;
     const int64_t nk = (g.k + BK - 1) / BK;
-    const SplitPlan sp = gemm_split_plan(T, nk, (int64_t)g.tiles_m * BM + (int64_t)g.tiles_n * BN, cus,
-                                         tile_rate(CFG, g.a.gather || g.b.gather));
+    SplitPlan sp = gemm_split_plan(T, nk, (int64_t)g.tiles_m * BM + (int64_t)g.tiles_n * BN, cus,
+                                   tile_rate(CFG, g.a.gather || g.b.gather));
+    if (sp.nsplit) {
+        st = gemm_workspace(s, (size_t)2 * sp.sw * BM * BN * sizeof(double), &g.ws, uncut_bytes(g, cus));
+        if (st != DTCF_OK) return st;
+        if (!g.ws) sp = SplitPlan();
+    }
     g.t_full = T - sp.nsplit;
     g.sw = sp.sw;
     g.steps = (int64_t)sp.nsplit * nk;
-    if (sp.nsplit) {
-        st = gemm_workspace(s, (size_t)2 * sp.sw * BM * BN * sizeof(double), &g.ws);
-        if (st != DTCF_OK) return st;
-    }
     hipLaunchKernelGGL(kern, dim3(g.t_full + g.sw), dim3(NT), lds, s, g);
     DTCF_HIP(hipGetLastError());
     if (sp.nsplit) {
@@ -666,9 +677,10 @@ int launch_group(GemmGroupArgs ga, hipStream_t s)
     int st = allow_lds(kern, lds, once, attr_err);
     if (st != DTCF_OK) return st;
     uint64_t total = 0;
-    int64_t steps = 0;
+    int64_t steps = 0, nk_min = INT64_MAX;
     for (int i = 0; i < ga.np; i++) {
         GemmGroupProb &P = ga.p[i];
+        nk_min = std::min<int64_t>(nk_min, (P.k + BK - 1) / BK);
         P.tiles_m = (uint32_t)((P.m + BM - 1) / BM);
         P.tiles_n = (uint32_t)((P.n + BN - 1) / BN);
         P.nfast = fast_steps(P.k, (AM == kDMN && P.m % 2) || (BMD == kDMN && P.n % 2));
@@ -690,6 +702,13 @@ int launch_group(GemmGroupArgs ga, hipStream_t s)
     // 158, 171; 1568 x 850: 195, 218; 2180 x 1000: 294, 288; 8525 x 2050: 2160,
     // 2132).
     if (Occ<BM, BN>::v == 4 && total > (uint64_t)cus * 4) sp = SplitPlan();
+    ga.ws = nullptr;
+    if (sp.nsplit) {
+        st = gemm_workspace(s, (size_t)2 * sp.sw * BM * BN * sizeof(double), &ga.ws,
+                            gemm_uncut_bytes((uint32_t)total, 2 * cus, nk_min, (size_t)BM * BN));
+        if (st != DTCF_OK) return st;
+        if (!ga.ws) sp = SplitPlan();
+    }
     uint32_t left = sp.nsplit;
     for (int i = ga.np - 1; i >= 0; i--) {
         GemmGroupProb &P = ga.p[i];
@@ -717,11 +736,6 @@ int launch_group(GemmGroupArgs ga, hipStream_t s)
     }
     ga.wg_whole = (uint32_t)wg;
     ga.sw = (uint32_t)std::min<int64_t>(sp.sw, ga.steps);
-    ga.ws = nullptr;
-    if (ga.sw) {
-        st = gemm_workspace(s, (size_t)2 * ga.sw * BM * BN * sizeof(double), &ga.ws);
-        if (st != DTCF_OK) return st;
-    }
     hipLaunchKernelGGL(kern, dim3(ga.wg_whole + ga.sw), dim3(NT), lds, s, ga);
     DTCF_HIP(hipGetLastError());
     if (ga.sw) {

@@ -1221,8 +1221,23 @@ int64_t fp32_steps(int64_t tiles, int64_t nk, int cus)
     return (nk + pieces - 1) / pieces;
 }
 
+// gemm_uncut_bytes of a slice product, on 128 x 128 tiles cut into pieces of at
+// least 16 steps: a grid under half of the CUs, or a last round of at most
+// half.
+size_t oz_uncut_bytes(const OzArgs &g, int cus)
+{
+    const int64_t T = g.Mp / 128 * (g.Np / 128), nk = g.Kp / OZ_BK, rem = T % cus;
+    int64_t cut = 0;
+    if (nk >= 32 && T < cus / 2) cut = T;
+    else if (nk >= 32 && T > cus && rem > 0 && rem <= cus / 2) cut = rem;
+    const int64_t sk = cut ? std::min<int64_t>(cus / cut, nk / 16) : 0;
+    if (sk < 2) return 0;
+    const int64_t steps = (nk + sk - 1) / sk;
+    return (size_t)cut * ((nk + steps - 1) / steps) * 128 * 128 * sizeof(double);
+}
+
 template <int P, int NS, int L, typename T>
-int oz_launch(OzArgs g, const SplitPlan &sp, hipStream_t s)
+int oz_launch(OzArgs g, SplitPlan sp, hipStream_t s)
 {
     auto kern = ozaki_kernel<P, NS, L, T>;
     constexpr size_t lds = (size_t)2 * NS * (T::BM + T::BN) * OZ_BK;
@@ -1236,14 +1251,18 @@ int oz_launch(OzArgs g, const SplitPlan &sp, hipStream_t s)
     g.tiles_m = (uint32_t)((g.M + T::BM - 1) / T::BM);
     g.tiles_n = (uint32_t)((g.N + T::BN - 1) / T::BN);
     const uint32_t tiles = g.tiles_m * g.tiles_n;
+    g.ws = nullptr;
+    if (sp.nsplit) {
+        int cus = 0;
+        int st = gemm_device_cus(&cus);
+        if (st != DTCF_OK) return st;
+        st = gemm_workspace(s, (size_t)2 * sp.sw * T::BM * T::BN * sizeof(double), &g.ws, oz_uncut_bytes(g, cus));
+        if (st != DTCF_OK) return st;
+        if (!g.ws) sp = SplitPlan();
+    }
     g.t_full = tiles - sp.nsplit;
     g.sw = sp.sw;
     g.steps = (int64_t)sp.nsplit * (g.Kp / OZ_BK);
-    g.ws = nullptr;
-    if (sp.nsplit) {
-        const int st = gemm_workspace(s, (size_t)2 * sp.sw * T::BM * T::BN * sizeof(double), &g.ws);
-        if (st != DTCF_OK) return st;
-    }
     hipLaunchKernelGGL(kern, dim3(g.t_full + g.sw), dim3(64 * OZ_WAVES), lds, s, g);
     DTCF_HIP(hipGetLastError());
     if (sp.nsplit) {

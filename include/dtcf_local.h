@@ -133,7 +133,9 @@ int dtcf_view_scatter_f64(const double *src, int64_t ld, dtcf_view v, double *ds
 
 /* GEMMs that split K keep their partial sums in a workspace of the stream
  * they run on, grown on demand (an allocation).  Under HIP graph capture it
- * cannot grow: such a GEMM returns DTCF_ERR_INVALID.  This call grows the
+ * cannot grow: a GEMM that whole tiles serve nearly as well (most of every
+ * round of the device's workgroups filled) then runs without the split, any
+ * other returns DTCF_ERR_INVALID.  This call grows the
  * stream's workspace now to the bound any GEMM launch on this device can
  * need (151 MB on 256 CUs), so captures on that stream never allocate;
  * call it, outside capture, for every stream a graph will record GEMMs on.

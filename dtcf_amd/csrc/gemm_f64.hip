@@ -140,7 +140,7 @@ SplitPlan gemm_split_plan(uint32_t T, int64_t nk, int64_t panel, int cus, const 
     best.us += 0.012 * R;
     auto consider = [&](uint32_t W, double pieces) {
         const double n = (double)((steps + W - 1) / W);
-        const double us = whole + run_us(n, (W + cus - 1) / cus) + 0.012 * W + 4.0 +
+        const double us = whole + run_us(n, (W + cus - 1) / cus) + 0.012 * W + t.cut_us +
                           pieces * t.bm * t.bn * 16.0 / 6.0e6 + 0.7 * (pieces / R / 8.0 + 1.0);
         if (us < best.us) {
             best.us = us;

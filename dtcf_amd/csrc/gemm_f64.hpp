@@ -136,6 +136,7 @@ struct TileRate {
     int bm, bn, occ;
     double step_us, share[4];
     bool even = false;
+    double cut_us = 4.0;  // what any cut costs beside its pieces
 };
 TileRate tile_rate(int cfg, bool gather = false);
 // panel: rows of A and B together that one K step of the whole product

@@ -694,14 +694,13 @@ int launch_group(GemmGroupArgs ga, hipStream_t s)
     int cus = 0;
     st = gemm_device_cus(&cus);
     if (st != DTCF_OK) return st;
-    SplitPlan sp = gemm_split_plan((uint32_t)total, std::max<int64_t>(1, steps / (int64_t)total), 0, cus,
-                                   tile_rate(CFG));
-    // Past one round of 64 x 64 tiles nothing is cut: four workgroups per CU
-    // absorb the ragged end of problems of different K, which equal runs then
-    // only lengthen (1802 tiles x 930: 237 us whole, 265-270 cut; 1354 x 800:
-    // 158, 171; 1568 x 850: 195, 218; 2180 x 1000: 294, 288; 8525 x 2050: 2160,
-    // 2132).
-    if (Occ<BM, BN>::v == 4 && total > (uint64_t)cus * 4) sp = SplitPlan();
+    // Past one round of 64 x 64 tiles a cut has to gain more: four workgroups
+    // per CU absorb the ragged end of problems of different K, which equal runs
+    // then lengthen by 10 to 30 us (1802 tiles x 930: 237 us whole, 265-270 cut;
+    // 1354 x 800: 158, 171; 1568 x 850: 195, 218; but 8525 x 2050: 2160, 2132).
+    TileRate rate = tile_rate(CFG);
+    if (Occ<BM, BN>::v == 4 && total > (uint64_t)cus * 4) rate.cut_us += 20.0;
+    SplitPlan sp = gemm_split_plan((uint32_t)total, std::max<int64_t>(1, steps / (int64_t)total), 0, cus, rate);
     ga.ws = nullptr;
     if (sp.nsplit) {
         st = gemm_workspace(s, (size_t)2 * sp.sw * BM * BN * sizeof(double), &ga.ws,

@@ -1241,13 +1241,16 @@ int oz_launch(OzArgs g, SplitPlan sp, hipStream_t s)
 {
     auto kern = ozaki_kernel<P, NS, L, T>;
     constexpr size_t lds = (size_t)2 * NS * (T::BM + T::BN) * OZ_BK;
-    static std::once_flag once;
-    static hipError_t attr_err = hipSuccess;
-    std::call_once(once, [&] {
-        attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    // once per device (gemm_device_cus has checked its index)
+    static std::once_flag once[64];
+    static hipError_t attr_err[64];
+    int dev = 0;
+    DTCF_HIP(hipGetDevice(&dev));
+    std::call_once(once[dev], [&] {
+        attr_err[dev] = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
-    DTCF_HIP(attr_err);
+    DTCF_HIP(attr_err[dev]);
     g.tiles_m = (uint32_t)((g.M + T::BM - 1) / T::BM);
     g.tiles_n = (uint32_t)((g.N + T::BN - 1) / T::BN);
     const uint32_t tiles = g.tiles_m * g.tiles_n;

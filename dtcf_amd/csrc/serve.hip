@@ -1509,7 +1509,7 @@ extern "C" int dtcf_program_statement_plan(dtcf_program p, int64_t i, int64_t *o
     if (s.res[0]) f |= DTCF_PLAN_RES_A;
     if (s.res[1]) f |= DTCF_PLAN_RES_B;
     out[DTCF_PLAN_FLAGS] = f;
-    out[DTCF_PLAN_TILE] = s.mixed ? -1 : pick_config(s.m, s.n, s.k);
+    out[DTCF_PLAN_TILE] = s.mixed ? -1 : pick_config(s.m, s.n, s.k, s.av->gather || s.bv->gather);
     return DTCF_OK;
 }
 

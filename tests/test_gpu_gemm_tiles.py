@@ -103,16 +103,16 @@ def test_views_off_alignment(dev, cfg_reset, cfg, ka, kb):
                                        (3, 2112, 2112, 80), (3, 2200, 2050, 333), (0, 128, 128, 9000),
                                        (0, 1300, 1200, 700), (0, 2400, 2400, 171), (0, 2944, 2944, 100),
                                        (4, 192, 48, 20001), (5, 48, 192, 20001), (1, 1000, 900, 800)])
-@pytest.mark.parametrize("overwrite_view", [False, True])
-def test_split_runs(dev, cfg_reset, cfg, m, n, k, overwrite_view):
+@pytest.mark.parametrize("cview", [False, True])
+def test_split_runs(dev, cfg_reset, cfg, m, n, k, cview):
     ops.set_gemm_config(cfg)
     A, B, C = _rand(m * k, 7, dev), _rand(n * k, 8, dev), _rand(m * n, 9, dev)
     ref = C.view(m, n) - 2.0 * (A.view(m, k) @ B.view(n, k).t().contiguous())
-    print("split", cfg, m, n, k, overwrite_view, flush=True)
+    print("split", cfg, m, n, k, cview, flush=True)
     outs = []
     for _ in range(2):
         X = C.clone()
-        if overwrite_view:  # C through a view of its transpose
+        if cview:  # C through a view of its transpose
             X = X.view(m, n).t().contiguous().reshape(-1)
             v = ops.View(m, n, np.arange(m), np.arange(n) * m)
             ops.gemm_view(m, n, k, -2.0, A, ops.View(m, k, np.arange(m) * k, np.arange(k)), B,
@@ -201,3 +201,30 @@ def test_group_fills_the_chip_like_a_lone_launch(dev):
     a, b = us(run), us(lone)
     print("group", a, "lone", b, flush=True)
     assert a <= 1.25 * b, (a, b)
+
+
+# One served product with a fresh result: every element stored, none read or
+# cleared before, by whole tiles, by runs that cover a tile and by the sums of
+# cut ones.  The request block is first left full of another program's values.
+@pytest.mark.parametrize("cfg", [-1, 0, 3])
+@pytest.mark.parametrize("m,n,k", [(500, 500, 500), (130, 70, 3001), (2200, 2050, 333), (1300, 1200, 700)])
+def test_served_overwrite(dev, cfg_reset, cfg, m, n, k):
+    from dtcf_amd import serve, termlist
+
+    text = ("range M = 1.0;\nrange N = 1.0;\nrange K = 1.0;\nindex i = M;\nindex j = N;\nindex l = K;\n"
+            "array a([M][K]), b([K][N]), c([M][N]);\nc[i,j] = (a[i,l] * b[l,j])\n")
+    tl = termlist.parse(text)
+    ops.set_gemm_config(cfg)
+    with serve.Server(1 << 29, 1) as srv:
+        system = serve.System(srv, 0, 0, [tl], sizes={"M": m, "N": n, "K": k})
+        prog = serve.Program(srv, tl, system)
+        print("served overwrite", cfg, m, n, k, flush=True)
+        out = [torch.full((m * n,), float("nan"), dtype=torch.float64, device=dev)]
+        for _ in range(2):
+            rid = prog.submit(out)[0]
+            _lib.check(srv.wait(rid, 60000.0))
+            srv.release(rid)
+        prog.destroy()
+        ref = system.host("a") @ system.host("b")
+    got = out[0].view(m, n).cpu().numpy()
+    assert np.abs(got - ref).max() / np.abs(ref).max() <= TOL

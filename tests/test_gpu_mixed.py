@@ -144,9 +144,10 @@ def test_fused_int8_matches_per_product(dev, ns, lev, m, n, k, cview):
 @pytest.mark.parametrize("m,n,k,cview", [(2176, 2048, 2048, False), (2304, 2304, 2048, True)])
 def test_fused_int8_tail_split_matches_per_product(dev, ns, lev, m, n, k, cview):
     """Grids one partial round past the CU count (272 and 324 C tiles of
-    128 x 128 on 256 CUs): the tiles of the last round are cut into K slices
-    (after the whole ones) and summed in order by a second kernel; against
-    the per-product path, to FP64 rounding."""
+    128 x 128 on 256 CUs): from level 5 the tiles of the last round are cut
+    into K slices (after the whole ones) and summed in order by a second
+    kernel; three digits to level 4 take whole 128 x 192 tiles; against the
+    per-product path, to FP64 rounding."""
     rng = np.random.default_rng(m + n + k + ns)
     A = rng.standard_normal((m, k))
     B = rng.standard_normal((n, k))
@@ -215,9 +216,10 @@ def test_fused_int8_flush_interval_at_largest_digits(dev, ns, lev):
     positive and each level sum grows by 98-99% of the per-K bound the flush
     interval is sized for.  A bound that left out a product or undercounted a
     digit (so the interval too long) overflows INT32 here; the exact result is
-    alpha K x^2 up to the dropped levels.  132 C tiles: enough for the fused
-    kernel to run without a K split, so every workgroup sums all K = 50,000
-    and flushes inside its loop."""
+    alpha K x^2 up to the dropped levels.  132 C tiles of 128 x 128: from
+    level 5 the fused kernel runs without a K split, so every workgroup sums
+    all K = 50,000 and flushes inside its loop (level 4 cuts its 96 wide tiles
+    in two; test_gpu_slice_tiles flushes inside those)."""
     m, n, k = 1536, 1408, 50000
     X = -(63 * 256 ** (ns - 1) + 128 * (256 ** (ns - 1) - 1) // 255)
     x = X / 2.0 ** (8 * ns - 2)

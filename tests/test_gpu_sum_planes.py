@@ -12,8 +12,28 @@ from dtcf_amd import serve, termlist
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("which,oa,ob", [("t2", 22, 23), ("t2", 32, 31), ("t1", 32, 33), ("t1", 45, 46),
-                                         ("t1", 54, 53), ("t1", 54, 56)])
+SIZES = (("t2", 22, 23), ("t2", 32, 31), ("t1", 32, 33), ("t1", 38, 40), ("t1", 45, 46), ("t1", 54, 53),
+         ("t1", 54, 56))
+
+
+def _instances(which, oa, ob):
+    """(pairs, elements per thread of 512) of the sum statements' planes."""
+    tl, ext, out = termlist.load(which), {"Oa": oa, "Ob": ob, "Va": 3, "Vb": 2}, set()
+    for s in tl.statements:
+        shape = [1] * 4 + [ext[r] for r in tl.arrays[s.lhs.name].ranges]
+        d2, d3 = shape[-2:]
+        if s.kind == "sum" and (d2 + 1) * d3 <= 3072:
+            pairs = d2 % 2 == 0 and d3 % 2 == 0
+            out.add((pairs, min(x for x in ((2, 4, 6) if pairs else (1, 2, 4, 6)) if 512 * x >= d2 * d3)))
+    return out
+
+
+def test_sizes_reach_every_instance(dev):
+    assert set().union(*[_instances(*x) for x in SIZES]) == {(True, x) for x in (2, 4, 6)} | {
+        (False, x) for x in (1, 2, 4, 6)}
+
+
+@pytest.mark.parametrize("which,oa,ob", SIZES)
 def test_sum_planes(dev, which, oa, ob):
     tl = termlist.load(which)
     print("sum planes", which, oa, ob, flush=True)

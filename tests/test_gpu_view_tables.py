@@ -127,3 +127,31 @@ def test_gathered_operands_fill_the_chip(dev, dims, oa, ob):
     p, q = us(view(x, oa), view(y, ob)), us(view(x, (0, 1, 2, 3)), view(y, (0, 1, 2, 3)))
     print("gathered", p, "rows first", q, flush=True)
     assert p <= 1.3 * q, (p, q)
+
+
+# Rectangles of a view keep its pair flags only where they start and end on
+# pairs: odd and even first rows and columns, odd counts, of views whose pairs
+# run along K or the rows, aligned or not.
+@pytest.mark.parametrize("kind", ["k", "k odd", "r", "r odd"])
+@pytest.mark.parametrize("r0,c0,m,k", [(0, 0, 66, 48), (1, 0, 65, 47), (2, 1, 64, 48), (3, 3, 61, 33), (4, 2, 63, 34)])
+def test_sub_views(dev, kind, r0, c0, m, k):
+    import ctypes as C
+
+    from dtcf_amd import _lib
+
+    rows, cols, n = 70, 52, 40
+    ro, co = {"k": (np.arange(rows) * cols, np.arange(cols)), "k odd": (np.arange(rows) * (cols + 1), np.arange(cols)),
+              "r": (np.arange(rows), np.arange(cols) * rows), "r odd": (np.arange(rows), np.arange(cols) * (rows + 1))}[kind]
+    A, B, X = _rand(int(ro.max() + co.max()) + 1, 1, dev), _rand(n * k, 2, dev), _rand(m * n, 3, dev)
+    parent = ops.View(rows, cols, ro, co)
+    sub = ops.View.__new__(ops.View)
+    h = C.c_void_p()
+    L = _lib.lib()
+    _lib.check(L.dtcf_view_sub(parent.h, C.c_int64(r0), C.c_int64(m), C.c_int64(c0), C.c_int64(k), C.byref(h)))
+    sub.h, sub.rows, sub.cols = h, m, k
+    bv = ops.View(n, k, np.arange(n) * k, np.arange(k))
+    at = torch.from_numpy(ro[r0:r0 + m, None] + co[None, c0:c0 + k]).to(dev)
+    ref = X.view(m, n) + A[at] @ B.view(n, k).t().contiguous()
+    print("sub", kind, r0, c0, m, k, flush=True)
+    ops.gemm_view(m, n, k, 1.0, A, sub, B, bv, X, None, ldc=n)
+    assert ((X.view(m, n) - ref).abs().max() / ref.abs().max()).item() <= TOL

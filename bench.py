@@ -21,6 +21,7 @@ Prints ONE JSON line.  --gpus N > 1 exits: one rank's share runs on one GPU.
 from __future__ import annotations
 
 import argparse
+import hashlib
 import itertools
 import json
 import os
@@ -193,8 +194,8 @@ def traffic_record(mode, o, v, live_ms):
     """HBM bytes per launch of the step's GEMM from profiles/traffic.json
     (FETCH_SIZE x fetch_scale + WRITE_SIZE x write_scale, KiB per dispatch)
     for this workload, with the profiled kernel's average duration beside
-    the live one: a kernel that has changed since its profile shows as a
-    duration mismatch (traffic_stale)."""
+    the live one: a kernel that has changed since its profile shows in the
+    hash of its sources or as a duration mismatch (traffic_stale)."""
     try:
         with open(TRAFFIC_FILE) as f:
             recs = json.load(f)
@@ -209,8 +210,21 @@ def traffic_record(mode, o, v, live_ms):
         prof_ms = r["avg_duration_us"] / 1e3
         return {"traffic": round(traffic, -6), "traffic_source": f"profiles/traffic.json:{key}",
                 "traffic_profile_kernel_ms": round(prof_ms, 4),
-                "traffic_stale": abs(prof_ms - live_ms) > 0.05 * live_ms}
+                "traffic_stale": abs(prof_ms - live_ms) > 0.05 * live_ms or
+                r.get("sources_sha256") != sources_sha256(r.get("sources", []))}
     return {}
+
+
+def sources_sha256(names):
+    """Hash of the named files of dtcf_amd/csrc, one after another."""
+    h = hashlib.sha256()
+    for n in names:
+        try:
+            with open(os.path.join(ROOT, "dtcf_amd", "csrc", n), "rb") as f:
+                h.update(f.read())
+        except OSError:
+            return None
+    return h.hexdigest()
 
 
 def leg_ccsd(log, o=96, v=384, iters=3):

@@ -19,7 +19,7 @@
 // 8-byte read per slice; every read of a wave is one contiguous span (no
 // bank conflicts).
 //
-// Two ways to fill a stage:
+// Three ways to fill a stage:
 //   direct (both operands' pairs adjacent and 16-byte aligned, no block
 //   table): global_load_lds, 16 bytes per lane, lane l's pair straight to
 //   byte 16 l of its fragment.  No staging registers and no LDS stores, and

@@ -599,10 +599,13 @@ int plan_contraction(dtcf_program p, PStmt &s, const std::vector<std::string> &c
     // otherwise gather single elements.  Resident inputs are split once, at
     // bind, from the array itself.  The FP64 GEMM loads elements too (pairs
     // that are off alignment, or broken at the ends of runs), so there runs
-    // of four elements on average in either direction are contiguous enough:
-    // a copy of an operand with odd extents is no better aligned than the
-    // operand (T1 and T2 at Oa, Ob, Va, Vb = 10, 9, 100, 99 on eight slots:
-    // 14.2 ms with the copies, 9.2 without).
+    // of four elements on average in either direction are contiguous enough.
+    // A copy would take the direct loads when K is even, but it costs a pass
+    // of its own before the product that waits for it, and what the unaligned
+    // loads cost is less.  T1 and T2 at Oa, Ob, Va, Vb = 10, 9, 100, 99 on
+    // eight slots: 14.2 ms with the copies, 9.2 without; 30 systems of odd,
+    // even and mixed extents, Oa, Ob = 3..25 and Va, Vb = 24..150, on one and
+    // on eight slots: 0.38 to 1.00 of the time with the copies, never slower.
     auto runs = [](const std::vector<int64_t> &x) {
         size_t one = 0;
         for (size_t i = 0; i + 1 < x.size(); i++) one += x[i + 1] == x[i] + 1;
